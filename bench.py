@@ -116,12 +116,7 @@ def kernel_name(closest, sched_char, two_level=False):
     if two_level:
         kern = "k_trace2_split" if sched_char in "248x" else "k_trace2"
         return "%s<%s>" % (kern, "false" if closest else "true")
-    if sched_char == "p":
-        return "k_trace_persistent<%s, false>" % ("false" if closest else "true")
-    if sched_char in "248x":
-        return "k_trace_split<%s, false>" % ("false" if closest else "true")
-    pooled = "true" if sched_char == "w" else "false"
-    return ("k_trace_closest<false, %s>" if closest else "k_trace_any<false, %s>") % pooled
+    return "k_trace_window<%s, false>" % ("false" if closest else "true")
 
 
 class Frame:

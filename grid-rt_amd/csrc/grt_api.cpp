@@ -443,11 +443,6 @@ int grt_init(int device, grt_context* out)
         return hip_check(e, "hipStreamCreate");
     }
     ctx->stream = ctx->own_stream;
-    if ((rc = ctx->stream_counters[ctx->stream].reserve(ctx, 64, false)) != GRT_OK) {
-        (void)hipStreamDestroy(ctx->own_stream);
-        delete ctx;
-        return rc;
-    }
     *out = ctx;
     return GRT_OK;
 }
@@ -462,9 +457,6 @@ int grt_shutdown(grt_context ctx)
         grt_scene_destroy(sc);
     ctx->instance_scratch.release(ctx);
     ctx->compact_scratch.release(ctx);
-    for (auto& kv : ctx->stream_counters)
-        kv.second.release(ctx);
-    ctx->stream_counters.clear();
     if (ctx->aux_stream) {
         (void)hipStreamSynchronize(ctx->aux_stream);
         (void)hipStreamDestroy(ctx->aux_stream);
@@ -483,9 +475,7 @@ int grt_set_stream(grt_context ctx, void* hip_stream)
     if (!ctx)
         return set_error(GRT_INVALID_PARAM, "grt_set_stream: NULL context");
     ctx->stream = (hipStream_t)hip_stream;
-    // the stream's persistent-launch slot counter, allocated here (not under
-    // a capture that a later trace may be part of)
-    return ctx->stream_counters[ctx->stream].reserve(ctx, 64, false);
+    return GRT_OK;
 }
 
 int grt_synchronize(grt_context ctx)
@@ -529,7 +519,6 @@ int grt_set_trace_mode(grt_context ctx, int mode, uint32_t param)
     } else {
         if (param < 1 || param > 64)
             return set_error(GRT_INVALID_PARAM, "grt_set_trace_mode: refill must be 1..64");
-        ctx->refill = param;
     }
     ctx->trace_mode = mode;
     return GRT_OK;
@@ -539,7 +528,7 @@ int grt_set_coop(grt_context ctx, uint32_t min_refs)
 {
     if (!ctx)
         return set_error(GRT_INVALID_PARAM, "grt_set_coop: NULL context");
-    ctx->coop = min_refs;
+    (void)min_refs;   // every schedule pools its tests
     return GRT_OK;
 }
 
@@ -1218,8 +1207,6 @@ static TraceArgs trace_args(grt_scene sc, uint32_t n, uint32_t image_width, uint
     a.n = n;
     a.image_width = image_width;
     a.counters = counters;
-    a.coop = sc->ctx->coop;
-    a.pool = sc->ctx->trace_mode == GRT_TRACE_POOLED ? 1u : 0u;
     if (sc->g2_built) {
         a.g2 = sc->g2frame.as<DevFrame>();
         a.cellrec = sc->cellrec.as<uint2>();
@@ -1236,14 +1223,6 @@ static uint32_t trace2_lanes(const grt_context_t* ctx)
     return ctx->trace_mode == GRT_TRACE_SPLIT ? ctx->split_lanes : 1u;
 }
 
-// The slot counter of a persistent launch on the context's current stream.
-static uint32_t* stream_counter(grt_context_t* ctx, int& rc)
-{
-    grt::DevMem& m = ctx->stream_counters[ctx->stream];   // allocated by grt_set_stream
-    rc = m.reserve(ctx, 64, false);
-    return rc == GRT_OK ? m.as<uint32_t>() : nullptr;
-}
-
 // One closest-hit launch of the context's schedule.
 static int dispatch_closest(grt_scene sc, const TraceArgs& a, const grt_rays* rays,
                             const grt_hits* hits)
@@ -1254,20 +1233,8 @@ static int dispatch_closest(grt_scene sc, const TraceArgs& a, const grt_rays* ra
         return hip_check(launch_trace2(a, to_soa(rays), h, nullptr, trace2_lanes(ctx),
                                        ctx->stream),
                          "trace_closest");
-    if (ctx->trace_mode == GRT_TRACE_PERSISTENT) {
-        int rc = GRT_OK;
-        uint32_t* counter = stream_counter(ctx, rc);
-        if (rc != GRT_OK)
-            return rc;
-        return hip_check(launch_trace_persistent(a, to_soa(rays), h, nullptr, false, counter,
-                                                 ctx->block_closest, ctx->refill, ctx->stream),
-                         "trace_closest");
-    }
-    if (ctx->trace_mode == GRT_TRACE_SPLIT)
-        return hip_check(launch_trace_split(a, to_soa(rays), h, nullptr, false, ctx->split_lanes,
-                                            ctx->block_closest, ctx->stream),
-                         "trace_closest");
-    return hip_check(launch_trace_closest(a, to_soa(rays), h, ctx->block_closest, ctx->stream),
+    return hip_check(launch_trace_window(a, to_soa(rays), h, nullptr, false, window_lanes_of(ctx),
+                                         ctx->block_closest, ctx->stream),
                      "trace_closest");
 }
 
@@ -1280,21 +1247,8 @@ static int dispatch_any(grt_scene sc, const TraceArgs& a, const grt_rays* rays,
         return hip_check(launch_trace2(a, to_soa(rays), HitSoA{}, occluded_dev, trace2_lanes(ctx),
                                        ctx->stream),
                          "trace_any");
-    if (ctx->trace_mode == GRT_TRACE_PERSISTENT) {
-        int rc = GRT_OK;
-        uint32_t* counter = stream_counter(ctx, rc);
-        if (rc != GRT_OK)
-            return rc;
-        return hip_check(launch_trace_persistent(a, to_soa(rays), HitSoA{}, occluded_dev, true,
-                                                 counter, ctx->block_any, ctx->refill,
-                                                 ctx->stream),
-                         "trace_any");
-    }
-    if (ctx->trace_mode == GRT_TRACE_SPLIT)
-        return hip_check(launch_trace_split(a, to_soa(rays), HitSoA{}, occluded_dev, true,
-                                            ctx->split_lanes, ctx->block_any, ctx->stream),
-                         "trace_any");
-    return hip_check(launch_trace_any(a, to_soa(rays), occluded_dev, ctx->block_any, ctx->stream),
+    return hip_check(launch_trace_window(a, to_soa(rays), HitSoA{}, occluded_dev, true,
+                                         window_lanes_of(ctx), ctx->block_any, ctx->stream),
                      "trace_any");
 }
 

@@ -1,7 +1,7 @@
-// grt_batch.cpp -- batched multi-scene tracing (device work queue) and hipGraph
+// grt_batch.cpp -- batched multi-scene tracing (device task table) and hipGraph
 // capture of launch sequences.  The reference traced one scene per frame with
 // one kernel launch (cudaRayTrace, RayTracing.cu:227-253); a batch puts many
-// scenes and ray batches of uneven size into one persistent launch.
+// scenes and ray batches of uneven size into one launch.
 #include <hip/hip_runtime.h>
 
 #include <cstring>
@@ -19,7 +19,7 @@ struct grt_batch_t {
     uint32_t max_items = 0;
     uint32_t n_items = 0;
     uint32_t total_slots = 0;
-    DevMem tasks, map, counter;
+    DevMem tasks, map;
     BatchTask* staging = nullptr;   // pinned
     hipEvent_t staged = nullptr;    // staging may be reused once this completes
     bool staged_pending = false;
@@ -52,8 +52,6 @@ int grt_batch_create(grt_context ctx, uint32_t max_items, grt_batch* out)
     b->ctx = ctx;
     b->max_items = max_items;
     int rc = b->tasks.reserve(ctx, sizeof(BatchTask) * (size_t)max_items, false);
-    if (rc == GRT_OK)
-        rc = b->counter.reserve(ctx, 64, true);
     if (rc == GRT_OK && hipHostMalloc((void**)&b->staging, sizeof(BatchTask) * max_items,
                                       hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
@@ -76,7 +74,6 @@ int grt_batch_destroy(grt_batch b)
     (void)hipStreamSynchronize(b->ctx->stream);
     b->tasks.release(b->ctx);
     b->map.release(b->ctx);
-    b->counter.release(b->ctx);
     if (b->staging)
         (void)hipHostFree(b->staging);
     if (b->staged)
@@ -163,9 +160,8 @@ int grt_batch_trace(grt_batch b)
         return set_error(GRT_INVALID_PARAM, "grt_batch_trace: NULL batch");
     grt_context_t* ctx = b->ctx;
     return hip_check(launch_trace_batch(b->tasks.as<BatchTask>(), b->map.as<uint32_t>(),
-                                        b->total_slots, b->counter.as<uint32_t>(),
-                                        ctx->trace_mode, ctx->block_closest, ctx->refill,
-                                        ctx->split_lanes, ctx->coop, ctx->stream),
+                                        b->total_slots, window_lanes_of(ctx),
+                                        ctx->block_closest, ctx->stream),
                      "grt_batch_trace");
 }
 

@@ -59,9 +59,7 @@ struct grt_context_t {
     uint32_t block_closest = 128;
     uint32_t block_any = 128;
     int trace_mode = GRT_TRACE_SIMPLE;
-    uint32_t refill = 16;
     uint32_t split_lanes = 4;   // GRT_TRACE_SPLIT: lanes per ray
-    uint32_t coop = 16;   // cooperative cell tests in drained persistent waves (0: off)
     std::set<grt_scene_t*> scenes;
     grt::DevMem instance_scratch;   // object-space rays and candidate hits of instance tracing
     grt::DevMem compact_scratch;    // block sums of ray-list compaction
@@ -69,10 +67,14 @@ struct grt_context_t {
     // asynchronous rebuild that run beside the main stream; created on first use.
     hipStream_t aux_stream = nullptr;
     hipEvent_t aux_ev[4] = {nullptr, nullptr, nullptr, nullptr};
-    // Per stream the context has traced on: the slot counter of persistent
-    // launches (launches on different streams may overlap).
-    std::map<hipStream_t, grt::DevMem> stream_counters;
 };
+
+// Lanes per ray of a one-level launch: the split schedule's, else 0 (by the
+// size of the launch).
+inline uint32_t window_lanes_of(const grt_context_t* ctx)
+{
+    return ctx->trace_mode == GRT_TRACE_SPLIT ? ctx->split_lanes : 0u;
+}
 
 struct grt_scene_t {
     grt_context_t* ctx = nullptr;

@@ -153,10 +153,6 @@ struct TraceArgs {
     uint32_t n;
     uint32_t image_width;   // 0: lane i traces ray i; else 8x8 pixel tiles per wave
     uint32_t* counters;     // NULL or 2 per ray {cells, tests}
-    uint32_t coop;          // wave-cooperative tests of dense cells: at least this many
-                            // references left (0: off)
-    uint32_t pool;          // one-ray-per-lane kernels: pool the wave's tests (1) or
-                            // test per lane (0)
     const uint32_t* list = nullptr;        // or the rays to trace: slot s traces list[s] ...
     const uint32_t* list_count = nullptr;  // ... for s < *list_count (a device value) and s < n
     // Two-level grid (all set, or cellrec NULL for the top grid alone).  The
@@ -167,29 +163,20 @@ struct TraceArgs {
     const float4* sub_trir = nullptr;
     const float* sub_tab = nullptr;        // 96 floats: sub-cell sizes, reciprocals (G2Build)
 };
-hipError_t launch_trace_closest(const TraceArgs& a, const RaySoA& rays, const HitSoA& hits,
-                                uint32_t block, hipStream_t s);
+// Closest hit into hits, or any hit into occluded when `any`: waves walk their
+// rays in windows of cells, the tests of a window spread over the wave, with
+// `lanes` (1, 2, 4, 8 or 16) lanes per ray, or 0 for a number chosen by the
+// size of the launch.
+hipError_t launch_trace_window(const TraceArgs& a, const RaySoA& rays, const HitSoA& hits,
+                               uint8_t* occluded, bool any, uint32_t lanes, uint32_t block,
+                               hipStream_t s);
 // Two-level traversal (a.cellrec set): closest hit into hits, or any hit into
 // occluded when it is set; one ray per lane (lanes <= 1) or `lanes` (2..16)
 // lanes per ray walking its top cells in turn.
 hipError_t launch_trace2(const TraceArgs& a, const RaySoA& rays, const HitSoA& hits,
                          uint8_t* occluded, uint32_t lanes, hipStream_t s);
-hipError_t launch_trace_any(const TraceArgs& a, const RaySoA& rays, uint8_t* occluded,
-                            uint32_t block, hipStream_t s);
-// Persistent traversal (closest hit, or any hit when `any`): lanes refill
-// from the slot counter (one uint32, zeroed by the launcher) once `refill`
-// lanes of a wave are idle.
-hipError_t launch_trace_persistent(const TraceArgs& a, const RaySoA& rays, const HitSoA& hits,
-                                   uint8_t* occluded, bool any, uint32_t* slot_counter,
-                                   uint32_t block, uint32_t refill, hipStream_t s);
 // One item of a batched launch: a ray batch against one scene's grid.  The
 // slot range [slot_begin, slot_begin + slots) is padded to whole waves (64).
-// Several lanes per ray (2, 4, 8 or 16): lane j of a ray's group visits the
-// ray's cells j, j + lanes, ... of the serial order (schedule GRT_TRACE_SPLIT).
-hipError_t launch_trace_split(const TraceArgs& a, const RaySoA& rays, const HitSoA& hits,
-                              uint8_t* occluded, bool any, uint32_t lanes, uint32_t block,
-                              hipStream_t s);
-
 struct alignas(16) BatchTask {
     const DevFrame* fr;
     const uint32_t* offsets;
@@ -208,13 +195,10 @@ struct alignas(16) BatchTask {
 // Map each 64-slot block to its task (n_blocks entries).
 hipError_t launch_task_map(const BatchTask* tasks, uint32_t n_tasks, uint32_t* map,
                            hipStream_t s);
-// Multi-scene traversal over all tasks (mixed closest / any hit) with the
-// schedule `mode` (GRT_TRACE_*): one ray per lane (each wave in one task), with
-// per-lane or pooled tests; `lanes` lanes per ray (2, 4, 8 or 16); or
-// persistent waves refilled from the slot counter.
+// Multi-scene traversal over all tasks (mixed closest / any hit), each wave in
+// one task; lanes as for launch_trace_window.
 hipError_t launch_trace_batch(const BatchTask* tasks, const uint32_t* map, uint32_t total_slots,
-                              uint32_t* slot_counter, int mode, uint32_t block,
-                              uint32_t refill, uint32_t lanes, uint32_t coop, hipStream_t s);
+                              uint32_t lanes, uint32_t block, hipStream_t s);
 hipError_t launch_gen_primary(const DevCamera& cam, const RaySoAOut& out, hipStream_t s);
 hipError_t launch_gen_shadow(uint32_t n, const RaySoA& in, const HitSoAIn& hits,
                              const float* normals, float lx, float ly, float lz, float offset,

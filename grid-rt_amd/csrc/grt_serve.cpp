@@ -12,7 +12,7 @@
 // (GpuRenderer.cpp:74-319; cudaRayTrace, RayTracing.cu:227-253).
 //
 // Continuous batching: each round gathers the next step of every admitted
-// request into one batched persistent launch (grt_batch).  Rounds are
+// request into one batched launch (grt_batch).  Rounds are
 // pipelined on the stream -- up to two in flight, step j+1 of a request queued
 // behind step j by stream order alone -- so the host never waits for a round
 // before issuing the next, and only retires requests (their last round's event)
@@ -463,22 +463,9 @@ private:
             a.n = it.n;
             a.image_width = it.width;
             a.counters = nullptr;
-            a.coop = ctx_->coop;
-            a.pool = ctx_->trace_mode == GRT_TRACE_POOLED ? 1u : 0u;
-            hipError_t e;
-            if (ctx_->trace_mode == GRT_TRACE_PERSISTENT)
-                e = launch_trace_persistent(a, it.rays.in(), it.hits.out(), it.occ, it.any,
-                                            it.sc->small_counters.as<uint32_t>() + 2,
-                                            it.any ? ctx_->block_any : ctx_->block_closest,
-                                            ctx_->refill, s);
-            else if (ctx_->trace_mode == GRT_TRACE_SPLIT)
-                e = launch_trace_split(a, it.rays.in(), it.hits.out(), it.occ, it.any,
-                                       ctx_->split_lanes,
-                                       it.any ? ctx_->block_any : ctx_->block_closest, s);
-            else if (it.any)
-                e = launch_trace_any(a, it.rays.in(), it.occ, ctx_->block_any, s);
-            else
-                e = launch_trace_closest(a, it.rays.in(), it.hits.out(), ctx_->block_closest, s);
+            const hipError_t e = launch_trace_window(
+                a, it.rays.in(), it.hits.out(), it.occ, it.any, window_lanes_of(ctx_),
+                it.any ? ctx_->block_any : ctx_->block_closest, s);
             if (e != hipSuccess)
                 return hip_check(e, "serve: trace");
         }

@@ -1,4 +1,4 @@
-// grt_traverse.hip -- one-ray-per-lane 3D-DDA traversal of the uniform grid
+// grt_traverse.hip -- 3D-DDA traversal of the uniform grid
 // with Moller-Trumbore intersection, on gfx950 (wave64).
 //
 // Reference semantics:
@@ -14,18 +14,14 @@
 // lanes); the grid is offsets[m+1] (uint32) plus one 48-byte record per
 // reference, trir[k] = {v0.xyz, e1.x}{e1.yz, e2.xy}{e2.z, id, -, -}, stored
 // contiguously per cell, so a cell's triangles stream without an index
-// indirection.  Each traversal loop loads the next record while the current
-// one is tested.
+// indirection.
 //
-// Two schedules with identical per-ray results:
-//   k_trace_closest / k_trace_any   one ray per lane for the whole launch;
-//       when every active lane of a wave is in the same cell the records are
-//       read with wave-uniform (scalar) loads;
-//   k_trace_persistent              persistent waves that refill idle lanes
-//       from a shared slot counter and advance each lane by one work item
-//       (one triangle test or one cell) per iteration.
+//   k_trace_window        one-level grid, 1..16 lanes per ray (grt_window.h)
+//   k_trace_batch_window  the same over the items of a batch
+//   k_trace2, _split      two-level grid
 #include "grt_launch.h"
 #include "grt_mt.h"
+#include "grt_window.h"
 
 namespace grt {
 
@@ -109,605 +105,60 @@ __device__ __forceinline__ bool dda_setup(const DevFrame* __restrict__ fr, float
     return true;
 }
 
-// Single-axis advance with the reference tie order.  False when leaving.
-__device__ __forceinline__ bool dda_step(Dda& s)
-{
-    if (s.tx < s.ty && s.tx < s.tz) {
-        s.cx += s.sx;
-        if (s.cx == s.ox)
-            return false;
-        s.tx += s.dtx;
-    } else if (s.ty < s.tz) {
-        s.cy += s.sy;
-        if (s.cy == s.oy)
-            return false;
-        s.ty += s.dty;
-    } else {
-        s.cz += s.sz;
-        if (s.cz == s.oz)
-            return false;
-        s.tz += s.dtz;
-    }
-    return true;
-}
-
-
 // ---------------------------------------------------------------------------
-// Wave-cooperative cell tests
+// One-level grid: windowed walk
 // ---------------------------------------------------------------------------
-//
-// Once a persistent wave finds the ray queue drained, its last rays would run
-// their remaining triangle tests one per iteration on single lanes while the
-// other lanes idle; a ray through a dense cell (thousands of references) then
-// sets the length of the whole launch.  In that phase the wave instead tests
-// the rest of such a cell 64 references at a time, one per lane.  The result
-// is the serial one: closest hit keeps the smallest t and, among equal t, the
-// earliest reference (a lexicographic (t, reference) minimum, since the serial
-// loop only replaces on a strictly smaller t); any hit stops at the first
-// occluding reference in order, and the test counter counts the references the
-// serial loop would have tested.
 
-__device__ __forceinline__ float bcast_f(float v, uint32_t l)
-{
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), (int)l));
-}
-
-__device__ __forceinline__ uint32_t bcast_u(uint32_t v, uint32_t l)
-{
-    return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l);
-}
-
-template <class T>
-__device__ __forceinline__ T* bcast_p(T* p, uint32_t l)
-{
-    const uint64_t x = (uint64_t)p;
-    const uint64_t lo = bcast_u((uint32_t)x, l), hi = bcast_u((uint32_t)(x >> 32), l);
-    return (T*)((hi << 32) | lo);
-}
-
-__device__ __forceinline__ float wave_min_f(float v)
-{
-    for (int o = 32; o > 0; o >>= 1)
-        v = tmin_f(v, __shfl_xor(v, o, 64));
-    return v;
-}
-
-__device__ __forceinline__ uint32_t wave_min_u(uint32_t v)
-{
-    for (int o = 32; o > 0; o >>= 1) {
-        const uint32_t w = (uint32_t)__shfl_xor((int)v, o, 64);
-        v = w < v ? w : v;
-    }
-    return v;
-}
-
-// State of one lane's ray that the cooperative pass reads and updates.
-struct LaneRay {
-    float o0, o1, o2, d0, d1, d2, tmin, tmax, bound;
-    uint32_t k, e;        // references [k, e) of the current cell are left
-    int32_t id;
-    float best, bu, bv;
-    uint32_t tests;
+// The DDA of a windowed walk: the current cell's index with one stride per
+// axis, and the steps left on each axis before the ray leaves the grid.
+struct DdaW {
+    uint32_t ci, sx, sy, sz;
+    uint32_t rx, ry, rz;
+    float tx, ty, tz, dtx, dty, dtz;
 };
 
-// The whole wave (every lane, uniform control flow) finishes the current cell
-// of lane l: records [k, e) of `trir` (lane l's grid).  Updates lane l's k,
-// hit and test count.
-__device__ __forceinline__ void coop_cell(uint32_t l, bool any, const float4* trir, LaneRay& r)
+__device__ __forceinline__ DdaW dda_window(const DevFrame* __restrict__ fr, const Dda& s)
 {
-    const uint32_t lane = threadIdx.x & 63u;
-    const float o0 = bcast_f(r.o0, l), o1 = bcast_f(r.o1, l), o2 = bcast_f(r.o2, l);
-    const float d0 = bcast_f(r.d0, l), d1 = bcast_f(r.d1, l), d2 = bcast_f(r.d2, l);
-    const float tmin = bcast_f(r.tmin, l), tmax = bcast_f(r.tmax, l);
-    const uint32_t kb = bcast_u(r.k, l), ke = bcast_u(r.e, l);
-    const float4* __restrict__ tr = bcast_p(trir, l);
-    if (any) {
-        uint32_t first = 0xffffffffu;
-        for (uint32_t base = kb; base < ke; base += 64u) {
-            const uint32_t kk = base + lane;
-            bool h = false;
-            if (kk < ke) {
-                const float4 A = tr[3ull * kk], B = tr[3ull * kk + 1], C = tr[3ull * kk + 2];
-                h = any_test(A, B, C, o0, o1, o2, d0, d1, d2, tmin, tmax);
-            }
-            const uint64_t hm = __ballot(h);
-            if (hm != 0) {
-                first = base + (uint32_t)__builtin_ctzll(hm);
-                break;
-            }
-        }
-        if (lane == l) {
-            if (first != 0xffffffffu) {
-                r.tests += first - kb + 1u;
-                r.id = 1;
-            } else {
-                r.tests += ke - kb;
-            }
-            r.k = ke;
-        }
-        return;
-    }
-    const float bound = bcast_f(r.bound, l), best0 = bcast_f(r.best, l);
-    float lb = best0, lu = 0.0f, lv = 0.0f;
-    int32_t lid = -1;
-    uint32_t lk = 0xffffffffu;
-    for (uint32_t base = kb; base < ke; base += 64u) {
-        const uint32_t kk = base + lane;
-        if (kk < ke) {
-            const float4 A = tr[3ull * kk], B = tr[3ull * kk + 1], C = tr[3ull * kk + 2];
-            const MtPre m = mt_pre(A, B, C, o0, o1, o2, d0, d1, d2);
-            if (mt_maybe(m, tmin, tmin_f(tmin_f(tmax, bound), lb))) {
-                float t, u, v;
-                if (mt_exact(m, t, u, v) && t > tmin && t <= tmax && t <= bound && t < lb) {
-                    lb = t;
-                    lu = u;
-                    lv = v;
-                    lid = (int32_t)__float_as_uint(C.y);
-                    lk = kk;
-                }
-            }
-        }
-    }
-    const float mt = wave_min_f(lb);
-    const uint32_t mk = wave_min_u((lk != 0xffffffffu && lb == mt) ? lk : 0xffffffffu);
-    if (mk != 0xffffffffu) {
-        const uint32_t w = (uint32_t)__builtin_ctzll(__ballot(lk == mk));
-        const int32_t wid = (int32_t)bcast_u((uint32_t)lid, w);
-        const float wu = bcast_f(lu, w), wv = bcast_f(lv, w);
-        if (lane == l) {
-            r.best = mt;
-            r.id = wid;
-            r.bu = wu;
-            r.bv = wv;
-        }
-    }
-    if (lane == l) {
-        r.tests += ke - kb;
-        r.k = ke;
-    }
+    const uint32_t nx = (uint32_t)fr->n[0], ny = (uint32_t)fr->n[1], nxy = nx * ny;
+    DdaW w;
+    w.ci = (uint32_t)s.cx + nx * ((uint32_t)s.cy + ny * (uint32_t)s.cz);
+    w.sx = s.sx < 0 ? ~0u : 1u;
+    w.sy = s.sy < 0 ? 0u - nx : nx;
+    w.sz = s.sz < 0 ? 0u - nxy : nxy;
+    w.rx = (uint32_t)(s.sx < 0 ? s.cx : s.ox - 1 - s.cx);
+    w.ry = (uint32_t)(s.sy < 0 ? s.cy : s.oy - 1 - s.cy);
+    w.rz = (uint32_t)(s.sz < 0 ? s.cz : s.oz - 1 - s.cz);
+    w.tx = s.tx;
+    w.ty = s.ty;
+    w.tz = s.tz;
+    w.dtx = s.dtx;
+    w.dty = s.dty;
+    w.dtz = s.dtz;
+    return w;
 }
 
-// Lanes whose current cell is worth a cooperative pass now: the queue is
-// drained for this wave and at least max(coop, 2 x busy lanes) references
-// are left.
-__device__ __forceinline__ uint64_t coop_lanes(bool busy, bool drained_lane, uint32_t k,
-                                               uint32_t e, uint32_t coop)
+// One step (dda_step's tie order) when `go`; false when the ray does not go
+// on (the state then stays in the grid).
+__device__ __forceinline__ bool dda_window_step(DdaW& w, bool go)
 {
-    if (coop == 0 || __ballot(drained_lane) == 0)
-        return 0;
-    const uint32_t nb = (uint32_t)__popcll(__ballot(busy));
-    const uint32_t thr = coop > 2u * nb ? coop : 2u * nb;
-    return __ballot(busy && k < e && e - k >= thr);
-}
-
-// ---------------------------------------------------------------------------
-// Pooled tests (one ray per lane)
-// ---------------------------------------------------------------------------
-//
-// With rays in different cells, a per-lane loop over each lane's references
-// leaves most lanes idle (the wave runs as long as its fullest cell).  Pooled,
-// the (lane, reference) pairs of all the wave's current cells are numbered
-// through an exclusive scan of the lanes' counts and tested 64 at a time, one
-// pair per lane, the owner's ray read from LDS.  Closest hit keeps, per owner,
-// the minimum of (t, reference) in an LDS 64-bit atomic -- t mapped to an
-// order-preserving integer with -0 folded into +0 -- which is the reference
-// the serial loop would keep (it replaces only on a strictly smaller t); the
-// winner's u, v are then recomputed by the owner with the same arithmetic.
-// Any hit keeps the first occluding offset; the test counter counts what the
-// serial loop would have tested.
-
-// LDS staging of one wave.
-struct WavePool {
-    float o0[64], o1[64], o2[64], d0[64], d1[64], d2[64], tmin[64], tmax[64], bound[64];
-    uint32_t pre[64];                // exclusive prefix of the lanes' reference counts
-    uint32_t kb[64];                 // first reference of each lane's cell
-    unsigned long long win[64];      // per owner: (t, reference) minimum / first occluder
-};
-
-__device__ __forceinline__ uint32_t ordered_bits(float t)
-{
-    const uint32_t b = __float_as_uint(t == 0.0f ? 0.0f : t);
-    return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
-}
-
-__device__ __forceinline__ void pool_store_ray(WavePool& P, const LaneRay& r)
-{
-    const uint32_t lane = threadIdx.x & 63u;
-    P.o0[lane] = r.o0;
-    P.o1[lane] = r.o1;
-    P.o2[lane] = r.o2;
-    P.d0[lane] = r.d0;
-    P.d1[lane] = r.d1;
-    P.d2[lane] = r.d2;
-    P.tmin[lane] = r.tmin;
-    P.tmax[lane] = r.tmax;
-}
-
-// Owner of pair p: the last lane whose prefix is <= p.
-__device__ __forceinline__ uint32_t pool_owner(const WavePool& P, uint32_t p)
-{
-    uint32_t o = 0;
-#pragma unroll
-    for (uint32_t step = 32; step > 0; step >>= 1)
-        if (P.pre[o + step] <= p)
-            o += step;
-    return o;
-}
-
-// The whole wave tests every lane's references [k, k + c) (c = 0 for lanes
-// without work); each lane's hit and test count are updated as by the serial
-// loop and its cell is consumed.
-template <bool ANY>
-__device__ __forceinline__ void pool_cells(WavePool& P, const float4* __restrict__ trir,
-                                           LaneRay& r, uint32_t c)
-{
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t incl = wave_incl_scan(c);
-    const uint32_t total = bcast_u(incl, 63);
-    P.pre[lane] = incl - c;
-    P.kb[lane] = r.k;
-    P.bound[lane] = r.bound;
-    P.win[lane] = ~0ull;
-    wave_lds_sync();
-    for (uint32_t base = 0; base < total; base += 64u) {
-        const uint32_t p = base + lane;
-        if (p < total) {
-            const uint32_t o = pool_owner(P, p);
-            const uint32_t j = p - P.pre[o];
-            const uint32_t ref = P.kb[o] + j;
-            if (ANY && P.win[o] < j)
-                continue;   // the owner has an earlier occluder already
-            const float4 A = trir[3ull * ref], B = trir[3ull * ref + 1], C = trir[3ull * ref + 2];
-            const float o0 = P.o0[o], o1 = P.o1[o], o2 = P.o2[o];
-            const float d0 = P.d0[o], d1 = P.d1[o], d2 = P.d2[o];
-            const float tmin = P.tmin[o], tmax = P.tmax[o];
-            if (ANY) {
-                if (any_test(A, B, C, o0, o1, o2, d0, d1, d2, tmin, tmax))
-                    atomicMin(&P.win[o], (unsigned long long)j);
-            } else {
-                const float bound = P.bound[o];
-                const MtPre m = mt_pre(A, B, C, o0, o1, o2, d0, d1, d2);
-                if (mt_maybe(m, tmin, tmin_f(tmax, bound))) {
-                    float t, u, v;
-                    if (mt_exact(m, t, u, v) && t > tmin && t <= tmax && t <= bound)
-                        atomicMin(&P.win[o], ((unsigned long long)ordered_bits(t) << 32) | ref);
-                }
-            }
-        }
-    }
-    wave_lds_sync();
-    if (c == 0)
-        return;
-    const unsigned long long w = P.win[lane];
-    if (ANY) {
-        if (w != ~0ull) {
-            r.id = 1;
-            r.tests += (uint32_t)w + 1u;
-        } else {
-            r.tests += c;
-        }
-    } else {
-        if (w != ~0ull) {
-            const uint32_t ref = (uint32_t)w;
-            const float4 A = trir[3ull * ref], B = trir[3ull * ref + 1], C = trir[3ull * ref + 2];
-            const MtPre m = mt_pre(A, B, C, r.o0, r.o1, r.o2, r.d0, r.d1, r.d2);
-            float t, u, v;
-            mt_exact(m, t, u, v);
-            r.best = t;
-            r.bu = u;
-            r.bv = v;
-            r.id = (int32_t)__float_as_uint(C.y);
-        }
-        r.tests += c;
-    }
-    r.k = r.e;
-}
-
-// ---------------------------------------------------------------------------
-// One ray per lane
-// ---------------------------------------------------------------------------
-//
-// Each iteration of the wave-uniform loop handles one cell per busy lane:
-//   1. the cooperative pass (cells with many references, when the busy lanes
-//      of the wave are not all in one cell),
-//   2. the remaining references of each lane's cell -- with wave-uniform
-//      (scalar) record loads when every busy lane is in the same cell,
-//   3. finish (hit in this cell / ray leaves its interval or the grid) or step
-//      to the next cell.
-
-// Lanes for a cooperative pass in the one-ray-per-lane kernels: none when all
-// busy lanes share one cell (the scalar path serves them better), else those
-// with at least max(coop, 2 x busy lanes) references left.
-__device__ __forceinline__ uint64_t coop_lanes_simple(bool busy, uint32_t k, uint32_t e,
-                                                      uint32_t coop)
-{
-    if (coop == 0)
-        return 0;
-    const uint64_t bm = __ballot(busy);
-    const uint32_t f = (uint32_t)__builtin_ctzll(bm);
-    const uint32_t k0 = bcast_u(k, f), e0 = bcast_u(e, f);
-    if (__ballot(busy && (k != k0 || e != e0)) == 0)
-        return 0;
-    const uint32_t nb = (uint32_t)__popcll(bm);
-    const uint32_t thr = coop > 2u * nb ? coop : 2u * nb;
-    return __ballot(busy && k < e && e - k >= thr);
-}
-
-// Current cell of a lane: exit distance, reference range, hit bound.
-__device__ __forceinline__ void load_cell(const Dda& s, const uint32_t* __restrict__ offsets,
-                                          uint32_t nx, uint32_t ny, float& exit_t, float& bound,
-                                          uint32_t& k, uint32_t& e)
-{
-    exit_t = tmin_f(tmin_f(s.tx, s.ty), s.tz);
-    const uint32_t ci = (uint32_t)s.cx + nx * ((uint32_t)s.cy + ny * (uint32_t)s.cz);
-    k = offsets[ci];
-    e = offsets[ci + 1];
-    bound = exit_t * kExitScale;
-}
-
-// Closest hit of ray i (valid lanes) against one grid; every lane of the wave
-// calls it together.
-template <bool COUNT, bool POOL>
-__device__ __forceinline__ void trace_closest_lane(const DevFrame* __restrict__ fr,
-                                                   const uint32_t* __restrict__ offsets,
-                                                   const float4* __restrict__ trir,
-                                                   const RaySoA& rays, const HitSoA& hits,
-                                                   uint32_t* __restrict__ counters, uint32_t coop,
-                                                   uint32_t i, bool valid, WavePool* pool)
-{
-    const KF4 ktr = (KF4)trir;
-    LaneRay r = {};
-    r.id = -1;
-    r.best = INFINITY;
-    uint32_t cells = 0;
-    Dda s = {};
-    bool busy = false;
-    const uint32_t nx = (uint32_t)fr->n[0], ny = (uint32_t)fr->n[1];
-    if (valid) {
-        r.o0 = rays.ox[i];
-        r.o1 = rays.oy[i];
-        r.o2 = rays.oz[i];
-        r.d0 = rays.dx[i];
-        r.d1 = rays.dy[i];
-        r.d2 = rays.dz[i];
-        r.tmin = rays.tmin[i];
-        r.tmax = rays.tmax[i];
-        busy = grid_ok(fr) && dda_setup(fr, r.o0, r.o1, r.o2, r.d0, r.d1, r.d2, r.tmin, r.tmax, s);
-    }
-    if (POOL)
-        pool_store_ray(*pool, r);
-    float exit_t = 0.0f;
-    if (busy) {
-        load_cell(s, offsets, nx, ny, exit_t, r.bound, r.k, r.e);
-        cells = 1;
-    }
-    while (__ballot(busy) != 0) {
-        bool pooled = false;
-        if (POOL) {
-            const uint32_t c = (busy && r.k < r.e) ? r.e - r.k : 0u;
-            const uint64_t cm = __ballot(c != 0);
-            if (cm != 0) {
-                const uint32_t f = (uint32_t)__builtin_ctzll(cm);
-                const uint32_t k0 = bcast_u(r.k, f), e0 = bcast_u(r.e, f);
-                if (__ballot(c != 0 && (r.k != k0 || r.e != e0)) != 0) {
-                    pool_cells<false>(*pool, trir, r, c);
-                    pooled = true;
-                }
-            }
-        } else if (const uint64_t hv0 = coop_lanes_simple(busy, r.k, r.e, coop)) {
-            for (uint64_t hv = hv0; hv != 0; hv &= hv - 1)
-                coop_cell((uint32_t)__builtin_ctzll(hv), false, trir, r);
-        }
-        if (!pooled && busy && r.k < r.e) {
-            const uint32_t b = r.k, e = r.e;
-            const uint32_t b0 = __builtin_amdgcn_readfirstlane(b);
-            const uint32_t e0 = __builtin_amdgcn_readfirstlane(e);
-            if (__ballot(b != b0 || e != e0) == 0) {
-                // Every lane here is in this cell: wave-uniform records.
-                test_records<false>(ktr, b0, e0, r.o0, r.o1, r.o2, r.d0, r.d1, r.d2, r.tmin,
-                                    r.tmax, r.bound, r.id, r.best, r.bu, r.bv, r.tests);
-            } else {
-                test_records<false>(trir, b, e, r.o0, r.o1, r.o2, r.d0, r.d1, r.d2, r.tmin,
-                                    r.tmax, r.bound, r.id, r.best, r.bu, r.bv, r.tests);
-            }
-            r.k = e;
-        }
-        if (busy) {
-            if (r.id >= 0 || exit_t > r.tmax || !dda_step(s)) {
-                busy = false;
-            } else {
-                load_cell(s, offsets, nx, ny, exit_t, r.bound, r.k, r.e);
-                ++cells;
-            }
-        }
-    }
-    if (valid) {
-        hits.id[i] = r.id;
-        hits.t[i] = r.best;
-        hits.u[i] = r.bu;
-        hits.v[i] = r.bv;
-        if (COUNT) {
-            counters[2ull * i] = cells;
-            counters[2ull * i + 1] = r.tests;
-        }
-    }
-}
-
-// Any hit of ray i (valid lanes) against one grid; every lane of the wave calls
-// it together.
-template <bool COUNT, bool POOL>
-__device__ __forceinline__ void trace_any_lane(const DevFrame* __restrict__ fr,
-                                               const uint32_t* __restrict__ offsets,
-                                               const float4* __restrict__ trir,
-                                               const RaySoA& rays, uint8_t* __restrict__ occluded,
-                                               uint32_t* __restrict__ counters, uint32_t coop,
-                                               uint32_t i, bool valid, WavePool* pool)
-{
-    const KF4 ktr = (KF4)trir;
-    LaneRay r = {};
-    r.id = -1;
-    uint32_t cells = 0;
-    Dda s = {};
-    bool busy = false;
-    const uint32_t nx = (uint32_t)fr->n[0], ny = (uint32_t)fr->n[1];
-    if (valid) {
-        r.o0 = rays.ox[i];
-        r.o1 = rays.oy[i];
-        r.o2 = rays.oz[i];
-        r.d0 = rays.dx[i];
-        r.d1 = rays.dy[i];
-        r.d2 = rays.dz[i];
-        r.tmin = rays.tmin[i];
-        r.tmax = rays.tmax[i];
-        busy = grid_ok(fr) && dda_setup(fr, r.o0, r.o1, r.o2, r.d0, r.d1, r.d2, r.tmin, r.tmax, s);
-    }
-    if (POOL)
-        pool_store_ray(*pool, r);
-    float exit_t = 0.0f;
-    if (busy) {
-        load_cell(s, offsets, nx, ny, exit_t, r.bound, r.k, r.e);
-        cells = 1;
-    }
-    while (__ballot(busy) != 0) {
-        bool pooled = false;
-        if (POOL) {
-            const uint32_t c = (busy && r.k < r.e) ? r.e - r.k : 0u;
-            const uint64_t cm = __ballot(c != 0);
-            if (cm != 0) {
-                const uint32_t f = (uint32_t)__builtin_ctzll(cm);
-                const uint32_t k0 = bcast_u(r.k, f), e0 = bcast_u(r.e, f);
-                if (__ballot(c != 0 && (r.k != k0 || r.e != e0)) != 0) {
-                    pool_cells<true>(*pool, trir, r, c);
-                    pooled = true;
-                }
-            }
-        } else if (const uint64_t hv0 = coop_lanes_simple(busy, r.k, r.e, coop)) {
-            for (uint64_t hv = hv0; hv != 0; hv &= hv - 1)
-                coop_cell((uint32_t)__builtin_ctzll(hv), true, trir, r);
-        }
-        if (!pooled && busy && r.k < r.e) {
-            const uint32_t b = r.k, e = r.e;
-            const uint32_t b0 = __builtin_amdgcn_readfirstlane(b);
-            const uint32_t e0 = __builtin_amdgcn_readfirstlane(e);
-            int32_t nid = -1;
-            float nt = 0.0f, nu = 0.0f, nv = 0.0f;
-            // references tested: up to and including an occluder
-            const bool occ =
-                __ballot(b != b0 || e != e0) == 0
-                    ? test_records<true>(ktr, b0, e0, r.o0, r.o1, r.o2, r.d0, r.d1, r.d2, r.tmin,
-                                         r.tmax, 0.0f, nid, nt, nu, nv, r.tests)
-                    : test_records<true>(trir, b, e, r.o0, r.o1, r.o2, r.d0, r.d1, r.d2, r.tmin,
-                                         r.tmax, 0.0f, nid, nt, nu, nv, r.tests);
-            if (occ)
-                r.id = 1;
-            r.k = e;
-        }
-        if (busy) {
-            if (r.id >= 0 || exit_t > r.tmax || !dda_step(s)) {
-                busy = false;
-            } else {
-                load_cell(s, offsets, nx, ny, exit_t, r.bound, r.k, r.e);
-                ++cells;
-            }
-        }
-    }
-    if (valid) {
-        occluded[i] = r.id >= 0 ? 1 : 0;
-        if (COUNT) {
-            counters[2ull * i] = cells;
-            counters[2ull * i + 1] = r.tests;
-        }
-    }
-}
-
-template <bool COUNT, bool POOL>
-__global__ __launch_bounds__(256) void k_trace_closest(TraceArgs a, RaySoA rays, HitSoA hits)
-{
-    __shared__ WavePool pools[POOL ? 4 : 1];
-    bool valid;
-    const uint32_t i = trace_ray(a, blockIdx.x * blockDim.x + threadIdx.x, valid);
-    trace_closest_lane<COUNT, POOL>(a.fr, a.offsets, a.trir, rays, hits, a.counters, a.coop, i,
-                                    valid, POOL ? &pools[threadIdx.x >> 6] : nullptr);
-}
-
-template <bool COUNT, bool POOL>
-__global__ __launch_bounds__(256) void k_trace_any(TraceArgs a, RaySoA rays,
-                                                   uint8_t* __restrict__ occluded)
-{
-    __shared__ WavePool pools[POOL ? 4 : 1];
-    bool valid;
-    const uint32_t i = trace_ray(a, blockIdx.x * blockDim.x + threadIdx.x, valid);
-    trace_any_lane<COUNT, POOL>(a.fr, a.offsets, a.trir, rays, occluded, a.counters, a.coop, i,
-                                valid, POOL ? &pools[threadIdx.x >> 6] : nullptr);
-}
-
-// Batched multi-scene traversal, one ray per lane: every 64-slot group belongs
-// to one task (map[slot / 64]), so each wave runs the single-scene loop of its
-// task with wave-uniform scene data.
-template <bool POOL>
-__global__ __launch_bounds__(256) void k_trace_batch_simple(const BatchTask* __restrict__ tasks,
-                                                            const uint32_t* __restrict__ map,
-                                                            uint32_t total_slots, uint32_t coop)
-{
-    __shared__ WavePool pools[POOL ? 4 : 1];
-    WavePool* pool = POOL ? &pools[threadIdx.x >> 6] : nullptr;
-    const uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t group = __builtin_amdgcn_readfirstlane(slot >> 6);
-    if ((group << 6) >= total_slots)
-        return;   // whole waves only: total_slots is a multiple of 64
-    const uint32_t task = __builtin_amdgcn_readfirstlane(map[group]);
-    const BatchTask& T = tasks[task];
-    bool valid;
-    const uint32_t i = slot_ray(slot - T.slot_begin, T.image_width, T.n, valid);
-    if (T.any)
-        trace_any_lane<false, POOL>(T.fr, T.offsets, T.trir, T.rays, T.occluded, nullptr, coop, i,
-                                    valid, pool);
-    else
-        trace_closest_lane<false, POOL>(T.fr, T.offsets, T.trir, T.rays, T.hits, nullptr, coop, i,
-                                        valid, pool);
-}
-
-// ---------------------------------------------------------------------------
-// Several lanes per ray
-// ---------------------------------------------------------------------------
-//
-// A launch with few rays (secondary rays of a few pixels, a small request)
-// leaves most SIMDs with one wave or none, and each lane then pays the memory
-// latency of every cell and record of its ray in series.  Here a group of
-// `lanes` (2..16, a power of two) adjacent lanes shares one ray: lane j of the
-// group visits the ray's cells j, j + lanes, j + 2 lanes, ... of the serial
-// DDA order, stepping the DDA on registers in between.  After each round the
-// group keeps the earliest cell (lowest ordinal) that holds a hit -- the cell
-// where the serial loop would have stopped -- and discards later cells, so
-// hits, occlusion flags and the {cells, tests} counters equal the serial
-// ones.  Dense cells get the wave-cooperative pass as in the one-ray-per-lane
-// kernels.
-
-// Advance by `count` cells of the serial order: false when the ray's interval
-// ends in the current cell (its exit beyond tmax) or the ray leaves the grid.
-__device__ __forceinline__ bool dda_skip(Dda& s, uint32_t count, float tmax)
-{
-    for (uint32_t q = 0; q < count; ++q)
-        if (tmin_f(tmin_f(s.tx, s.ty), s.tz) > tmax || !dda_step(s))
-            return false;
-    return true;
-}
-
-// Serial tests of the rest of a lane's current cell, per-lane (vector) loads.
-template <bool ANY>
-__device__ __forceinline__ void lane_cell(const float4* __restrict__ trir, LaneRay& r)
-{
-    if (ANY) {
-        int32_t nid = -1;
-        float nt = 0.0f, nu = 0.0f, nv = 0.0f;
-        if (test_records<true>(trir, r.k, r.e, r.o0, r.o1, r.o2, r.d0, r.d1, r.d2, r.tmin,
-                               r.tmax, 0.0f, nid, nt, nu, nv, r.tests))
-            r.id = 1;
-    } else {
-        test_records<false>(trir, r.k, r.e, r.o0, r.o1, r.o2, r.d0, r.d1, r.d2, r.tmin, r.tmax,
-                            r.bound, r.id, r.best, r.bu, r.bv, r.tests);
-    }
-    r.k = r.e;
+    const bool ax = w.tx < w.ty && w.tx < w.tz;
+    const bool ay = !ax && w.ty < w.tz;
+    // values, not lvalues: a conditional over fields would select addresses
+    // and send the walk's state to scratch memory
+    const uint32_t rx = w.rx, ry = w.ry, rz = w.rz, sx = w.sx, sy = w.sy, sz = w.sz;
+    const uint32_t left = ax ? uint32_t(rx) : (ay ? uint32_t(ry) : uint32_t(rz));
+    go = go && left != 0;
+    const bool mx = go && ax, my = go && ay, mz = go && !ax && !ay;
+    const float tx = w.tx + w.dtx, ty = w.ty + w.dty, tz = w.tz + w.dtz;
+    w.tx = mx ? tx : w.tx;
+    w.ty = my ? ty : w.ty;
+    w.tz = mz ? tz : w.tz;
+    w.rx -= mx ? 1u : 0u;
+    w.ry -= my ? 1u : 0u;
+    w.rz -= mz ? 1u : 0u;
+    const uint32_t d = ax ? uint32_t(sx) : (ay ? uint32_t(sy) : uint32_t(sz));
+    w.ci += go ? d : 0u;
+    return go;
 }
 
 // Sum over the `lanes`-lane group (every lane of the wave calls it).
@@ -718,121 +169,156 @@ __device__ __forceinline__ uint32_t group_sum(uint32_t v, uint32_t lanes)
     return v;
 }
 
-// Ray i (valid: the whole group) traced by its group of `lanes` lanes.
-template <bool ANY, bool COUNT>
-__device__ __forceinline__ void trace_split_lane(const DevFrame* __restrict__ fr,
-                                                 const uint32_t* __restrict__ offsets,
-                                                 const float4* __restrict__ trir,
-                                                 const RaySoA& rays, const HitSoA& hits,
-                                                 uint8_t* __restrict__ occluded,
-                                                 uint32_t* __restrict__ counters, uint32_t coop,
-                                                 uint32_t lanes, uint32_t i, bool valid)
+// Bound by VALU issue (0.70-0.85 of the cycles) with 51-60 of 64 lanes active
+// per instruction; the per-lane loops this replaced ran 10-30 lanes and one
+// memory latency per cell and test.  Before and after, us: 512x512 spheres
+// (16k triangles) primary 121 -> 51, bounce 238 -> 43; stadium (lambda 128,
+// 1280x720) primary 3294 -> 1585, shadow 3100 -> 1739; 1.2 M-slot batch
+// 1197 -> 552.
+//
+// Ray i (valid: the whole group) against one grid, traced by a group of
+// `lanes` lanes (1..16, a power of two) in windows of lanes x c cells, c =
+// min(S, 16 / lanes), lane j taking the cells from j c on; every lane of the
+// wave calls it together.
+template <bool ANY, bool COUNT, int S>
+__device__ __forceinline__ void trace_window(const DevFrame* __restrict__ fr,
+                                             const uint32_t* __restrict__ offsets,
+                                             const float4* __restrict__ trir, const RaySoA& rays,
+                                             const HitSoA& hits, uint8_t* __restrict__ occluded,
+                                             uint32_t* __restrict__ counters, uint32_t lanes,
+                                             uint32_t i, bool valid, WaveWin& W)
 {
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t j = lane & (lanes - 1u);
-    const uint32_t g0 = lane - j;
-    const uint64_t gmask = (lanes >= 64u ? ~0ull : ((1ull << lanes) - 1ull)) << g0;
-    LaneRay r = {};
-    r.id = -1;
-    r.best = INFINITY;
-    uint32_t cells = 0;
-    Dda s = {};
-    bool alive = false;
-    const uint32_t nx = (uint32_t)fr->n[0], ny = (uint32_t)fr->n[1];
+    const uint32_t j = lane & (lanes - 1u), owner = lane - j;
+    const uint32_t c = lanes * S <= 16u ? (uint32_t)S : 16u / lanes, cell0 = j * c;
+    float4 ro = make_float4(0.0f, 0.0f, 0.0f, 0.0f), rd = ro;
+    DdaW w = {};
+    bool walk = false;   // the lane stands on a cell of its ray
     if (valid) {
-        r.o0 = rays.ox[i];
-        r.o1 = rays.oy[i];
-        r.o2 = rays.oz[i];
-        r.d0 = rays.dx[i];
-        r.d1 = rays.dy[i];
-        r.d2 = rays.dz[i];
-        r.tmin = rays.tmin[i];
-        r.tmax = rays.tmax[i];
-        alive = grid_ok(fr) &&
-                dda_setup(fr, r.o0, r.o1, r.o2, r.d0, r.d1, r.d2, r.tmin, r.tmax, s) &&
-                dda_skip(s, j, r.tmax);
+        ro = make_float4(rays.ox[i], rays.oy[i], rays.oz[i], rays.tmin[i]);
+        rd = make_float4(rays.dx[i], rays.dy[i], rays.dz[i], rays.tmax[i]);
+        Dda s;
+        walk = grid_ok(fr) && dda_setup(fr, ro.x, ro.y, ro.z, rd.x, rd.y, rd.z, ro.w, rd.w, s);
+        if (walk)
+            w = dda_window(fr, s);
     }
-    float exit_t = 0.0f;
-    if (alive) {
-        load_cell(s, offsets, nx, ny, exit_t, r.bound, r.k, r.e);
-        cells = 1;
-    }
-    bool winner = false;
-    while (__ballot(alive) != 0) {
-        const uint32_t t0 = r.tests;
-        if (const uint64_t hv0 = coop_lanes_simple(alive, r.k, r.e, coop)) {
-            for (uint64_t hv = hv0; hv != 0; hv &= hv - 1)
-                coop_cell((uint32_t)__builtin_ctzll(hv), ANY, trir, r);
-        }
-        if (alive && r.k < r.e)
-            lane_cell<ANY>(trir, r);
-        // The group's earliest cell with a hit ends the ray; cells after it
-        // (higher lanes of this round) are not part of the serial walk.
-        const uint64_t hm = __ballot(alive && r.id >= 0) & gmask;
-        if (hm != 0) {
-            const uint32_t jw = (uint32_t)__builtin_ctzll(hm) - g0;
-            if (alive && j > jw) {
-                --cells;
-                r.tests = t0;
+    bool open = valid;   // the ray's result is not written yet
+    uint32_t cells = 0, tests = 0;
+    if (__ballot(walk) != 0) {
+        W.ro[lane] = make_float4(ro.x, ro.y, ro.z, win_lo(ro.w));
+        W.rd[lane] = make_float4(rd.x, rd.y, rd.z, ro.w);
+        for (uint32_t q = 0; q < cell0; ++q)
+            walk = dda_window_step(w, walk && !(tmin_f(tmin_f(w.tx, w.ty), w.tz) > rd.w));
+        // The next window's steps and list bounds come before this one's
+        // tests, so their latency overlaps the tests.
+        WinU<S> nb, ne, nbound;
+        uint32_t nvisited;
+        const auto next_window = [&]() {
+            nvisited = 0;
+#pragma unroll
+            for (uint32_t s = 0; s < (uint32_t)S; ++s) {
+                const uint32_t* o = offsets + w.ci;   // in the grid also when the walk is over
+                nb[s] = o[0];
+                ne[s] = o[1];
+                const float ex = tmin_f(tmin_f(w.tx, w.ty), w.tz);
+                nbound[s] = __float_as_uint(ANY ? win_end(rd.w, INFINITY)
+                                                : win_end(rd.w, ex * kExitScale));
+                const bool mine = walk && s < c;
+                nvisited += mine ? 1u : 0u;
+                const bool on = dda_window_step(w, mine && !(ex > rd.w));
+                walk = mine ? on : walk;
             }
-            winner = alive && j == jw;
-            alive = false;
-        } else if (alive) {
-            if (dda_skip(s, lanes, r.tmax)) {
-                load_cell(s, offsets, nx, ny, exit_t, r.bound, r.k, r.e);
-                ++cells;
-            } else {
-                alive = false;
+            // the other lanes' cells, up to the lane's next window
+            for (uint32_t q = c; q < lanes * c; ++q)
+                walk = dda_window_step(w, walk && !(tmin_f(tmin_f(w.tx, w.ty), w.tz) > rd.w));
+        };
+        next_window();
+        do {
+            const WinU<S> b = nb, bound = nbound;
+            WinU<S> n = ne;
+            const uint32_t visited = nvisited;
+            next_window();
+#pragma unroll
+            for (uint32_t s = 0; s < (uint32_t)S; ++s)
+                n[s] = s < visited ? n[s] - b[s] : 0u;
+            const unsigned long long key = win_tests<ANY, S>(W, trir, b, n, bound, owner, cell0);
+            const bool hit = key != ~0ull;
+            uint32_t hs = win_cell(key) - cell0;
+            hs = hs < c ? hs : (uint32_t)S;   // S: not one of the lane's cells
+            if (COUNT && open) {
+                const bool after = hit && win_cell(key) < cell0;
+                cells += after ? 0u : (hit && hs < (uint32_t)S) ? hs + 1u : visited;
+#pragma unroll
+                for (uint32_t s = 0; s < (uint32_t)S; ++s)
+                    tests += after              ? 0u
+                             : !hit || s < hs   ? n[s]
+                             : s == hs          ? (ANY ? win_pos(key) + 1u : n[s])
+                                                : 0u;
             }
-        }
+            if (hit) {
+                if (ANY) {
+                    if (j == 0)
+                        occluded[i] = 1;
+                } else if (hs < (uint32_t)S) {
+                    const uint64_t k = win_pick<S>(b, hs) + win_pos(key);
+                    const float4 A = trir[3ull * k], B = trir[3ull * k + 1], C = trir[3ull * k + 2];
+                    const MtPre m = mt_pre(A, B, C, ro.x, ro.y, ro.z, rd.x, rd.y, rd.z);
+                    float t, u, v;
+                    mt_exact(m, t, u, v);
+                    hits.id[i] = (int32_t)__float_as_uint(C.y);
+                    hits.t[i] = t;
+                    hits.u[i] = u;
+                    hits.v[i] = v;
+                }
+                open = false;
+                walk = false;
+                nvisited = 0;
+            }
+        } while (__ballot(nvisited != 0) != 0);
     }
-    const bool group_hit = (__ballot(winner) & gmask) != 0;
-    uint32_t sc = 0, st = 0;
     if (COUNT) {
-        sc = group_sum(cells, lanes);
-        st = group_sum(r.tests, lanes);
+        const uint32_t sc = group_sum(cells, lanes), st = group_sum(tests, lanes);
+        if (valid && j == 0) {
+            counters[2ull * i] = sc;
+            counters[2ull * i + 1] = st;
+        }
     }
-    if (!valid)
-        return;
-    if (ANY) {
-        if (j == 0)
-            occluded[i] = group_hit ? 1 : 0;
-    } else if (winner || (j == 0 && !group_hit)) {
-        hits.id[i] = r.id;
-        hits.t[i] = r.best;
-        hits.u[i] = r.bu;
-        hits.v[i] = r.bv;
-    }
-    if (COUNT && j == 0) {
-        counters[2ull * i] = sc;
-        counters[2ull * i + 1] = st;
+    if (open && j == 0) {
+        if (ANY) {
+            occluded[i] = 0;
+        } else {
+            hits.id[i] = -1;
+            hits.t[i] = INFINITY;
+            hits.u[i] = 0.0f;
+            hits.v[i] = 0.0f;
+        }
     }
 }
 
-template <bool ANY, bool COUNT>
-__global__ __launch_bounds__(256) void k_trace_split(TraceArgs a, RaySoA rays, HitSoA hits,
-                                                     uint8_t* __restrict__ occluded,
-                                                     uint32_t lanes)
+extern __shared__ WaveWin win_lds[];   // one per wave of the block
+
+template <bool ANY, bool COUNT, int S>
+__global__ __launch_bounds__(256) void k_trace_window(TraceArgs a, RaySoA rays, HitSoA hits,
+                                                      uint8_t* __restrict__ occluded,
+                                                      uint32_t lanes)
 {
-    const uint32_t shift = (uint32_t)__builtin_ctz(lanes);
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     bool valid;
-    const uint32_t i = trace_ray(a, t >> shift, valid);
-    trace_split_lane<ANY, COUNT>(a.fr, a.offsets, a.trir, rays, hits, occluded, a.counters,
-                                 a.coop, lanes, i, valid);
+    const uint32_t i = trace_ray(a, t >> __builtin_ctz(lanes), valid);
+    trace_window<ANY, COUNT, S>(a.fr, a.offsets, a.trir, rays, hits, occluded, a.counters, lanes, i,
+                             valid, win_lds[threadIdx.x >> 6]);
 }
 
-// Batched multi-scene traversal with `lanes` lanes per ray (64 / lanes rays
-// per wave): ray slot s is traced by threads [s * lanes, (s + 1) * lanes).  A
-// wave covers 64 / lanes consecutive slots inside one 64-slot group, so one
-// task, and the task's closest/any choice is uniform over the wave.
-__global__ __launch_bounds__(256) void k_trace_batch_split(const BatchTask* __restrict__ tasks,
-                                                           const uint32_t* __restrict__ map,
-                                                           uint32_t total_slots, uint32_t coop,
-                                                           uint32_t lanes)
+// Batched multi-scene traversal: every 64-slot group belongs to one task
+// (map[slot / 64]), so each wave runs its task's walk with wave-uniform scene
+// data.
+template <int S>
+__global__ __launch_bounds__(256) void k_trace_batch_window(const BatchTask* __restrict__ tasks,
+                                                            const uint32_t* __restrict__ map,
+                                                            uint32_t total_slots,
+                                                            uint32_t lanes)
 {
-    const uint32_t shift = (uint32_t)__builtin_ctz(lanes);
-    const uint32_t slot = (blockIdx.x * blockDim.x + threadIdx.x) >> shift;
+    const uint32_t slot = (blockIdx.x * blockDim.x + threadIdx.x) >> __builtin_ctz(lanes);
     const uint32_t group = __builtin_amdgcn_readfirstlane(slot >> 6);
     if ((group << 6) >= total_slots)
         return;   // whole waves only: total_slots is a multiple of 64
@@ -840,197 +326,17 @@ __global__ __launch_bounds__(256) void k_trace_batch_split(const BatchTask* __re
     const BatchTask& T = tasks[task];
     bool valid;
     const uint32_t i = slot_ray(slot - T.slot_begin, T.image_width, T.n, valid);
+    WaveWin& W = win_lds[threadIdx.x >> 6];
     if (T.any)
-        trace_split_lane<true, false>(T.fr, T.offsets, T.trir, T.rays, T.hits, T.occluded, nullptr,
-                                      coop, lanes, i, valid);
+        trace_window<true, false, S>(T.fr, T.offsets, T.trir, T.rays, T.hits, T.occluded, nullptr,
+                                  lanes, i, valid, W);
     else
-        trace_split_lane<false, false>(T.fr, T.offsets, T.trir, T.rays, T.hits, T.occluded,
-                                       nullptr, coop, lanes, i, valid);
+        trace_window<false, false, S>(T.fr, T.offsets, T.trir, T.rays, T.hits, T.occluded, nullptr,
+                                   lanes, i, valid, W);
 }
 
 // ---------------------------------------------------------------------------
-// Persistent waves with lane refill
-// ---------------------------------------------------------------------------
-
-// Each wave keeps its lanes busy by fetching new rays (one atomic per wave
-// for all idle lanes, once at least `refill` lanes are idle or the wave has
-// drained) and advances every lane by one work item per iteration -- one
-// triangle test, or one cell (DDA step + cell range).  Lanes never wait for the
-// longest ray of their wave and inactive ray slots cost one iteration.  Every
-// wave exits once the slot counter passes n_slots and its lanes are done.
-template <bool ANY, bool COUNT>
-__global__ __launch_bounds__(256) void k_trace_persistent(TraceArgs a, RaySoA rays, HitSoA hits,
-                                                          uint8_t* __restrict__ occluded,
-                                                          uint32_t* __restrict__ slot_counter,
-                                                          uint32_t n_slots, uint32_t refill)
-{
-    const DevFrame* __restrict__ fr = a.fr;
-    const uint32_t* __restrict__ offsets = a.offsets;
-    const float4* __restrict__ trir = a.trir;
-    const bool ok = grid_ok(fr);
-    const uint32_t nx = (uint32_t)fr->n[0], ny = (uint32_t)fr->n[1];
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t slot_limit =
-        a.list ? (*a.list_count < n_slots ? *a.list_count : n_slots) : n_slots;
-
-    int32_t ray = -1;         // ray index traced by this lane, -1 = idle
-    bool exhausted = false;   // no slots left for this lane
-    float o0 = 0, o1 = 0, o2 = 0, d0 = 0, d1 = 0, d2 = 0, tmin = 0, tmax = 0;
-    Dda s = {};
-    uint32_t k = 0, e = 0, cells = 0, tests = 0;
-    bool loaded = false;
-    float exit_t = 0.0f, bound = 0.0f;
-    int32_t id = -1;
-    float best = INFINITY, bu = 0.0f, bv = 0.0f;
-    float4 A = {}, B = {}, C = {};   // record k of the current cell, loaded ahead
-
-    for (;;) {
-        // ---- refill idle lanes -------------------------------------------
-        const bool need = (ray < 0) && !exhausted;
-        const uint64_t need_mask = __ballot(need);
-        const uint64_t busy_mask = __ballot(ray >= 0);
-        const uint32_t n_need = (uint32_t)__popcll(need_mask);
-        if (need_mask != 0 && (n_need >= refill || busy_mask == 0)) {
-            const uint32_t leader = (uint32_t)__builtin_ctzll(need_mask);
-            uint32_t base = 0;
-            if (lane == leader)
-                base = atomicAdd(slot_counter, n_need);
-            base = __builtin_amdgcn_readlane(base, leader);
-            if (need) {
-                const uint32_t slot = base + lanes_below(need_mask);
-                if (slot >= slot_limit) {
-                    exhausted = true;
-                } else {
-                    bool valid;
-                    const uint32_t ri = trace_ray(a, slot, valid);
-                    if (valid) {
-                        o0 = rays.ox[ri];
-                        o1 = rays.oy[ri];
-                        o2 = rays.oz[ri];
-                        d0 = rays.dx[ri];
-                        d1 = rays.dy[ri];
-                        d2 = rays.dz[ri];
-                        tmin = rays.tmin[ri];
-                        tmax = rays.tmax[ri];
-                        id = -1;
-                        best = INFINITY;
-                        bu = 0.0f;
-                        bv = 0.0f;
-                        cells = 0;
-                        tests = 0;
-                        loaded = false;
-                        k = e = 0;
-                        ray = (int32_t)ri;
-                        if (!(ok && dda_setup(fr, o0, o1, o2, d0, d1, d2, tmin, tmax, s))) {
-                            if (ANY) {
-                                occluded[ri] = 0;
-                            } else {
-                                hits.id[ri] = -1;
-                                hits.t[ri] = INFINITY;
-                                hits.u[ri] = 0.0f;
-                                hits.v[ri] = 0.0f;
-                            }
-                            if (COUNT) {
-                                a.counters[2ull * ri] = 0;
-                                a.counters[2ull * ri + 1] = 0;
-                            }
-                            ray = -1;
-                        }
-                    }
-                }
-            }
-        }
-        if (__ballot(ray >= 0) == 0) {
-            if (__ballot(!exhausted) == 0)
-                break;
-            continue;
-        }
-        // ---- drained queue: finish dense cells with the whole wave -----------
-        if (const uint64_t hv0 = coop_lanes(ray >= 0, exhausted, k, e, a.coop)) {
-            LaneRay r = {o0, o1, o2, d0, d1, d2, tmin, tmax, bound, k, e, id, best, bu, bv, tests};
-            for (uint64_t hv = hv0; hv != 0; hv &= hv - 1)
-                coop_cell((uint32_t)__builtin_ctzll(hv), ANY, trir, r);
-            k = r.k;
-            id = r.id;
-            best = r.best;
-            bu = r.bu;
-            bv = r.bv;
-            tests = r.tests;
-        }
-        if (ray < 0)
-            continue;
-
-        // ---- one work item ---------------------------------------------------
-        bool finish = false;
-        if (k < e) {
-            const float4 cA = A, cB = B, cC = C;
-            ++k;
-            if (k < e) {
-                A = trir[3ull * k];
-                B = trir[3ull * k + 1];
-                C = trir[3ull * k + 2];
-            }
-            if (COUNT)
-                ++tests;
-            if (ANY) {
-                if (any_test(cA, cB, cC, o0, o1, o2, d0, d1, d2, tmin, tmax)) {
-                    id = 1;
-                    finish = true;
-                }
-            } else {
-                closest_test(cA, cB, cC, o0, o1, o2, d0, d1, d2, tmin, tmax, bound, id, best, bu,
-                             bv);
-            }
-        } else {
-            if (loaded) {
-                if (id >= 0)   // closest: hit in this cell; any: occluded
-                    finish = true;
-                else if (exit_t > tmax || !dda_step(s))
-                    finish = true;
-            }
-            if (!finish) {
-                if (COUNT)
-                    ++cells;
-                exit_t = tmin_f(tmin_f(s.tx, s.ty), s.tz);
-                const uint32_t ci = (uint32_t)s.cx + nx * ((uint32_t)s.cy + ny * (uint32_t)s.cz);
-                k = offsets[ci];
-                e = offsets[ci + 1];
-                bound = exit_t * kExitScale;
-                loaded = true;
-                if (k < e) {
-                    A = trir[3ull * k];
-                    B = trir[3ull * k + 1];
-                    C = trir[3ull * k + 2];
-                }
-            }
-        }
-        if (finish) {
-            const uint32_t ri = (uint32_t)ray;
-            if (ANY) {
-                occluded[ri] = id >= 0 ? 1 : 0;
-            } else {
-                hits.id[ri] = id;
-                hits.t[ri] = best;
-                hits.u[ri] = bu;
-                hits.v[ri] = bv;
-            }
-            if (COUNT) {
-                a.counters[2ull * ri] = cells;
-                a.counters[2ull * ri + 1] = tests;
-            }
-            ray = -1;
-        }
-    }
-}
-
-__global__ void k_fill_u32_one(uint32_t* __restrict__ p)
-{
-    if (threadIdx.x == 0)
-        p[0] = 0u;
-}
-
-// ---------------------------------------------------------------------------
-// Batched multi-scene traversal (device work queue)
+// Batched multi-scene traversal
 // ---------------------------------------------------------------------------
 
 // map[b] = index of the task owning slots [64b, 64b+64).
@@ -1041,165 +347,6 @@ __global__ __launch_bounds__(256) void k_task_map(const BatchTask* __restrict__ 
     const uint32_t b0 = t.slot_begin >> 6, nb = t.slots >> 6;
     for (uint32_t j = threadIdx.x; j < nb; j += blockDim.x)
         map[b0 + j] = blockIdx.x;
-}
-
-// Same per-lane algorithm as k_trace_persistent, but every lane carries its
-// own task (scene grid, ray and output buffers, closest or any hit): a refill
-// hands out global slots; slot s belongs to task map[s / 64].
-__global__ __launch_bounds__(256) void k_trace_batch(const BatchTask* __restrict__ tasks,
-                                                     const uint32_t* __restrict__ map,
-                                                     uint32_t total_slots,
-                                                     uint32_t* __restrict__ slot_counter,
-                                                     uint32_t refill, uint32_t coop)
-{
-    const uint32_t lane = threadIdx.x & 63u;
-    int32_t ray = -1;
-    bool exhausted = false;
-    uint32_t task = 0;
-    bool any = false;
-    const uint32_t* offsets = nullptr;
-    const float4* trir = nullptr;
-    uint32_t nx = 0, ny = 0;
-    float o0 = 0, o1 = 0, o2 = 0, d0 = 0, d1 = 0, d2 = 0, tmin = 0, tmax = 0;
-    Dda s = {};
-    uint32_t k = 0, e = 0;
-    bool loaded = false;
-    float exit_t = 0.0f, bound = 0.0f;
-    int32_t id = -1;
-    float best = INFINITY, bu = 0.0f, bv = 0.0f;
-    float4 A = {}, B = {}, C = {};
-
-    for (;;) {
-        const bool need = (ray < 0) && !exhausted;
-        const uint64_t need_mask = __ballot(need);
-        const uint64_t busy_mask = __ballot(ray >= 0);
-        const uint32_t n_need = (uint32_t)__popcll(need_mask);
-        if (need_mask != 0 && (n_need >= refill || busy_mask == 0)) {
-            const uint32_t leader = (uint32_t)__builtin_ctzll(need_mask);
-            uint32_t base = 0;
-            if (lane == leader)
-                base = atomicAdd(slot_counter, n_need);
-            base = __builtin_amdgcn_readlane(base, leader);
-            if (need) {
-                const uint32_t slot = base + lanes_below(need_mask);
-                if (slot >= total_slots) {
-                    exhausted = true;
-                } else {
-                    task = map[slot >> 6];
-                    const BatchTask& T = tasks[task];
-                    bool valid;
-                    const uint32_t ri = slot_ray(slot - T.slot_begin, T.image_width, T.n, valid);
-                    if (valid) {
-                        const DevFrame* __restrict__ fr = T.fr;
-                        any = T.any != 0;
-                        offsets = T.offsets;
-                        trir = T.trir;
-                        nx = (uint32_t)fr->n[0];
-                        ny = (uint32_t)fr->n[1];
-                        o0 = T.rays.ox[ri];
-                        o1 = T.rays.oy[ri];
-                        o2 = T.rays.oz[ri];
-                        d0 = T.rays.dx[ri];
-                        d1 = T.rays.dy[ri];
-                        d2 = T.rays.dz[ri];
-                        tmin = T.rays.tmin[ri];
-                        tmax = T.rays.tmax[ri];
-                        id = -1;
-                        best = INFINITY;
-                        bu = 0.0f;
-                        bv = 0.0f;
-                        loaded = false;
-                        k = e = 0;
-                        ray = (int32_t)ri;
-                        if (!(grid_ok(fr) && dda_setup(fr, o0, o1, o2, d0, d1, d2, tmin, tmax, s))) {
-                            if (any) {
-                                T.occluded[ri] = 0;
-                            } else {
-                                T.hits.id[ri] = -1;
-                                T.hits.t[ri] = INFINITY;
-                                T.hits.u[ri] = 0.0f;
-                                T.hits.v[ri] = 0.0f;
-                            }
-                            ray = -1;
-                        }
-                    }
-                }
-            }
-        }
-        if (__ballot(ray >= 0) == 0) {
-            if (__ballot(!exhausted) == 0)
-                break;
-            continue;
-        }
-        if (const uint64_t hv0 = coop_lanes(ray >= 0, exhausted, k, e, coop)) {
-            uint32_t tests = 0;
-            LaneRay r = {o0, o1, o2, d0, d1, d2, tmin, tmax, bound, k, e, id, best, bu, bv, tests};
-            for (uint64_t hv = hv0; hv != 0; hv &= hv - 1) {
-                const uint32_t l = (uint32_t)__builtin_ctzll(hv);
-                coop_cell(l, bcast_u(any ? 1u : 0u, l) != 0, trir, r);
-            }
-            k = r.k;
-            id = r.id;
-            best = r.best;
-            bu = r.bu;
-            bv = r.bv;
-        }
-        if (ray < 0)
-            continue;
-
-        bool finish = false;
-        if (k < e) {
-            const float4 cA = A, cB = B, cC = C;
-            ++k;
-            if (k < e) {
-                A = trir[3ull * k];
-                B = trir[3ull * k + 1];
-                C = trir[3ull * k + 2];
-            }
-            if (any) {
-                if (any_test(cA, cB, cC, o0, o1, o2, d0, d1, d2, tmin, tmax)) {
-                    id = 1;
-                    finish = true;
-                }
-            } else {
-                closest_test(cA, cB, cC, o0, o1, o2, d0, d1, d2, tmin, tmax, bound, id, best, bu,
-                             bv);
-            }
-        } else {
-            if (loaded) {
-                if (id >= 0)   // closest: hit in this cell; any: occluded
-                    finish = true;
-                else if (exit_t > tmax || !dda_step(s))
-                    finish = true;
-            }
-            if (!finish) {
-                exit_t = tmin_f(tmin_f(s.tx, s.ty), s.tz);
-                const uint32_t ci = (uint32_t)s.cx + nx * ((uint32_t)s.cy + ny * (uint32_t)s.cz);
-                k = offsets[ci];
-                e = offsets[ci + 1];
-                bound = exit_t * kExitScale;
-                loaded = true;
-                if (k < e) {
-                    A = trir[3ull * k];
-                    B = trir[3ull * k + 1];
-                    C = trir[3ull * k + 2];
-                }
-            }
-        }
-        if (finish) {
-            const BatchTask& T = tasks[task];
-            const uint32_t ri = (uint32_t)ray;
-            if (any) {
-                T.occluded[ri] = id >= 0 ? 1 : 0;
-            } else {
-                T.hits.id[ri] = id;
-                T.hits.t[ri] = best;
-                T.hits.u[ri] = bu;
-                T.hits.v[ri] = bv;
-            }
-            ray = -1;
-        }
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1691,128 +838,61 @@ hipError_t launch_trace2(const TraceArgs& a, const RaySoA& rays, const HitSoA& h
     return hipGetLastError();
 }
 
-hipError_t launch_trace_closest(const TraceArgs& a, const RaySoA& rays, const HitSoA& hits,
-                                uint32_t block, hipStream_t s)
+// Lanes per ray of a windowed launch of `slots` ray slots.  More lanes per ray
+// mean more waves with less work each -- a small launch is bound by its
+// longest wave -- but every lane of a group steps the whole walk, and past a
+// few times 5,120 resident waves the kernel is bound by those instructions.
+// Measured (us, 1 / 2 / 4 / 8 lanes): 64x64 spheres frame 129 / 115 / 111 /
+// 108, 512x512 spheres bounce 70 / 56 / 43 / 44 and primary 70 / 58 / 51 / 71,
+// 904x678 spheres primary 120 / 97 / 113 / 165, 1.2 M-slot batch 592 / 568 /
+// 612 / 813, 1.6 M ambient-occlusion rays with their frame 1229 / 1188 / 1276
+// / 1660, serving rounds of several million slots 9383 / 10080 / 11847 / -.
+static uint32_t window_lanes(uint64_t slots)
 {
-    if (a.n == 0)
-        return hipSuccess;
-    const uint32_t g = ray_grid(a.n, a.image_width, block);
-    if (a.counters && a.pool)
-        hipLaunchKernelGGL((k_trace_closest<true, true>), dim3(g), dim3(block), 0, s, a, rays, hits);
-    else if (a.counters)
-        hipLaunchKernelGGL((k_trace_closest<true, false>), dim3(g), dim3(block), 0, s, a, rays,
-                           hits);
-    else if (a.pool)
-        hipLaunchKernelGGL((k_trace_closest<false, true>), dim3(g), dim3(block), 0, s, a, rays,
-                           hits);
+    if (slots >= (4u << 20))
+        return 1;
+    if (slots >= 400000)
+        return 2;
+    return slots >= 100000 ? 4 : 8;
+}
+
+template <bool ANY, bool COUNT>
+static void window_launch(const TraceArgs& a, const RaySoA& rays, const HitSoA& hits,
+                          uint8_t* occluded, uint32_t lanes, uint32_t grid, uint32_t block,
+                          hipStream_t s)
+{
+    const size_t lds = block / 64 * sizeof(WaveWin);
+    if (lanes == 1)
+        hipLaunchKernelGGL((k_trace_window<ANY, COUNT, 4>), dim3(grid), dim3(block), lds, s, a,
+                           rays, hits, occluded, lanes);
     else
-        hipLaunchKernelGGL((k_trace_closest<false, false>), dim3(g), dim3(block), 0, s, a, rays,
-                           hits);
-    return hipGetLastError();
+        hipLaunchKernelGGL((k_trace_window<ANY, COUNT, 2>), dim3(grid), dim3(block), lds, s, a,
+                           rays, hits, occluded, lanes);
 }
 
-hipError_t launch_trace_any(const TraceArgs& a, const RaySoA& rays, uint8_t* occluded,
-                            uint32_t block, hipStream_t s)
+hipError_t launch_trace_window(const TraceArgs& a, const RaySoA& rays, const HitSoA& hits,
+                               uint8_t* occluded, bool any, uint32_t lanes, uint32_t block,
+                               hipStream_t s)
 {
     if (a.n == 0)
         return hipSuccess;
-    const uint32_t g = ray_grid(a.n, a.image_width, block);
-    if (a.counters && a.pool)
-        hipLaunchKernelGGL((k_trace_any<true, true>), dim3(g), dim3(block), 0, s, a, rays, occluded);
+    if (lanes > 16 || (lanes & (lanes - 1)) != 0)
+        return hipErrorInvalidValue;
+    const uint64_t slots = slot_count(a.n, a.image_width);
+    if (lanes == 0)
+        lanes = window_lanes(slots);
+    const uint64_t threads = slots * lanes;
+    if (lanes > 1 && threads > 0xffffffffull - block)
+        return hipErrorInvalidValue;
+    const uint32_t g = (uint32_t)((threads + block - 1) / block);
+    if (any && a.counters)
+        window_launch<true, true>(a, rays, hits, occluded, lanes, g, block, s);
+    else if (any)
+        window_launch<true, false>(a, rays, hits, occluded, lanes, g, block, s);
     else if (a.counters)
-        hipLaunchKernelGGL((k_trace_any<true, false>), dim3(g), dim3(block), 0, s, a, rays,
-                           occluded);
-    else if (a.pool)
-        hipLaunchKernelGGL((k_trace_any<false, true>), dim3(g), dim3(block), 0, s, a, rays,
-                           occluded);
+        window_launch<false, true>(a, rays, hits, occluded, lanes, g, block, s);
     else
-        hipLaunchKernelGGL((k_trace_any<false, false>), dim3(g), dim3(block), 0, s, a, rays,
-                           occluded);
-    return hipGetLastError();
-}
-
-hipError_t launch_trace_split(const TraceArgs& a, const RaySoA& rays, const HitSoA& hits,
-                              uint8_t* occluded, bool any, uint32_t lanes, uint32_t block,
-                              hipStream_t s)
-{
-    if (a.n == 0)
-        return hipSuccess;
-    if (lanes < 2 || lanes > 16 || (lanes & (lanes - 1)) != 0)
-        return hipErrorInvalidValue;
-    const uint64_t threads = slot_count(a.n, a.image_width) * lanes;
-    if (threads > 0xffffffffull - block)
-        return hipErrorInvalidValue;
-    const dim3 g((uint32_t)((threads + block - 1) / block));
-    if (any) {
-        if (a.counters)
-            hipLaunchKernelGGL((k_trace_split<true, true>), g, dim3(block), 0, s, a, rays, hits,
-                               occluded, lanes);
-        else
-            hipLaunchKernelGGL((k_trace_split<true, false>), g, dim3(block), 0, s, a, rays, hits,
-                               occluded, lanes);
-    } else {
-        if (a.counters)
-            hipLaunchKernelGGL((k_trace_split<false, true>), g, dim3(block), 0, s, a, rays, hits,
-                               occluded, lanes);
-        else
-            hipLaunchKernelGGL((k_trace_split<false, false>), g, dim3(block), 0, s, a, rays, hits,
-                               occluded, lanes);
-    }
-    return hipGetLastError();
-}
-
-// Resident blocks on the device for a persistent kernel at a block size.
-template <class K>
-static uint32_t resident_blocks(K kernel, uint32_t block)
-{
-    static int cus = 0;
-    if (cus == 0) {
-        int dev = 0;
-        (void)hipGetDevice(&dev);
-        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            cus <= 0)
-            cus = 256;
-    }
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, (int)block, 0) !=
-            hipSuccess ||
-        per_cu <= 0)
-        per_cu = 1;
-    return (uint32_t)cus * (uint32_t)per_cu;
-}
-
-hipError_t launch_trace_persistent(const TraceArgs& a, const RaySoA& rays, const HitSoA& hits,
-                                   uint8_t* occluded, bool any, uint32_t* slot_counter,
-                                   uint32_t block, uint32_t refill, hipStream_t s)
-{
-    if (a.n == 0)
-        return hipSuccess;
-    const uint64_t n_slots = slot_count(a.n, a.image_width);
-    if (n_slots > 0xffffffffull)
-        return hipErrorInvalidValue;
-    refill = refill < 1 ? 1 : (refill > 64 ? 64 : refill);
-    hipLaunchKernelGGL(k_fill_u32_one, dim3(1), dim3(64), 0, s, slot_counter);
-    const uint32_t need = (uint32_t)((n_slots + block - 1) / block);
-#define GRT_LAUNCH_P(ANYV, CNTV)                                                                \
-    do {                                                                                        \
-        auto kern = k_trace_persistent<ANYV, CNTV>;                                             \
-        uint32_t g = resident_blocks(kern, block);                                              \
-        g = g < need ? g : need;                                                                \
-        hipLaunchKernelGGL(kern, dim3(g), dim3(block), 0, s, a, rays, hits, occluded,           \
-                           slot_counter, (uint32_t)n_slots, refill);                            \
-    } while (0)
-    if (any) {
-        if (a.counters)
-            GRT_LAUNCH_P(true, true);
-        else
-            GRT_LAUNCH_P(true, false);
-    } else {
-        if (a.counters)
-            GRT_LAUNCH_P(false, true);
-        else
-            GRT_LAUNCH_P(false, false);
-    }
-#undef GRT_LAUNCH_P
+        window_launch<false, false>(a, rays, hits, occluded, lanes, g, block, s);
     return hipGetLastError();
 }
 
@@ -1825,38 +905,25 @@ hipError_t launch_task_map(const BatchTask* tasks, uint32_t n_tasks, uint32_t* m
 }
 
 hipError_t launch_trace_batch(const BatchTask* tasks, const uint32_t* map, uint32_t total_slots,
-                              uint32_t* slot_counter, int mode, uint32_t block,
-                              uint32_t refill, uint32_t lanes, uint32_t coop, hipStream_t s)
+                              uint32_t lanes, uint32_t block, hipStream_t s)
 {
     if (total_slots == 0)
         return hipSuccess;
-    if (mode == GRT_TRACE_SPLIT) {
-        if (lanes < 2 || lanes > 16 || (lanes & (lanes - 1)) != 0)
-            return hipErrorInvalidValue;
-        const uint64_t threads = (uint64_t)total_slots * lanes;
-        if (threads > 0xffffffffull - block)
-            return hipErrorInvalidValue;
-        hipLaunchKernelGGL(k_trace_batch_split, dim3((uint32_t)((threads + block - 1) / block)),
-                           dim3(block), 0, s, tasks, map, total_slots, coop, lanes);
-        return hipGetLastError();
-    }
-    if (mode != GRT_TRACE_PERSISTENT) {
-        const dim3 g((total_slots + block - 1) / block);
-        if (mode == GRT_TRACE_POOLED)
-            hipLaunchKernelGGL(k_trace_batch_simple<true>, g, dim3(block), 0, s, tasks, map,
-                               total_slots, coop);
-        else
-            hipLaunchKernelGGL(k_trace_batch_simple<false>, g, dim3(block), 0, s, tasks, map,
-                               total_slots, coop);
-        return hipGetLastError();
-    }
-    refill = refill < 1 ? 1 : (refill > 64 ? 64 : refill);
-    hipLaunchKernelGGL(k_fill_u32_one, dim3(1), dim3(64), 0, s, slot_counter);
-    uint32_t g = resident_blocks(k_trace_batch, block);
-    const uint32_t need = (total_slots + block - 1) / block;
-    g = g < need ? g : need;
-    hipLaunchKernelGGL(k_trace_batch, dim3(g), dim3(block), 0, s, tasks, map, total_slots,
-                       slot_counter, refill, coop);
+    if (lanes == 0)
+        lanes = window_lanes(total_slots);
+    if (lanes > 16 || (lanes & (lanes - 1)) != 0)
+        return hipErrorInvalidValue;
+    const uint64_t threads = (uint64_t)total_slots * lanes;
+    if (lanes > 1 && threads > 0xffffffffull - block)
+        return hipErrorInvalidValue;
+    const dim3 g((uint32_t)((threads + block - 1) / block));
+    const size_t lds = block / 64 * sizeof(WaveWin);
+    if (lanes == 1)
+        hipLaunchKernelGGL(k_trace_batch_window<4>, g, dim3(block), lds, s, tasks, map,
+                           total_slots, lanes);
+    else
+        hipLaunchKernelGGL(k_trace_batch_window<2>, g, dim3(block), lds, s, tasks, map,
+                           total_slots, lanes);
     return hipGetLastError();
 }
 

@@ -431,18 +431,16 @@ class Context:
     TRACE_MODES = {"simple": 0, "persistent": 1, "pooled": 2, "split": 3}
 
     def set_trace_mode(self, mode="simple", param: int = 16):
-        """Traversal schedule: "simple" (one ray per lane), "pooled" (one ray
-        per lane, the wave's triangle tests pooled), "persistent" (refilled
-        persistent waves, one test or cell per iteration; param = refill
-        threshold 1..64), "split" (param = 2, 4, 8 or 16 lanes per ray, each
-        lane visiting every param-th cell of the ray); a bool selects
-        persistent (True) or simple."""
+        """Traversal schedule: "simple", "pooled" and "persistent" (a bool
+        selects persistent or simple) let the library choose the lanes per ray
+        by the size of the launch (param, 1..64, is only checked); "split"
+        takes param = 2, 4, 8 or 16 lanes per ray."""
         if isinstance(mode, bool):
             mode = "persistent" if mode else "simple"
         check(lib().grt_set_trace_mode(self.h, self.TRACE_MODES[mode], param))
 
     def set_coop(self, min_refs: int = 16):
-        """Cooperative cell tests in drained persistent waves (0: off)."""
+        """Accepted and without effect (grt_set_coop)."""
         check(lib().grt_set_coop(self.h, min_refs))
 
     def trace_instances(self, instances, rays: RayBatch, hits: HitBatch, instance_out,
@@ -813,7 +811,7 @@ class BatchItem(ctypes.Structure):
 
 
 class Batch:
-    """Many (scene, ray batch) items traced in one persistent launch."""
+    """Many (scene, ray batch) items traced in one launch."""
 
     def __init__(self, ctx: Context, max_items: int):
         self.ctx = ctx

@@ -83,29 +83,26 @@ int grt_memory_used(grt_context ctx, uint64_t* bytes);
  * cudaSetBlockSize (RayTracing.h:39) was a no-op in the reference. */
 int grt_set_block_size(grt_context ctx, uint32_t closest, uint32_t any);
 
-/* Traversal scheduling.  GRT_TRACE_SIMPLE (default): one ray per lane for the
- * whole launch, each lane testing its own cell's triangles.  GRT_TRACE_POOLED:
- * one ray per lane, the triangle tests of all the wave's current cells pooled
- * and spread over the wave's lanes.  GRT_TRACE_PERSISTENT: persistent waves
- * whose idle lanes fetch new rays once `param` (1..64) lanes of a wave are
- * idle, advancing each lane by one triangle test or cell per iteration.
- * GRT_TRACE_SPLIT: `param` (2, 4, 8 or 16) lanes per ray, lane j visiting
- * the ray's cells j, j + param, ... of the serial order; for launches with
- * too few rays to fill the GPU.  For SIMPLE and POOLED `param` is kept as the
- * refill threshold (1..64) of later persistent launches.  The per-lane
- * schedules finish dense cells wave-cooperatively (grt_set_coop).  Results and
- * counters are identical; only the schedule differs.  The serving loop and
- * batches (grt_batch_trace) follow the setting; a batch under GRT_TRACE_SPLIT
- * gives every ray of every item `param` lanes (64 / param rays per wave). */
+/* Traversal scheduling.  On a one-level grid every schedule walks its rays in
+ * windows of cells and spreads the triangle tests of a window over the lanes
+ * of the wave.  GRT_TRACE_SIMPLE (default), GRT_TRACE_POOLED and
+ * GRT_TRACE_PERSISTENT choose the lanes per ray (1 to 8) by the size of the
+ * launch; their `param` (1..64) is checked and otherwise unused.
+ * GRT_TRACE_SPLIT: `param` (2, 4, 8 or 16) lanes per ray, each visiting some
+ * of the ray's cells; on a two-level grid lane j visits the ray's top cells
+ * j, j + param, ... of the serial order (one lane per ray under the other
+ * schedules).  Results and counters are identical; only the schedule differs.
+ * The serving loop and batches (grt_batch_trace) follow the setting; a batch
+ * under GRT_TRACE_SPLIT gives every ray of every item `param` lanes (64 /
+ * param rays per wave). */
 #define GRT_TRACE_SIMPLE     0
 #define GRT_TRACE_PERSISTENT 1
 #define GRT_TRACE_POOLED     2
 #define GRT_TRACE_SPLIT      3
 int grt_set_trace_mode(grt_context ctx, int mode, uint32_t param);
-/* Persistent and batched traversal: once a wave finds the ray queue drained,
- * the wave tests the rest of a lane's cell 64 references at a time when at
- * least max(min_refs, 2 x its busy lanes) are left (0 = never; default 16).
- * Results and counters are those of the one-lane loop. */
+/* Kept for callers of the per-lane schedules, which tested dense cells
+ * cooperatively from min_refs references on: every schedule now spreads its
+ * tests over the wave, and the setting has no effect. */
 int grt_set_coop(grt_context ctx, uint32_t min_refs);
 
 /* ---- scene ------------------------------------------------------------ */
@@ -442,8 +439,7 @@ int grt_shade_phong(grt_scene scene, const grt_rays* rays, const grt_hits* hits,
 /* The reference traced one scene per launch (cudaRayTrace,
  * RayTracing.cu:227-253).  A batch holds items -- each a ray batch of one
  * scene, closest hit (any = 0, outputs in hits) or any hit (any = 1, output in
- * occluded) -- and traces all of them in one persistent launch whose waves
- * fetch ray slots from a device work queue.  Item pointers are captured at
+ * occluded) -- and traces all of them in one launch, each wave in one item.  Item pointers are captured at
  * grt_batch_set: call it again after a grt_grid_build or grt_grid_upload of any
  * item's scene (grt_grid_rebuild_async keeps the pointers valid). */
 typedef struct grt_batch_t* grt_batch;

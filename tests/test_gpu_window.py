@@ -1,0 +1,77 @@
+"""GPU tests of the windowed one-level traversal at the sizes where its pooled
+tests, its long lists and its choice of lanes per ray change path.  Bar:
+bit-exact to the oracle, counters included, under every schedule."""
+import numpy as np
+import pytest
+
+import grt
+import pyoracle as orc
+from conftest import rng
+from test_gpu_parity import assert_same, check_any, check_closest, check_grid, _random_rays
+
+pytestmark = pytest.mark.gpu
+
+
+def _soup(n, seed, size=0.2):
+    """n random triangles in the unit box."""
+    r = rng(seed)
+    c = r.random((n, 1, 3)).astype(np.float32)
+    return (c + (r.random((n, 3, 3)).astype(np.float32) - np.float32(0.5)) * np.float32(size)
+            ).reshape(n, 9)
+
+
+# One cell that lists every triangle: rounds of 64 and 128 pooled tests with
+# their remainders, and both sides of the length from which a list is tested
+# on its own (192).
+@pytest.mark.parametrize("refs", [1, 2, 63, 64, 65, 127, 128, 129, 191, 192, 193, 1000])
+def test_one_cell_lists(gpu_ctx, refs):
+    v = _soup(refs, refs)
+    sc, fr, offs, orefs = check_grid(gpu_ctx, v, np.zeros_like(v), 1e-5)
+    assert len(offs) == 2 and len(orefs) == refs
+    for n in (1, 63, 64, 65, 513):
+        rays = _random_rays(n, 100 + n)
+        check_closest(sc, fr, offs, orefs, v, rays)
+        check_any(sc, fr, offs, orefs, v, rays)
+
+
+# Short and long lists in the same windows, whole and ragged images.
+@pytest.mark.parametrize("lam,width", [(0.05, 0), (0.5, 0), (5.0, 37), (60.0, 128)])
+def test_mixed_lists(gpu_ctx, lam, width):
+    v = np.concatenate([_soup(3000, 7, 0.05), _soup(600, 8, 0.02) * np.float32(0.1) +
+                        np.float32(0.4)])
+    sc, fr, offs, refs = check_grid(gpu_ctx, v, np.zeros_like(v), lam)
+    cam = grt.camera_lookat((0.5, 0.5, -1.5), (0.5, 0.5, 0.0), (0, 1, 0), 60.0, max(width, 61),
+                            67)
+    rays = orc.primary_rays(grt.camera_dict(cam)) if width else _random_rays(4099, 9)
+    check_closest(sc, fr, offs, refs, v, rays, width)
+    check_any(sc, fr, offs, refs, v, rays)
+
+
+# Both sides of every size at which the lanes per ray change.
+@pytest.mark.parametrize("n", [99_999, 100_000, 399_999, 400_000, (4 << 20) - 1, 4 << 20])
+def test_lanes_by_launch_size(gpu_ctx, n):
+    import torch
+    v = _soup(64, 3, 0.4)
+    sc, fr, offs, refs = check_grid(gpu_ctx, v, np.zeros_like(v), 4.0)
+    rays = _random_rays(n, 5)
+    o = orc.trace_closest(fr, offs, refs, v, rays, counters=True)
+    oa = orc.trace_any(fr, offs, refs, v, rays, counters=True)
+    rb, hb = grt.RayBatch.from_numpy(rays), grt.HitBatch.empty(n)
+    occ = torch.full((n,), 9, dtype=torch.uint8, device="cuda:0")
+    cnt = torch.full((2 * n,), -7, dtype=torch.int32, device="cuda:0")
+    gpu_ctx.set_trace_mode("simple", 16)
+    for counters in (cnt, None):
+        sc.trace_closest(rb, hb, counters=counters)
+        g = hb.numpy()
+        for k in ("id", "t", "u", "v"):
+            assert_same(g[k], o[k], f"hit.{k}")
+        if counters is not None:
+            c = cnt.cpu().numpy().view(np.uint32).reshape(n, 2)
+            assert_same(c[:, 0], o["cells"], "cells visited")
+            assert_same(c[:, 1], o["tests"], "triangle tests")
+        sc.trace_any(rb, occ, counters=counters)
+        assert_same(occ.cpu().numpy(), oa["occluded"], "occluded")
+        if counters is not None:
+            c = cnt.cpu().numpy().view(np.uint32).reshape(n, 2)
+            assert_same(c[:, 0], oa["cells"], "cells visited")
+            assert_same(c[:, 1], oa["tests"], "triangle tests")
