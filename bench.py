@@ -111,12 +111,10 @@ def grid_tag(lam, sub):
 
 
 def kernel_name(closest, sched_char, two_level=False):
-    """The traversal kernel a stage launches under a schedule character (a
-    two-level grid is walked by its own kernel under every schedule)."""
-    if two_level:
-        kern = "k_trace2_split" if sched_char in "248x" else "k_trace2"
-        return "%s<%s>" % (kern, "false" if closest else "true")
-    return "k_trace_window<%s, false>" % ("false" if closest else "true")
+    """The traversal kernel a stage launches (under every schedule; a two-level
+    grid is walked by its own kernel)."""
+    return "%s<%s, false>" % ("k_trace2_window" if two_level else "k_trace_window",
+                              "false" if closest else "true")
 
 
 class Frame:
@@ -357,9 +355,9 @@ def autotune(frame, grids, sched, lists):
     (lambda, sub) pairs, sub = None for one level or (lambda2, min_refs).  For
     a one-level grid, every stage is timed under each schedule, with and
     without ray lists (each stage's time includes its ray generation and list
-    compaction), and the fastest per stage is kept.  A two-level grid has two
-    traversal kernels, one ray per lane ('s') and 2..16 lanes per ray ('2',
-    '4', '8', 'x'), chosen per stage the same way."""
+    compaction), and the fastest per stage is kept; a two-level grid likewise,
+    with the lanes per ray chosen by the launch ('s') or given ('2', '4', '8',
+    'x')."""
     from grt.autotune import Autotuner
     tuner = Autotuner()
     table = {}
@@ -376,8 +374,7 @@ def autotune(frame, grids, sched, lists):
                           "frame_ms": round(sum(ms), 3), "lam": c["lam"], "sub": c["sub"]}
             return sum(ms)
         by = {}
-        # on a two-level grid 's', 'w' and 'p' launch the same one-ray-per-lane
-        # kernel; '2'..'x' its lanes-per-ray variant
+        # 's', 'w' and 'p' are the same launch on a two-level grid
         for ch in (Frame.SCHEDULES if sub is None else "s248x"):
             for kind in (("-",) if lists else ("-", "c")):
                 frame.sched = ch * 4

@@ -1217,12 +1217,6 @@ static TraceArgs trace_args(grt_scene sc, uint32_t n, uint32_t image_width, uint
     return a;
 }
 
-// Lanes per ray of a two-level trace: the split schedule's, else one.
-static uint32_t trace2_lanes(const grt_context_t* ctx)
-{
-    return ctx->trace_mode == GRT_TRACE_SPLIT ? ctx->split_lanes : 1u;
-}
-
 // One closest-hit launch of the context's schedule.
 static int dispatch_closest(grt_scene sc, const TraceArgs& a, const grt_rays* rays,
                             const grt_hits* hits)
@@ -1230,7 +1224,7 @@ static int dispatch_closest(grt_scene sc, const TraceArgs& a, const grt_rays* ra
     const HitSoA h{hits->id, hits->t, hits->u, hits->v};
     grt_context_t* ctx = sc->ctx;
     if (a.cellrec)
-        return hip_check(launch_trace2(a, to_soa(rays), h, nullptr, trace2_lanes(ctx),
+        return hip_check(launch_trace2(a, to_soa(rays), h, nullptr, window_lanes_of(ctx),
                                        ctx->stream),
                          "trace_closest");
     return hip_check(launch_trace_window(a, to_soa(rays), h, nullptr, false, window_lanes_of(ctx),
@@ -1244,7 +1238,7 @@ static int dispatch_any(grt_scene sc, const TraceArgs& a, const grt_rays* rays,
 {
     grt_context_t* ctx = sc->ctx;
     if (a.cellrec)
-        return hip_check(launch_trace2(a, to_soa(rays), HitSoA{}, occluded_dev, trace2_lanes(ctx),
+        return hip_check(launch_trace2(a, to_soa(rays), HitSoA{}, occluded_dev, window_lanes_of(ctx),
                                        ctx->stream),
                          "trace_any");
     return hip_check(launch_trace_window(a, to_soa(rays), HitSoA{}, occluded_dev, true,

@@ -69,8 +69,8 @@ struct grt_context_t {
     hipEvent_t aux_ev[4] = {nullptr, nullptr, nullptr, nullptr};
 };
 
-// Lanes per ray of a one-level launch: the split schedule's, else 0 (by the
-// size of the launch).
+// Lanes per ray of a launch: the split schedule's, else 0 (by the size of the
+// launch).
 inline uint32_t window_lanes_of(const grt_context_t* ctx)
 {
     return ctx->trace_mode == GRT_TRACE_SPLIT ? ctx->split_lanes : 0u;

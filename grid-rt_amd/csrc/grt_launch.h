@@ -170,9 +170,8 @@ struct TraceArgs {
 hipError_t launch_trace_window(const TraceArgs& a, const RaySoA& rays, const HitSoA& hits,
                                uint8_t* occluded, bool any, uint32_t lanes, uint32_t block,
                                hipStream_t s);
-// Two-level traversal (a.cellrec set): closest hit into hits, or any hit into
-// occluded when it is set; one ray per lane (lanes <= 1) or `lanes` (2..16)
-// lanes per ray walking its top cells in turn.
+// The same over the two-level grid (a.cellrec set): closest hit into hits, or
+// any hit into occluded when it is set.
 hipError_t launch_trace2(const TraceArgs& a, const RaySoA& rays, const HitSoA& hits,
                          uint8_t* occluded, uint32_t lanes, hipStream_t s);
 // One item of a batched launch: a ray batch against one scene's grid.  The

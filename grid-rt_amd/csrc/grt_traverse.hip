@@ -18,7 +18,7 @@
 //
 //   k_trace_window        one-level grid, 1..16 lanes per ray (grt_window.h)
 //   k_trace_batch_window  the same over the items of a batch
-//   k_trace2, _split      two-level grid
+//   k_trace2_window       two-level grid, 1..16 lanes per ray
 #include "grt_launch.h"
 #include "grt_mt.h"
 #include "grt_window.h"
@@ -241,7 +241,8 @@ __device__ __forceinline__ void trace_window(const DevFrame* __restrict__ fr,
 #pragma unroll
             for (uint32_t s = 0; s < (uint32_t)S; ++s)
                 n[s] = s < visited ? n[s] - b[s] : 0u;
-            const unsigned long long key = win_tests<ANY, S>(W, trir, b, n, bound, owner, cell0);
+            const unsigned long long key = win_tests<ANY, false, S>(
+                W, WinRecs{trir, trir}, b, n, bound, 0u, owner, cell0);
             const bool hit = key != ~0ull;
             uint32_t hs = win_cell(key) - cell0;
             hs = hs < c ? hs : (uint32_t)S;   // S: not one of the lane's cells
@@ -350,51 +351,34 @@ __global__ __launch_bounds__(256) void k_task_map(const BatchTask* __restrict__ 
 }
 
 // ---------------------------------------------------------------------------
-// Host launchers
-// ---------------------------------------------------------------------------
-static uint32_t ray_grid(uint32_t n, uint32_t img_w, uint32_t block)
-{
-    return (uint32_t)((slot_count(n, img_w) + block - 1) / block);
-}
-
-// ---------------------------------------------------------------------------
-// Two-level grid: one ray per lane
+// Two-level grid: windowed walk
 // ---------------------------------------------------------------------------
 //
-// The top DDA as in the one-level kernels; a top cell whose record carries a
-// sub-grid resolution is walked by a DDA of its own from the point where the
-// ray entered the cell (the clipped entry, then each top cell's exit), with
-// hits bounded by the sub-cell's exit; other cells test their references
-// bounded by the cell's exit.  The first (sub-)cell holding a hit ends a
-// closest-hit ray, the first triangle in (tmin, tmax] an any-hit ray.
-// Counters: top cells plus sub-cells visited, triangle tests.
+// The walk over the top grid goes item by item.  An item is a cell of the
+// grid; for an empty cell with skip radius rr > 0 it is the cells ahead of it
+// within rr on every axis (all empty), left in one step.  Each item's exit is
+// its first boundary plane crossed, from the plane formula of the DDA set-up
+// (t = ((float)k cell_a + bmin_a - o_a) / d_a), in the DDA's tie order.  A top
+// cell whose record carries a sub-grid resolution is walked by a DDA of its
+// own from the point where the ray entered the cell (the clipped entry, then
+// each item's exit), with hits bounded by the sub-cell's exit; other cells
+// test their references bounded by the cell's exit.  The first (sub-)cell
+// holding a hit ends a closest-hit ray, the first triangle in (tmin, tmax] an
+// any-hit ray, and a sub-cell whose exit lies beyond tmax ends either.
+// Counters: top items plus sub-cells visited, triangle tests.
 
-// Tests records [b, e) of `rec`: closest (bound) or any.  True when the ray is
-// done (a hit in this cell, or an occluder).
-template <bool ANY>
-__device__ __forceinline__ bool trace2_cell(const float4* __restrict__ rec, uint32_t b,
-                                            uint32_t e, float o0, float o1, float o2, float d0,
-                                            float d1, float d2, float tmin, float tmax,
-                                            float bound, int32_t& id, float& best, float& bu,
-                                            float& bv, uint32_t& tests)
-{
-    return test_records<ANY>(rec, b, e, o0, o1, o2, d0, d1, d2, tmin, tmax, bound, id, best, bu,
-                             bv, tests);
-}
-
-__device__ __forceinline__ int32_t sub_vox(float val, float bmin, float inv, int32_t r)
-{
-    float x = (val - bmin) * inv;
-    x = x > 0.0f ? x : 0.0f;
-    const float hi = (float)(r - 1);
-    x = x < hi ? x : hi;
-    return (int32_t)x;
-}
+// Top items per window at most, and the lanes below which another one waits
+// for the next window while other lanes stand in sub-grids (stadium at
+// 1920x1080, us, primary / shadow / bounce: 692 / 666 / 1057 with 2 items a
+// window, 676 / 669 / 1022 with 4, 685 / 685 / 1037 with 8; 688 / 695 / 1058
+// without the wait).
+constexpr int kTopSteps = 4;
+constexpr int kTopMin = 16;
 
 // Per-ray constants of the two-level walk.
 struct Ray2 {
     float o0, o1, o2, d0, d1, d2, i0, i1, i2, tmin, tmax;
-    bool n0, n1, n2;
+    int32_t m0, m1, m2;   // -1 on the axes of negative direction, else 0
 };
 
 // Sub-cell sizes and their reciprocals by resolution, staged in LDS by every
@@ -408,19 +392,24 @@ __device__ __forceinline__ void stage_sub_tab(const TraceArgs& a, float* tab)
     __syncthreads();
 }
 
-// DDA state inside a top cell's sub-grid: current sub-cell (and its index si
-// in the sub-cell arrays, which a step along y or z changes by sy or sz; by
-// +-1 along x), next boundary crossings and their increments.
-struct Sub2 {
-    uint32_t si, sy, sz;
-    int32_t qx, qy, qz, ox, oy, oz;
+// DDA state inside a top cell's sub-grid: the sub-cell's index in the sub-cell
+// arrays, which a step along y or z changes by sy or sz (by +-1 along x), the
+// steps left on each axis before the sub-grid ends (8 bits each), the next
+// boundary crossings and their increments.
+struct SubW {
+    uint32_t si, sy, sz, left;
     float tx, ty, tz, dtx, dty, dtz;
 };
 
+// vox(): the clamp as one median (NaN goes to 0 as there).
+__device__ __forceinline__ int32_t vox_median(float val, float bmin, float inv, float hi)
+{
+    return (int32_t)__builtin_amdgcn_fmed3f((val - bmin) * inv, 0.0f, hi);
+}
+
 // Entry into the sub-grid of the top cell at s (record rec) at t_enter.
-__device__ __forceinline__ void sub_setup(const DevFrame* __restrict__ fr, const float* tab,
-                                          const Ray2& r, const Dda& s, uint2 rec, float t_enter,
-                                          Sub2& q)
+__device__ __forceinline__ SubW sub_setup(const DevFrame* __restrict__ fr, const float* tab,
+                                          const Ray2& r, const Dda& s, uint2 rec, float t_enter)
 {
     const uint32_t base = rec.x & 0x7fffffffu;
     const int32_t r0 = (int32_t)(rec.y & 255u);
@@ -431,96 +420,43 @@ __device__ __forceinline__ void sub_setup(const DevFrame* __restrict__ fr, const
     const float sb2 = (float)s.cz * fr->cell[2] + fr->bmin[2];
     const float sc0 = tab[r0 - 1], sc1 = tab[16 + r1 - 1], sc2 = tab[32 + r2 - 1];
     const float si0 = tab[48 + r0 - 1], si1 = tab[64 + r1 - 1], si2 = tab[80 + r2 - 1];
-    q.qx = sub_vox(r.o0 + r.d0 * t_enter, sb0, si0, r0);
-    q.qy = sub_vox(r.o1 + r.d1 * t_enter, sb1, si1, r1);
-    q.qz = sub_vox(r.o2 + r.d2 * t_enter, sb2, si2, r2);
-    q.ox = r.n0 ? -1 : r0;
-    q.oy = r.n1 ? -1 : r1;
-    q.oz = r.n2 ? -1 : r2;
-    q.tx = ((float)(q.qx + (r.n0 ? 0 : 1)) * sc0 + sb0 - r.o0) * r.i0;
-    q.ty = ((float)(q.qy + (r.n1 ? 0 : 1)) * sc1 + sb1 - r.o1) * r.i1;
-    q.tz = ((float)(q.qz + (r.n2 ? 0 : 1)) * sc2 + sb2 - r.o2) * r.i2;
+    const int32_t qx = vox_median(r.o0 + r.d0 * t_enter, sb0, si0, (float)(r0 - 1));
+    const int32_t qy = vox_median(r.o1 + r.d1 * t_enter, sb1, si1, (float)(r1 - 1));
+    const int32_t qz = vox_median(r.o2 + r.d2 * t_enter, sb2, si2, (float)(r2 - 1));
+    SubW q;
+    q.left = (uint32_t)(r.m0 ? qx : r0 - 1 - qx) | (uint32_t)(r.m1 ? qy : r1 - 1 - qy) << 8 |
+             (uint32_t)(r.m2 ? qz : r2 - 1 - qz) << 16;
+    q.tx = ((float)(qx + 1 + r.m0) * sc0 + sb0 - r.o0) * r.i0;
+    q.ty = ((float)(qy + 1 + r.m1) * sc1 + sb1 - r.o1) * r.i1;
+    q.tz = ((float)(qz + 1 + r.m2) * sc2 + sb2 - r.o2) * r.i2;
     q.dtx = fabsf(sc0 * r.i0);
     q.dty = fabsf(sc1 * r.i1);
     q.dtz = fabsf(sc2 * r.i2);
-    q.si = base + (uint32_t)q.qx +
-           (uint32_t)r0 * ((uint32_t)q.qy + (uint32_t)r1 * (uint32_t)q.qz);
-    q.sy = r.n1 ? 0u - (uint32_t)r0 : (uint32_t)r0;
-    q.sz = r.n2 ? 0u - (uint32_t)(r0 * r1) : (uint32_t)(r0 * r1);
+    q.si = base + (uint32_t)qx + (uint32_t)r0 * ((uint32_t)qy + (uint32_t)r1 * (uint32_t)qz);
+    // r0 and r0 r1, negated on the axes of negative direction
+    q.sy = (uint32_t)((r0 ^ r.m1) - r.m1);
+    q.sz = (uint32_t)((r0 * r1 ^ r.m2) - r.m2);
+    return q;
 }
 
-// One sub-grid step (the top DDA's tie order); false when it leaves the grid
-// (q is then left as it was).  Branch-free: the crossed axis selects which
-// coordinate, crossing and index change.
-__device__ __forceinline__ bool sub_step(const Ray2& r, Sub2& q)
+// Leaves the current sub-cell (the top DDA's tie order): its exit t, and
+// whether the next one is in the sub-grid.  The state is meaningless once it
+// is not.
+__device__ __forceinline__ float sub_step(SubW& q, uint32_t sx, bool& in)
 {
-    const bool ax = q.tx < q.ty && q.tx < q.tz;
-    const bool ay = !ax && q.ty < q.tz;
+    const float tx = q.tx, ty = q.ty, tz = q.tz;   // values: as in dda_window_step
+    const uint32_t sy = q.sy, sz = q.sz;
+    const bool ax = tx < ty && tx < tz;
+    const bool ay = !ax && ty < tz;
     const bool az = !ax && !ay;
-    const int32_t dx = r.n0 ? -1 : 1;
-    const int32_t qx = ax ? q.qx + dx : q.qx;
-    const int32_t qy = ay ? q.qy + (r.n1 ? -1 : 1) : q.qy;
-    const int32_t qz = az ? q.qz + (r.n2 ? -1 : 1) : q.qz;
-    if ((ax && qx == q.ox) || (ay && qy == q.oy) || (az && qz == q.oz))
-        return false;
-    q.qx = qx;
-    q.qy = qy;
-    q.qz = qz;
-    const float tx = q.tx + q.dtx, ty = q.ty + q.dty, tz = q.tz + q.dtz;
-    q.tx = ax ? tx : q.tx;
-    q.ty = ay ? ty : q.ty;
-    q.tz = az ? tz : q.tz;
-    q.si += ax ? (uint32_t)dx : (ay ? q.sy : q.sz);
-    return true;
-}
-
-// One non-empty top cell (index ci, coordinates of s, record rec) of the
-// two-level walk, entered at t_enter and left at exit_t: its sub-grid from t_enter when it has one and
-// the second level is valid, else its own references bounded by exit_t.
-// Counts the sub-cells visited and the tests.  True when the walk ends in this
-// cell: a hit (closest), an occluder (any, *occ set) or a sub-cell whose exit
-// lies beyond tmax.
-template <bool ANY>
-__device__ __forceinline__ bool top_cell2(const TraceArgs& a, const DevFrame* __restrict__ fr,
-                                          const float* tab, bool sub_ok, const Ray2& r,
-                                          const Dda& s, uint2 rec, uint32_t ci, float t_enter,
-                                          float exit_t, bool& occ, int32_t& id, float& best,
-                                          float& bu, float& bv, uint32_t& cells,
-                                          uint32_t& tests)
-{
-    const bool has_sub = (rec.x >> 31) != 0u;
-    if (!(sub_ok && has_sub)) {
-        // the top cell's own list (also for a sub-grid cell when the second
-        // level is not valid)
-        const uint32_t kb = has_sub ? a.offsets[ci] : rec.x;
-        const uint32_t ke = has_sub ? a.offsets[ci + 1] : rec.y;
-        if (trace2_cell<ANY>(a.trir, kb, ke, r.o0, r.o1, r.o2, r.d0, r.d1, r.d2, r.tmin, r.tmax,
-                             exit_t * kExitScale, id, best, bu, bv, tests)) {
-            occ = ANY;
-            return true;
-        }
-        return false;
-    }
-    Sub2 q;
-    sub_setup(fr, tab, r, s, rec, t_enter, q);
-    uint32_t kb = a.sub_offsets[q.si], ke = a.sub_offsets[q.si + 1];
-    for (;;) {
-        ++cells;
-        const float sexit = tmin_f(tmin_f(q.tx, q.ty), q.tz);
-        // the next sub-cell and its offsets, loaded before this one's tests
-        // (unconditionally: a step out of the sub-grid leaves q.si in place)
-        const uint32_t cb = kb, ce = ke;
-        const bool more = sub_step(r, q);
-        kb = a.sub_offsets[q.si];
-        ke = a.sub_offsets[q.si + 1];
-        if (trace2_cell<ANY>(a.sub_trir, cb, ce, r.o0, r.o1, r.o2, r.d0, r.d1, r.d2, r.tmin,
-                             r.tmax, sexit * kExitScale, id, best, bu, bv, tests)) {
-            occ = ANY;
-            return true;
-        }
-        if (sexit > r.tmax || !more)
-            return sexit > r.tmax;
-    }
+    const uint32_t sh = ax ? 0u : (ay ? 8u : 16u);
+    in = ((q.left >> sh) & 255u) != 0u;
+    q.left -= 1u << sh;
+    q.tx = ax ? tx + q.dtx : tx;
+    q.ty = ay ? ty + q.dty : ty;
+    q.tz = az ? tz + q.dtz : tz;
+    q.si += ax ? sx : (ay ? sy : sz);
+    return ax ? tx : (ay ? ty : tz);
 }
 
 // Set-up of a two-level ray: constants, the top DDA and the clipped entry.
@@ -545,17 +481,11 @@ __device__ __forceinline__ bool ray2_setup(const DevFrame* __restrict__ fr, cons
     t_enter = tmax_f(t_enter, tmin_f((fr->bmin[0] - r.o0) * r.i0, (fr->bmax[0] - r.o0) * r.i0));
     t_enter = tmax_f(t_enter, tmin_f((fr->bmin[1] - r.o1) * r.i1, (fr->bmax[1] - r.o1) * r.i1));
     t_enter = tmax_f(t_enter, tmin_f((fr->bmin[2] - r.o2) * r.i2, (fr->bmax[2] - r.o2) * r.i2));
-    r.n0 = __builtin_signbit(r.d0);
-    r.n1 = __builtin_signbit(r.d1);
-    r.n2 = __builtin_signbit(r.d2);
+    r.m0 = __float_as_int(r.d0) >> 31;
+    r.m1 = __float_as_int(r.d1) >> 31;
+    r.m2 = __float_as_int(r.d2) >> 31;
     return true;
 }
-
-// The walk over the top grid goes item by item.  An item is a cell of the
-// grid; for an empty cell with skip radius rr > 0 it is the cells ahead of it
-// within rr on every axis (all empty), left in one step.  Each item's exit is
-// its first boundary plane crossed, from the plane formula of the DDA set-up
-// (t = ((float)k cell_a + bmin_a - o_a) / d_a), in the DDA's tie order.
 
 // Skip radius of a cell record: {r, r} marks an empty cell.
 __device__ __forceinline__ int32_t skip_radius(uint2 rec, bool& empty)
@@ -564,249 +494,298 @@ __device__ __forceinline__ int32_t skip_radius(uint2 rec, bool& empty)
     return empty && rec.x <= (uint32_t)kSkipMax ? (int32_t)rec.x : 0;
 }
 
-// Exit t of the item at the walk's cell s with radius rr; axis: the axis
-// crossed.
-__device__ __forceinline__ float item_exit(const DevFrame* __restrict__ fr, const Ray2& r,
-                                           const Dda& s, int32_t rr, int& axis)
+// The item at the walk's cell s with skip radius rr: its exit t, the axis
+// crossed there, and on every axis the cell before the exit plane -- rr cells
+// ahead of s (behind, for a negative direction).
+struct Item {
+    float e;
+    bool ax, ay;
+    int32_t fx, fy, fz;
+};
+
+// (rr ^ m) + c: with m = -1 for a negative direction, else 0, the cell rr
+// ahead of c is that minus m and the index of its exit plane that plus 1.
+__device__ __forceinline__ Item item_exit(const DevFrame* __restrict__ fr, const Ray2& r,
+                                          const Dda& s, int32_t rr)
 {
-    const float t0 =
-        ((float)(r.n0 ? s.cx - rr : s.cx + rr + 1) * fr->cell[0] + fr->bmin[0] - r.o0) * r.i0;
-    const float t1 =
-        ((float)(r.n1 ? s.cy - rr : s.cy + rr + 1) * fr->cell[1] + fr->bmin[1] - r.o1) * r.i1;
-    const float t2 =
-        ((float)(r.n2 ? s.cz - rr : s.cz + rr + 1) * fr->cell[2] + fr->bmin[2] - r.o2) * r.i2;
-    if (t0 < t1 && t0 < t2) {
-        axis = 0;
-        return t0;
-    }
-    if (t1 < t2) {
-        axis = 1;
-        return t1;
-    }
-    axis = 2;
-    return t2;
+    const int32_t hx = (rr ^ r.m0) + s.cx, hy = (rr ^ r.m1) + s.cy, hz = (rr ^ r.m2) + s.cz;
+    const float t0 = ((float)(hx + 1) * fr->cell[0] + fr->bmin[0] - r.o0) * r.i0;
+    const float t1 = ((float)(hy + 1) * fr->cell[1] + fr->bmin[1] - r.o1) * r.i1;
+    const float t2 = ((float)(hz + 1) * fr->cell[2] + fr->bmin[2] - r.o2) * r.i2;
+    Item it;
+    it.ax = t0 < t1 && t0 < t2;
+    it.ay = !it.ax && t1 < t2;
+    it.e = it.ax ? t0 : (it.ay ? t1 : t2);
+    it.fx = hx - r.m0;
+    it.fy = hy - r.m1;
+    it.fz = hz - r.m2;
+    return it;
 }
 
-// v kept within the rr cells ahead of c (behind, for a negative direction).
-__device__ __forceinline__ int32_t skip_cell(int32_t v, int32_t c, int32_t rr, bool neg)
+// a, b, c's median: v kept between two cells in either order.
+__device__ __forceinline__ int32_t median(int32_t a, int32_t b, int32_t c)
 {
-    if (neg) {
-        v = v < c ? v : c;
-        return v > c - rr ? v : c - rr;
-    }
-    v = v > c ? v : c;
-    return v < c + rr ? v : c + rr;
+    const int32_t lo = a < b ? a : b, hi = a < b ? b : a, m = hi < c ? hi : c;
+    return lo > m ? lo : m;
 }
 
-// Step to the next item across the current one's exit (axis, at t = e);
-// false when that leaves the grid.  After a skip (rr > 0) the other two
-// axes take the cells of the exit point, kept within the skipped cells: no
-// axis ever moves backwards, and the crossed one moves by rr + 1.
+// Step to the next item across the current one's exit; false when that leaves
+// the grid (s is then meaningless).  The crossed axis takes the cell beyond
+// the exit plane.  After a skip (rr > 0) the other two take the cells of the
+// exit point, kept within the skipped cells, so no axis ever moves backwards;
+// without one those are the current cells, so no lane branches.
 __device__ __forceinline__ bool item_advance(const DevFrame* __restrict__ fr, const Ray2& r,
-                                             Dda& s, int32_t rr, int axis, float e)
+                                             Dda& s, const Item& it)
 {
-    if (axis == 0) {
-        const int32_t c = r.n0 ? s.cx - rr - 1 : s.cx + rr + 1;
-        if (c < 0 || c >= fr->n[0])
-            return false;
-        s.cx = c;
-    } else if (axis == 1) {
-        const int32_t c = r.n1 ? s.cy - rr - 1 : s.cy + rr + 1;
-        if (c < 0 || c >= fr->n[1])
-            return false;
-        s.cy = c;
-    } else {
-        const int32_t c = r.n2 ? s.cz - rr - 1 : s.cz + rr + 1;
-        if (c < 0 || c >= fr->n[2])
-            return false;
-        s.cz = c;
-    }
-    if (rr > 0) {
-        if (axis != 0)
-            s.cx = skip_cell(vox(r.o0 + r.d0 * e, fr->bmin[0], fr->inv[0], fr->n[0]), s.cx, rr,
-                             r.n0);
-        if (axis != 1)
-            s.cy = skip_cell(vox(r.o1 + r.d1 * e, fr->bmin[1], fr->inv[1], fr->n[1]), s.cy, rr,
-                             r.n1);
-        if (axis != 2)
-            s.cz = skip_cell(vox(r.o2 + r.d2 * e, fr->bmin[2], fr->inv[2], fr->n[2]), s.cz, rr,
-                             r.n2);
-    }
-    return true;
+    const int32_t kx = median(vox_median(r.o0 + r.d0 * it.e, fr->bmin[0], fr->inv[0],
+                                         (float)(fr->n[0] - 1)), s.cx, it.fx);
+    const int32_t ky = median(vox_median(r.o1 + r.d1 * it.e, fr->bmin[1], fr->inv[1],
+                                         (float)(fr->n[1] - 1)), s.cy, it.fy);
+    const int32_t kz = median(vox_median(r.o2 + r.d2 * it.e, fr->bmin[2], fr->inv[2],
+                                         (float)(fr->n[2] - 1)), s.cz, it.fz);
+    const bool az = !it.ax && !it.ay;
+    s.cx = it.ax ? it.fx + 2 * r.m0 + 1 : kx;
+    s.cy = it.ay ? it.fy + 2 * r.m1 + 1 : ky;
+    s.cz = az ? it.fz + 2 * r.m2 + 1 : kz;
+    const uint32_t n = (uint32_t)(it.ax ? fr->n[0] : (it.ay ? fr->n[1] : fr->n[2]));
+    return (uint32_t)(it.ax ? s.cx : (it.ay ? s.cy : s.cz)) < n;
 }
 
-template <bool ANY>
-__global__ __launch_bounds__(128) void k_trace2(TraceArgs a, RaySoA rays, HitSoA hits,
-                                                uint8_t* __restrict__ occluded)
+// A wave walks its rays in windows as trace_window does, `lanes` lanes per ray
+// (lanes x S <= 16 units a window): a unit is a top cell's list or a
+// sub-cell's, unit u of the window going to lane u / S of the group.  A window
+// is a few top items, until the lane stands in a sub-grid or its units are
+// used up, then sub-cells up to the window's end.
+//
+// Bound by VALU issue while the chip is full (0.69 of the cycles over the whole
+// launch, 8.7 k instructions a wave on primary rays, of which the top walk is
+// two fifths and the tests a quarter), then by the longest waves: one wave
+// alone takes up to 0.42 ms with a ray per lane, 0.18 ms with 16 lanes per ray.
+// The per-lane walk this replaced ran 15-32 of 64 lanes per instruction, this
+// one 33-44.  Stadium of 2^20 triangles, us before -> after: 1920x1080 primary
+// 821 -> 676, shadow 1110 -> 669, bounce 1463 -> 1022; 480x270 primary 768 ->
+// 293, shadow 1305 -> 211.  Waves that take new rays as lanes fall idle were
+// slower (primary 1229 us): rays of different image parts share fewer steps.
+// The next window's loads before this one's tests cost a wave per SIMD
+// (primary 854 against 746 us).
+template <bool ANY, bool COUNT, int S>
+__global__ __launch_bounds__(128) void k_trace2_window(TraceArgs a, RaySoA rays, HitSoA hits,
+                                                       uint8_t* __restrict__ occluded,
+                                                       uint32_t lanes)
 {
     __shared__ float tab[96];
     stage_sub_tab(a, tab);
-    const uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
+    WaveWin& W = win_lds[threadIdx.x >> 6];
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t j = lane & (lanes - 1u), owner = lane - j, cell0 = j * (uint32_t)S;
+    const uint32_t units = lanes * (uint32_t)S;
     bool valid;
-    const uint32_t i = trace_ray(a, slot, valid);
-    if (!valid)
-        return;
+    const uint32_t i = trace_ray(
+        a, (blockIdx.x * blockDim.x + threadIdx.x) >> __builtin_ctz(lanes), valid);
     const DevFrame* __restrict__ fr = a.fr;
-    int32_t id = -1;
-    float best = INFINITY, bu = 0.0f, bv = 0.0f;
-    bool occ = false;
-    uint32_t cells = 0, tests = 0;
+    const uint32_t nx = (uint32_t)fr->n[0], ny = (uint32_t)fr->n[1];
     // Over its capacity the second level's records are not complete: the top
     // grid alone then.
     const bool sub_ok = a.g2->status == 0;
-    Ray2 r;
-    Dda s;
-    float t_enter;
-    if (ray2_setup(fr, rays, i, r, s, t_enter)) {
-        const uint32_t nx = (uint32_t)fr->n[0], ny = (uint32_t)fr->n[1];
-        uint32_t ci = (uint32_t)s.cx + nx * ((uint32_t)s.cy + ny * (uint32_t)s.cz);
-        uint2 rec = a.cellrec[ci];
-        for (;;) {
-            ++cells;
-            bool empty;
-            const int32_t rr = skip_radius(rec, empty);
-            int axis;
-            const float e = item_exit(fr, r, s, rr, axis);
-            // the next item and its record, loaded before this cell's tests
-            Dda ns = s;
-            const bool more = !(e > r.tmax) && item_advance(fr, r, ns, rr, axis, e);
-            const uint32_t nci =
-                (uint32_t)ns.cx + nx * ((uint32_t)ns.cy + ny * (uint32_t)ns.cz);
-            // ns is inside the grid whether or not the walk goes on
-            const uint2 nrec = a.cellrec[nci];
-            if ((!empty && top_cell2<ANY>(a, fr, tab, sub_ok, r, s, rec, ci, t_enter, e, occ, id,
-                                          best, bu, bv, cells, tests)) ||
-                !more)
-                break;
-            t_enter = e;
-            s = ns;
-            ci = nci;
-            rec = nrec;
-        }
-    }
-    if (ANY) {
-        occluded[i] = occ ? 1 : 0;
-    } else {
-        hits.id[i] = id;
-        hits.t[i] = best;
-        hits.u[i] = bu;
-        hits.v[i] = bv;
-    }
-    if (a.counters) {
-        a.counters[2ull * i] = cells;
-        a.counters[2ull * i + 1] = tests;
-    }
-}
-
-// `count` items of the walk, each after checking its exit against tmax (the
-// serial walk's stop); t_enter receives the exit of the last item left.
-__device__ __forceinline__ bool walk_skip(const TraceArgs& a, const DevFrame* __restrict__ fr,
-                                          const Ray2& r, Dda& s, uint32_t count, float& t_enter)
-{
-    const uint32_t nx = (uint32_t)fr->n[0], ny = (uint32_t)fr->n[1];
-    for (uint32_t q = 0; q < count; ++q) {
-        const uint32_t ci = (uint32_t)s.cx + nx * ((uint32_t)s.cy + ny * (uint32_t)s.cz);
-        bool empty;
-        const int32_t rr = skip_radius(a.cellrec[ci], empty);
-        int axis;
-        const float e = item_exit(fr, r, s, rr, axis);
-        if (e > r.tmax || !item_advance(fr, r, s, rr, axis, e))
-            return false;
-        t_enter = e;
-    }
-    return true;
-}
-
-// Several lanes per ray (2..16, `lanes`): lane j of a ray's group walks the
-// ray's top cells j, j + lanes, ... of the serial order, each one whole (its
-// sub-grid included).  After every round the group's earliest cell that ends
-// the walk (a hit, an occluder, a sub-cell exit beyond tmax) decides: its
-// result is the serial result, and the cells after it in that round are not
-// counted.  Latency of a long ray drops about `lanes`-fold; the sparse
-// secondary stages are bound by it.
-template <bool ANY>
-__global__ __launch_bounds__(256) void k_trace2_split(TraceArgs a, RaySoA rays, HitSoA hits,
-                                                      uint8_t* __restrict__ occluded,
-                                                      uint32_t lanes)
-{
-    __shared__ float tab[96];
-    stage_sub_tab(a, tab);
-    const uint32_t shift = (uint32_t)__builtin_ctz(lanes);
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    bool valid;
-    const uint32_t i = trace_ray(a, t >> shift, valid);
-    const DevFrame* __restrict__ fr = a.fr;
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t j = lane & (lanes - 1u);
-    const uint32_t g0 = lane - j;
-    const uint64_t gmask = (lanes >= 64u ? ~0ull : ((1ull << lanes) - 1ull)) << g0;
-    const bool sub_ok = a.g2->status == 0;
-    const uint32_t nx = (uint32_t)fr->n[0], ny = (uint32_t)fr->n[1];
-    int32_t id = -1;
-    float best = INFINITY, bu = 0.0f, bv = 0.0f;
-    bool occ = false;
-    uint32_t cells = 0, tests = 0;
     Ray2 r = {};
     Dda s = {};
     float t_enter = 0.0f;
-    bool alive = valid && ray2_setup(fr, rays, i, r, s, t_enter) && walk_skip(a, fr, r, s, j, t_enter);
-    bool winner = false;
-    while (__ballot(alive) != 0) {
-        const uint32_t c0 = cells, t0 = tests;
-        bool stop = false;
-        int32_t rr = 0;
-        int axis = 0;
-        float e = 0.0f;
-        if (alive) {
-            ++cells;
-            const uint32_t ci = (uint32_t)s.cx + nx * ((uint32_t)s.cy + ny * (uint32_t)s.cz);
-            const uint2 rec = a.cellrec[ci];
-            bool empty;
-            rr = skip_radius(rec, empty);
-            e = item_exit(fr, r, s, rr, axis);
-            stop = !empty && top_cell2<ANY>(a, fr, tab, sub_ok, r, s, rec, ci, t_enter, e, occ,
-                                            id, best, bu, bv, cells, tests);
-        }
-        // The group's earliest cell that ends the walk ends the ray; cells
-        // after it (higher lanes of this round) are not part of the serial walk.
-        const uint64_t sm = __ballot(alive && stop) & gmask;
-        if (sm != 0) {
-            const uint32_t jw = (uint32_t)__builtin_ctzll(sm) - g0;
-            if (alive && j > jw) {
-                cells = c0;
-                tests = t0;
+    uint2 rec = make_uint2(0u, 0u);
+    bool top = valid && ray2_setup(fr, rays, i, r, s, t_enter);   // an item of the top walk is next
+    bool open = valid;                                            // the result is not written yet
+    uint32_t cells = 0, tests = 0;
+    if (__ballot(top) != 0) {
+        W.ro[lane] = make_float4(r.o0, r.o1, r.o2, win_lo(r.tmin));
+        W.rd[lane] = make_float4(r.d0, r.d1, r.d2, r.tmin);
+        uint32_t ci = (uint32_t)s.cx + nx * ((uint32_t)s.cy + ny * (uint32_t)s.cz);
+        if (top)
+            rec = a.cellrec[ci];
+        const uint32_t sx = (uint32_t)(r.m0 | 1);
+        bool insub = false;   // the walk stands in a sub-grid
+        SubW w = {};
+        WinU<S> nb, nn, nend, ncum;
+        uint32_t nsubs;
+        const auto next_window = [&]() {
+            uint32_t u = 0, idx[S];
+            nsubs = 0;
+#pragma unroll
+            for (int q = 0; q < S; ++q) {
+                nb[q] = 0u;
+                nn[q] = 0u;
+                nend[q] = ANY ? __float_as_uint(r.tmax) : 0u;
+                ncum[q] = 0u;
+                idx[q] = 0u;
             }
-            winner = alive && j == jw && (ANY ? occ : id >= 0);
-            alive = false;
-        } else if (alive) {
-            alive = !(e > r.tmax) && item_advance(fr, r, s, rr, axis, e);   // NaN tmax: no stop
-            if (alive) {
-                t_enter = e;
-                alive = walk_skip(a, fr, r, s, lanes - 1u, t_enter);
+            for (int k = 0; k < kTopSteps; ++k) {
+                const bool need = top && !insub && u < units;
+                const uint64_t m = __ballot(need);
+                if (m == 0 || (k != 0 && __popcll(m) < kTopMin && __ballot(insub) != 0))
+                    break;
+                if (need) {
+                    ++cells;
+                    bool empty;
+                    const int32_t rr = skip_radius(rec, empty);
+                    const Item it = item_exit(fr, r, s, rr);
+                    const bool has_sub = (rec.x >> 31) != 0u;
+                    if (!empty && has_sub && sub_ok) {
+                        w = sub_setup(fr, tab, r, s, rec, t_enter);
+                        insub = true;
+                    } else if (!empty) {
+                        // the top cell's own list (also for a sub-grid cell
+                        // when the second level is not valid)
+                        if (has_sub)
+                            rec = make_uint2(a.offsets[ci], a.offsets[ci + 1]);
+                        const uint32_t bound = __float_as_uint(win_end(r.tmax, it.e * kExitScale));
+#pragma unroll
+                        for (int q = 0; q < S; ++q) {
+                            const bool mine = u == cell0 + (uint32_t)q;
+                            nb[q] = mine ? rec.x : uint32_t(nb[q]);
+                            nn[q] = mine ? rec.y - rec.x : uint32_t(nn[q]);
+                            if (!ANY)
+                                nend[q] = mine ? bound : uint32_t(nend[q]);
+                            if (COUNT)
+                                ncum[q] = mine ? cells : uint32_t(ncum[q]);
+                        }
+                        ++u;
+                    }
+                    top = item_advance(fr, r, s, it) && !(it.e > r.tmax);
+                    t_enter = it.e;
+                    if (top) {
+                        ci = (uint32_t)s.cx + nx * ((uint32_t)s.cy + ny * (uint32_t)s.cz);
+                        rec = a.cellrec[ci];
+                    }
+                }
             }
+            if (__ballot(insub) == 0)
+                return;
+            for (uint32_t jj = 0; jj < lanes; ++jj) {
+#pragma unroll
+                for (int q = 0; q < S; ++q) {
+                    if (insub && jj * (uint32_t)S + (uint32_t)q >= u) {
+                        const bool mine = lanes == 1u || jj == j;
+                        ++cells;
+                        idx[q] = mine ? uint32_t(w.si) : idx[q];
+                        nsubs |= mine ? 1u << q : 0u;
+                        if (COUNT)
+                            ncum[q] = mine ? cells : uint32_t(ncum[q]);
+                        const float ex = sub_step(w, sx, insub);
+                        if (!ANY) {
+                            const uint32_t bound =
+                                __float_as_uint(win_end(r.tmax, ex * kExitScale));
+                            nend[q] = mine ? bound : uint32_t(nend[q]);
+                        }
+                        if (ex > r.tmax) {
+                            insub = false;
+                            top = false;
+                        }
+                    }
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < S; ++q) {
+                const uint32_t* o = a.sub_offsets + idx[q];
+                const uint32_t b = o[0], e = o[1];
+                const bool sub = (nsubs >> q) & 1u;
+                nb[q] = sub ? b : uint32_t(nb[q]);
+                nn[q] = sub ? e - b : uint32_t(nn[q]);
+            }
+        };
+        do {
+            next_window();
+            const WinU<S> b = nb, n = nn, bound = nend, cum = ncum;
+            const uint32_t subs = nsubs;
+            const unsigned long long key = win_tests<ANY, true, S>(
+                W, WinRecs{a.trir, a.sub_trir}, b, n, bound, subs, owner, cell0);
+            const bool hit = key != ~0ull;
+            const uint32_t hs = win_cell(key) - cell0;   // >= S: not one of the lane's units
+            if (COUNT && open) {
+                const bool after = hit && win_cell(key) < cell0;
+#pragma unroll
+                for (uint32_t q = 0; q < (uint32_t)S; ++q)
+                    tests += after                         ? 0u
+                             : !hit || hs >= (uint32_t)S || q < hs ? n[q]
+                             : q == hs                     ? (ANY ? win_pos(key) + 1u : n[q])
+                                                           : 0u;
+                if (hit)
+                    cells = hs < (uint32_t)S ? win_pick<S>(cum, hs) : 0u;
+            }
+            if (hit) {
+                if (ANY) {
+                    if (j == 0)
+                        occluded[i] = 1;
+                } else if (hs < (uint32_t)S) {
+                    const uint64_t k = win_pick<S>(b, hs) + win_pos(key);
+                    const float4* __restrict__ tri = (subs >> hs) & 1u ? a.sub_trir : a.trir;
+                    const float4 A = tri[3ull * k], B = tri[3ull * k + 1], C = tri[3ull * k + 2];
+                    const MtPre m = mt_pre(A, B, C, r.o0, r.o1, r.o2, r.d0, r.d1, r.d2);
+                    float t, u, v;
+                    mt_exact(m, t, u, v);
+                    hits.id[i] = (int32_t)__float_as_uint(C.y);
+                    hits.t[i] = t;
+                    hits.u[i] = u;
+                    hits.v[i] = v;
+                }
+                open = false;
+                top = false;
+                insub = false;
+            }
+        } while (__ballot(top || insub) != 0);
+        if (COUNT && open && j != 0)
+            cells = 0u;   // every lane of the group counted the whole walk
+    }
+    if (COUNT) {
+        const uint32_t sc = group_sum(cells, lanes), st = group_sum(tests, lanes);
+        if (valid && j == 0) {
+            a.counters[2ull * i] = sc;
+            a.counters[2ull * i + 1] = st;
         }
     }
-    const bool group_hit = (__ballot(winner) & gmask) != 0;
-    uint32_t sc = 0, st = 0;
-    if (a.counters) {
-        sc = group_sum(cells, lanes);
-        st = group_sum(tests, lanes);
+    if (open && j == 0) {
+        if (ANY) {
+            occluded[i] = 0;
+        } else {
+            hits.id[i] = -1;
+            hits.t[i] = INFINITY;
+            hits.u[i] = 0.0f;
+            hits.v[i] = 0.0f;
+        }
     }
-    if (!valid)
-        return;
-    if (ANY) {
-        if (j == 0)
-            occluded[i] = group_hit ? 1 : 0;
-    } else if (winner || (j == 0 && !group_hit)) {
-        hits.id[i] = winner ? id : -1;
-        hits.t[i] = winner ? best : INFINITY;
-        hits.u[i] = winner ? bu : 0.0f;
-        hits.v[i] = winner ? bv : 0.0f;
-    }
-    if (a.counters && j == 0) {
-        a.counters[2ull * i] = sc;
-        a.counters[2ull * i + 1] = st;
-    }
+}
+
+template <bool ANY, bool COUNT>
+static void trace2_launch(const TraceArgs& a, const RaySoA& rays, const HitSoA& hits,
+                          uint8_t* occluded, uint32_t lanes, uint32_t grid, hipStream_t s)
+{
+    constexpr uint32_t kBlock = 128;
+    const size_t lds = kBlock / 64 * sizeof(WaveWin);
+    if (lanes <= 4)
+        hipLaunchKernelGGL((k_trace2_window<ANY, COUNT, 4>), dim3(grid), dim3(kBlock), lds, s, a,
+                           rays, hits, occluded, lanes);
+    else if (lanes == 8)
+        hipLaunchKernelGGL((k_trace2_window<ANY, COUNT, 2>), dim3(grid), dim3(kBlock), lds, s, a,
+                           rays, hits, occluded, lanes);
+    else
+        hipLaunchKernelGGL((k_trace2_window<ANY, COUNT, 1>), dim3(grid), dim3(kBlock), lds, s, a,
+                           rays, hits, occluded, lanes);
+}
+
+// Lanes per ray of a two-level launch of `slots` ray slots.  The top walk is
+// stepped by every lane of a group, so large launches take one lane; small
+// ones are bound by their longest wave.  Measured on the stadium (us, 1 / 2 /
+// 4 / 8 / 16 lanes): 1360x765 primary 496 / 529 / 720 / - / -; 960x540 primary
+// 434 / 393 / 447 / 628 / -, shadow 419 / 295 / 389 / 528 / -, bounce 623 / 570
+// / 605 / 735 / -; 720x405 primary - / 340 / 365 / 422 / 631; 480x270 primary
+// 432 / 315 / 295 / 293 / 372, shadow 417 / 298 / 239 / 211 / 282, bounce 580 /
+// 377 / 399 / 365 / 411; 160x90 shadow 424 / 277 / 218 / 185 / 174.
+static uint32_t trace2_lanes(uint64_t slots)
+{
+    if (slots >= 1000000)
+        return 1;
+    if (slots >= 300000)
+        return 2;
+    if (slots >= 150000)
+        return 4;
+    return slots >= 32000 ? 8 : 16;
 }
 
 hipError_t launch_trace2(const TraceArgs& a, const RaySoA& rays, const HitSoA& hits,
@@ -814,27 +793,23 @@ hipError_t launch_trace2(const TraceArgs& a, const RaySoA& rays, const HitSoA& h
 {
     if (a.n == 0)
         return hipSuccess;
-    if (lanes <= 1) {
-        const uint32_t g = ray_grid(a.n, a.image_width, 128);
-        if (occluded)
-            hipLaunchKernelGGL(k_trace2<true>, dim3(g), dim3(128), 0, s, a, rays, hits, occluded);
-        else
-            hipLaunchKernelGGL(k_trace2<false>, dim3(g), dim3(128), 0, s, a, rays, hits,
-                               occluded);
-        return hipGetLastError();
-    }
     if (lanes > 16 || (lanes & (lanes - 1)) != 0)
         return hipErrorInvalidValue;
-    const uint64_t threads = slot_count(a.n, a.image_width) * lanes;
-    if (threads > 0xffffffffull - 256)
+    const uint64_t slots = slot_count(a.n, a.image_width);
+    if (lanes == 0)
+        lanes = trace2_lanes(slots);
+    const uint64_t threads = slots * lanes;
+    if (lanes > 1 && threads > 0xffffffffull - 256)
         return hipErrorInvalidValue;
-    const dim3 g((uint32_t)((threads + 255) / 256));
-    if (occluded)
-        hipLaunchKernelGGL(k_trace2_split<true>, g, dim3(256), 0, s, a, rays, hits, occluded,
-                           lanes);
+    const uint32_t g = (uint32_t)((threads + 127) / 128);
+    if (occluded && a.counters)
+        trace2_launch<true, true>(a, rays, hits, occluded, lanes, g, s);
+    else if (occluded)
+        trace2_launch<true, false>(a, rays, hits, occluded, lanes, g, s);
+    else if (a.counters)
+        trace2_launch<false, true>(a, rays, hits, occluded, lanes, g, s);
     else
-        hipLaunchKernelGGL(k_trace2_split<false>, g, dim3(256), 0, s, a, rays, hits, occluded,
-                           lanes);
+        trace2_launch<false, false>(a, rays, hits, occluded, lanes, g, s);
     return hipGetLastError();
 }
 

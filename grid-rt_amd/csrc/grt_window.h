@@ -39,7 +39,7 @@ struct WaveWin {
     uint2 seg_rb[kWinSegs];            // {first record - start, end of its hits}
     uint32_t seg_start[kWinSegs];      // first pooled test of the list
     uint32_t mark[128];
-    uint16_t seg_own[kWinSegs];        // lane | cell << 6
+    uint16_t seg_own[kWinSegs];        // lane | cell << 6 | second record array << 10
 };
 static_assert(sizeof(WaveWin) % 16 == 0, "WaveWin arrays stay 16-byte aligned");
 
@@ -97,10 +97,10 @@ __device__ __forceinline__ float win_lo(float tmin)
 }
 
 // The upper end of a list's hits: t <= end exactly when t <= tmax and t <=
-// bound, for every t above tmin.
+// bound (NaN, which no t is at most, when either is NaN).
 __device__ __forceinline__ float win_end(float tmax, float bound)
 {
-    return bound <= tmax ? bound : (tmax < bound ? tmax : -INFINITY);
+    return __builtin_elementwise_minimum(tmax, bound);
 }
 
 // One record against one ray; tbits receives the key's t part.
@@ -128,12 +128,19 @@ __device__ __forceinline__ bool win_test(const float4 A, const float4 B, const f
     return ANY || t < INFINITY;
 }
 
+// The record arrays that a window's lists point into: a two-level walk mixes
+// lists of top cells and of sub-cells.
+struct WinRecs {
+    const float4* __restrict__ top;
+    const float4* __restrict__ sub;
+};
+
 // Pooled tests [base, min(base + 64 K, end)), K consecutive ones per lane.
 // seg: lists staged, those before k0 start before base; carry: 1 + the list
 // holding the test before base.
-template <bool ANY, int K>
-__device__ __forceinline__ void win_round(WaveWin& W, const float4* __restrict__ trir,
-                                          uint32_t base, uint32_t end, uint32_t nseg, uint32_t& k0,
+template <bool ANY, bool TWO, int K>
+__device__ __forceinline__ void win_round(WaveWin& W, const WinRecs recs, uint32_t base,
+                                          uint32_t end, uint32_t nseg, uint32_t& k0,
                                           uint32_t& carry)
 {
     const uint32_t lane = threadIdx.x & 63u;
@@ -175,11 +182,12 @@ __device__ __forceinline__ void win_round(WaveWin& W, const float4* __restrict__
         const uint32_t p = base + K * lane + q;
         const uint2 rb = W.seg_rb[seg[q]];
         const uint64_t ref = (uint32_t)(rb.x + (p < end ? p : end - 1u));
-        A[q] = trir[3ull * ref];
-        B[q] = trir[3ull * ref + 1];
-        C[q] = trir[3ull * ref + 2];
-        hit_end[q] = __uint_as_float(rb.y);
         own[q] = W.seg_own[seg[q]];
+        const float4* __restrict__ rec = TWO && (own[q] & 1024u) ? recs.sub : recs.top;
+        A[q] = rec[3ull * ref];
+        B[q] = rec[3ull * ref + 1];
+        C[q] = rec[3ull * ref + 2];
+        hit_end[q] = __uint_as_float(rb.y);
     }
 #pragma unroll
     for (int q = 0; q < K; ++q) {
@@ -188,7 +196,7 @@ __device__ __forceinline__ void win_round(WaveWin& W, const float4* __restrict__
         const float4 ro = W.ro[o], rd = W.rd[o];
         uint32_t tb;
         if (p < end && win_test<ANY>(A[q], B[q], C[q], ro, rd, hit_end[q], tb))
-            atomicMin(&W.win[o], win_key(own[q] >> 6, tb, p - W.seg_start[seg[q]]));
+            atomicMin(&W.win[o], win_key((own[q] >> 6) & 15u, tb, p - W.seg_start[seg[q]]));
     }
 }
 
@@ -250,13 +258,13 @@ __device__ __forceinline__ void win_long(WaveWin& W, const float4* __restrict__ 
 // All tests of the wave's window: the lane's cells, numbers cell0.. of its
 // ray's window, hold the lists [b, b + n) (n = 0: none).  Every lane of the
 // wave calls it; W.ro and W.rd hold the rays.  The lanes that share a ray name
-// the same owner lane.  Returns the ray's key, ~0 without a hit.
-template <bool ANY, int S>
-__device__ __forceinline__ unsigned long long win_tests(WaveWin& W,
-                                                        const float4* __restrict__ trir,
+// the same owner lane.  Bit s of `subs`: list s is in the second record array
+// (TWO).  Returns the ray's key, ~0 without a hit.
+template <bool ANY, bool TWO, int S>
+__device__ __forceinline__ unsigned long long win_tests(WaveWin& W, const WinRecs recs,
                                                         const WinU<S> b, const WinU<S> n,
-                                                        const WinU<S> end, uint32_t owner,
-                                                        uint32_t cell0)
+                                                        const WinU<S> end, uint32_t subs,
+                                                        uint32_t owner, uint32_t cell0)
 {
     const uint32_t lane = threadIdx.x & 63u;
     uint32_t lists = 0, tests = 0, longm = 0;
@@ -285,7 +293,8 @@ __device__ __forceinline__ unsigned long long win_tests(WaveWin& W,
         if (n[s] != 0 && n[s] < kWinLong) {
             W.seg_start[k] = st;
             W.seg_rb[k] = make_uint2(b[s] - st, end[s]);
-            W.seg_own[k] = (uint16_t)(owner | ((cell0 + (uint32_t)s) << 6));
+            W.seg_own[k] = (uint16_t)(owner | ((cell0 + (uint32_t)s) << 6) |
+                                      (TWO ? ((subs >> s) & 1u) << 10 : 0u));
             ++k;
             st += n[s];
         }
@@ -293,9 +302,9 @@ __device__ __forceinline__ unsigned long long win_tests(WaveWin& W,
     wave_lds_sync();
     uint32_t k0 = 0, carry = 0, base = 0;
     for (; base + 64u < all_tests; base += 128u)
-        win_round<ANY, 2>(W, trir, base, all_tests, all_lists, k0, carry);
+        win_round<ANY, TWO, 2>(W, recs, base, all_tests, all_lists, k0, carry);
     if (base < all_tests)
-        win_round<ANY, 1>(W, trir, base, all_tests, all_lists, k0, carry);
+        win_round<ANY, TWO, 1>(W, recs, base, all_tests, all_lists, k0, carry);
     wave_lds_sync();
     if (any_long != 0) {
         for (;;) {
@@ -308,11 +317,14 @@ __device__ __forceinline__ unsigned long long win_tests(WaveWin& W,
             const bool skip = win_cell(W.win[owner]) < cell0 + s;
             const uint32_t lb = win_pick<S>(b, s), ln = win_pick<S>(n, s);
             const uint32_t le = win_pick<S>(end, s);
+            const float4* __restrict__ rec =
+                TWO && __builtin_amdgcn_readlane((int)((subs >> s) & 1u), (int)l) != 0 ? recs.sub
+                                                                                       : recs.top;
             if (lane == l)
                 longm &= longm - 1u;
             if (__builtin_amdgcn_readlane((int)skip, (int)l))
                 continue;
-            win_long<ANY>(W, trir, (uint32_t)__builtin_amdgcn_readlane((int)owner, (int)l),
+            win_long<ANY>(W, rec, (uint32_t)__builtin_amdgcn_readlane((int)owner, (int)l),
                           (uint32_t)__builtin_amdgcn_readlane((int)(cell0 + s), (int)l),
                           (uint32_t)__builtin_amdgcn_readlane((int)lb, (int)l),
                           (uint32_t)__builtin_amdgcn_readlane((int)ln, (int)l),

@@ -83,15 +83,14 @@ int grt_memory_used(grt_context ctx, uint64_t* bytes);
  * cudaSetBlockSize (RayTracing.h:39) was a no-op in the reference. */
 int grt_set_block_size(grt_context ctx, uint32_t closest, uint32_t any);
 
-/* Traversal scheduling.  On a one-level grid every schedule walks its rays in
- * windows of cells and spreads the triangle tests of a window over the lanes
- * of the wave.  GRT_TRACE_SIMPLE (default), GRT_TRACE_POOLED and
- * GRT_TRACE_PERSISTENT choose the lanes per ray (1 to 8) by the size of the
+/* Traversal scheduling.  Every schedule walks its rays in windows of cells and
+ * spreads the triangle tests of a window over the lanes of the wave.
+ * GRT_TRACE_SIMPLE (default), GRT_TRACE_POOLED and GRT_TRACE_PERSISTENT choose
+ * the lanes per ray (1 to 8, on a two-level grid 1 to 16) by the size of the
  * launch; their `param` (1..64) is checked and otherwise unused.
  * GRT_TRACE_SPLIT: `param` (2, 4, 8 or 16) lanes per ray, each visiting some
- * of the ray's cells; on a two-level grid lane j visits the ray's top cells
- * j, j + param, ... of the serial order (one lane per ray under the other
- * schedules).  Results and counters are identical; only the schedule differs.
+ * of the ray's cells.  Results and counters are identical; only the schedule
+ * differs.
  * The serving loop and batches (grt_batch_trace) follow the setting; a batch
  * under GRT_TRACE_SPLIT gives every ray of every item `param` lanes (64 /
  * param rays per wave). */

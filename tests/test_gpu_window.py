@@ -7,6 +7,7 @@ import pytest
 import grt
 import pyoracle as orc
 from conftest import rng
+from test_gpu_grid2 import _built, check_levels, check_trace2
 from test_gpu_parity import assert_same, check_any, check_closest, check_grid, _random_rays
 
 pytestmark = pytest.mark.gpu
@@ -45,6 +46,22 @@ def test_mixed_lists(gpu_ctx, lam, width):
     rays = orc.primary_rays(grt.camera_dict(cam)) if width else _random_rays(4099, 9)
     check_closest(sc, fr, offs, refs, v, rays, width)
     check_any(sc, fr, offs, refs, v, rays)
+
+
+# The same on two levels, with lists of both kinds (top cells, sub-cells) on
+# both sides of the length from which the wave tests a list on its own.
+@pytest.mark.parametrize("n", [31_999, 32_000, 149_999, 150_000, 299_999, 300_000, 999_999,
+                               1_000_000])
+def test_two_level_lanes_by_launch_size(gpu_ctx, n):
+    v = np.concatenate([_soup(230, 3, 1.2), _soup(400, 4, 0.02) * np.float32(0.1) +
+                        np.float32(0.45)])
+    sc = _built(gpu_ctx, v, np.zeros_like(v), 0.2, 0.1, 250)
+    fr, offs, refs, g2 = check_levels(sc, v, 0.2, 0.1, 250)
+    lens, sub = np.diff(offs), np.diff(g2[1])
+    plain = lens[(lens > 0) & (lens < 250)]
+    assert plain.max() >= 192 and plain.min() < 192 and sub.max() >= 192 and sub.min() < 192
+    check_trace2(sc, fr, offs, refs, g2, v, _random_rays(n, 5), one_level=False,
+                 modes=[("simple", 16)])
 
 
 # Both sides of every size at which the lanes per ray change.
