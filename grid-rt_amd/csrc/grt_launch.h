@@ -216,8 +216,13 @@ hipError_t launch_compact_rays(uint32_t n, uint32_t img_w, const float* tmin, co
 hipError_t launch_gen_ao(uint32_t n, uint32_t spp, uint64_t seed, const RaySoA& in,
                          const HitSoAIn& hits, const float* normals, float offset,
                          float ao_tmax, const RaySoAOut& out, hipStream_t s);
-hipError_t launch_count_active(const float* tmin, const float* tmax, uint32_t n,
-                               unsigned long long* count, hipStream_t s);
+// One step of a render request: the shadow rays of its hits and, unless mirror
+// is NULL, their mirror rays; *count grows by the active ones.  n < 2^32 - 1024.
+hipError_t launch_gen_step(uint32_t n, const RaySoA& in, const HitSoAIn& hits,
+                           const float* normals, float lx, float ly, float lz, float offset,
+                           const RaySoAOut& shadow, const RaySoAOut* mirror,
+                           unsigned long long* count, hipStream_t s);
+hipError_t launch_copy_hits(uint32_t n, const HitSoAIn& in, const HitSoA& out, hipStream_t s);
 // ---- kd-tree comparison accelerator (grt_kdtree_build.cpp, grt_kdtree.hip) ----------
 // Deepest level of a kd-tree; the device traversal keeps one stack entry per
 // level.

@@ -82,6 +82,45 @@ __device__ __forceinline__ void put_inactive(const RaySoAOut& out, uint32_t i)
     out.tmax[i] = -1.0f;
 }
 
+// Shadow ray from the hit point h with normal nn; true when it is active.
+__device__ __forceinline__ bool put_shadow(const float h[3], const float nn[3], float lx, float ly,
+                                           float lz, float offset, const RaySoAOut& out,
+                                           uint32_t i)
+{
+    const float l0 = lx - h[0], l1 = ly - h[1], l2 = lz - h[2];
+    if (dot3(nn[0], nn[1], nn[2], l0, l1, l2) <= 0.0f) {
+        put_inactive(out, i);
+        return false;
+    }
+    const float dist = sqrtf(dot3(l0, l1, l2, l0, l1, l2));
+    const float inv = 1.0f / dist;
+    out.ox[i] = h[0] + nn[0] * offset;
+    out.oy[i] = h[1] + nn[1] * offset;
+    out.oz[i] = h[2] + nn[2] * offset;
+    out.dx[i] = l0 * inv;
+    out.dy[i] = l1 * inv;
+    out.dz[i] = l2 * inv;
+    out.tmin[i] = 0.0f;
+    out.tmax[i] = dist;
+    return 0.0f <= dist;
+}
+
+// Mirror ray of direction d from the hit point h with normal nn.
+__device__ __forceinline__ void put_reflection(const float h[3], const float nn[3], float d0,
+                                               float d1, float d2, float offset,
+                                               const RaySoAOut& out, uint32_t i)
+{
+    const float proj = dot3(d0, d1, d2, nn[0], nn[1], nn[2]) * 2.0f;
+    out.ox[i] = h[0] + nn[0] * offset;
+    out.oy[i] = h[1] + nn[1] * offset;
+    out.oz[i] = h[2] + nn[2] * offset;
+    out.dx[i] = d0 - nn[0] * proj;
+    out.dy[i] = d1 - nn[1] * proj;
+    out.dz[i] = d2 - nn[2] * proj;
+    out.tmin[i] = 0.0f;
+    out.tmax[i] = INFINITY;
+}
+
 __global__ __launch_bounds__(256) void k_gen_shadow(uint32_t n, RaySoA in, HitSoAIn hits,
                                                     const float* __restrict__ normals, float lx,
                                                     float ly, float lz, float offset, RaySoAOut out)
@@ -94,25 +133,10 @@ __global__ __launch_bounds__(256) void k_gen_shadow(uint32_t n, RaySoA in, HitSo
         put_inactive(out, i);
         return;
     }
-    const float d0 = in.dx[i], d1 = in.dy[i], d2 = in.dz[i];
     float h[3], nn[3];
-    hit_frame(normals, id, hits.t[i], hits.u[i], hits.v[i], in.ox[i], in.oy[i], in.oz[i], d0, d1,
-              d2, h, nn);
-    const float l0 = lx - h[0], l1 = ly - h[1], l2 = lz - h[2];
-    if (dot3(nn[0], nn[1], nn[2], l0, l1, l2) <= 0.0f) {
-        put_inactive(out, i);
-        return;
-    }
-    const float dist = sqrtf(dot3(l0, l1, l2, l0, l1, l2));
-    const float inv = 1.0f / dist;
-    out.ox[i] = h[0] + nn[0] * offset;
-    out.oy[i] = h[1] + nn[1] * offset;
-    out.oz[i] = h[2] + nn[2] * offset;
-    out.dx[i] = l0 * inv;
-    out.dy[i] = l1 * inv;
-    out.dz[i] = l2 * inv;
-    out.tmin[i] = 0.0f;
-    out.tmax[i] = dist;
+    hit_frame(normals, id, hits.t[i], hits.u[i], hits.v[i], in.ox[i], in.oy[i], in.oz[i],
+              in.dx[i], in.dy[i], in.dz[i], h, nn);
+    put_shadow(h, nn, lx, ly, lz, offset, out, i);
 }
 
 __global__ __launch_bounds__(256) void k_gen_reflection(uint32_t n, RaySoA in, HitSoAIn hits,
@@ -131,15 +155,56 @@ __global__ __launch_bounds__(256) void k_gen_reflection(uint32_t n, RaySoA in, H
     float h[3], nn[3];
     hit_frame(normals, id, hits.t[i], hits.u[i], hits.v[i], in.ox[i], in.oy[i], in.oz[i], d0, d1,
               d2, h, nn);
-    const float proj = dot3(d0, d1, d2, nn[0], nn[1], nn[2]) * 2.0f;
-    out.ox[i] = h[0] + nn[0] * offset;
-    out.oy[i] = h[1] + nn[1] * offset;
-    out.oz[i] = h[2] + nn[2] * offset;
-    out.dx[i] = d0 - nn[0] * proj;
-    out.dy[i] = d1 - nn[1] * proj;
-    out.dz[i] = d2 - nn[2] * proj;
-    out.tmin[i] = 0.0f;
-    out.tmax[i] = INFINITY;
+    put_reflection(h, nn, d0, d1, d2, offset, out, i);
+}
+
+// The secondary rays of one step of a render request -- shadow rays and, with
+// MIRROR, mirror rays -- from one read of its hits, their active rays (tmin <=
+// tmax) added to *count.  Bound by its 48 (80 with MIRROR) bytes in and out per
+// ray plus the normals' gather.  A block takes kStepRays rays and adds to the
+// count once: with one atomic per wave on the request's one address, counting
+// 1024 x 1024 rays took 61 us, three times the generation itself.
+constexpr uint32_t kStepRays = 1024;
+
+template <bool MIRROR>
+__global__ __launch_bounds__(256) void k_gen_step(uint32_t n, RaySoA in, HitSoAIn hits,
+                                                  const float* __restrict__ normals, float lx,
+                                                  float ly, float lz, float offset,
+                                                  RaySoAOut shadow, RaySoAOut mirror,
+                                                  unsigned long long* __restrict__ count)
+{
+    __shared__ uint32_t s_active[4];
+    uint32_t active = 0;
+    for (uint32_t k = 0; k < kStepRays; k += 256u) {
+        const uint32_t i = blockIdx.x * kStepRays + k + threadIdx.x;
+        if (i >= n)
+            break;
+        const int32_t id = hits.id[i];
+        if (id < 0 || (uint32_t)id >= hits.n_tris) {
+            put_inactive(shadow, i);
+            if (MIRROR)
+                put_inactive(mirror, i);
+            continue;
+        }
+        const float d0 = in.dx[i], d1 = in.dy[i], d2 = in.dz[i];
+        float h[3], nn[3];
+        hit_frame(normals, id, hits.t[i], hits.u[i], hits.v[i], in.ox[i], in.oy[i], in.oz[i], d0,
+                  d1, d2, h, nn);
+        active += put_shadow(h, nn, lx, ly, lz, offset, shadow, i) ? 1u : 0u;
+        if (MIRROR) {
+            put_reflection(h, nn, d0, d1, d2, offset, mirror, i);
+            ++active;
+        }
+    }
+    active = wave_incl_scan(active);
+    if ((threadIdx.x & 63u) == 63u)
+        s_active[threadIdx.x >> 6] = active;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t sum = s_active[0] + s_active[1] + s_active[2] + s_active[3];
+        if (sum != 0)
+            atomicAdd(count, (unsigned long long)sum);
+    }
 }
 
 __device__ __forceinline__ uint64_t mix64(uint64_t z)
@@ -401,25 +466,39 @@ hipError_t launch_gen_ao(uint32_t n, uint32_t spp, uint64_t seed, const RaySoA& 
     return hipGetLastError();
 }
 
-// Number of active rays (tmin <= tmax) added to *count: one atomic per wave.
-__global__ __launch_bounds__(256) void k_count_active(const float* __restrict__ tmin,
-                                                      const float* __restrict__ tmax, uint32_t n,
-                                                      unsigned long long* __restrict__ count)
+__global__ __launch_bounds__(256) void k_copy_hits(uint32_t n, HitSoAIn in, HitSoA out)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool act = i < n && tmin[i] <= tmax[i];
-    const uint64_t m = __ballot(act);
-    if ((threadIdx.x & 63u) == 0 && m != 0)
-        atomicAdd(count, (unsigned long long)__popcll(m));
+    if (i >= n)
+        return;
+    out.id[i] = in.id[i];
+    out.t[i] = in.t[i];
+    out.u[i] = in.u[i];
+    out.v[i] = in.v[i];
 }
 
-hipError_t launch_count_active(const float* tmin, const float* tmax, uint32_t n,
-                               unsigned long long* count, hipStream_t s)
+hipError_t launch_gen_step(uint32_t n, const RaySoA& in, const HitSoAIn& hits,
+                           const float* normals, float lx, float ly, float lz, float offset,
+                           const RaySoAOut& shadow, const RaySoAOut* mirror,
+                           unsigned long long* count, hipStream_t s)
 {
     if (n == 0)
         return hipSuccess;
-    hipLaunchKernelGGL(k_count_active, dim3((n + 255) / 256), dim3(256), 0, s, tmin, tmax, n,
-                       count);
+    const dim3 g((n + kStepRays - 1) / kStepRays);
+    if (mirror)
+        hipLaunchKernelGGL(k_gen_step<true>, g, dim3(256), 0, s, n, in, hits, normals, lx, ly, lz,
+                           offset, shadow, *mirror, count);
+    else
+        hipLaunchKernelGGL(k_gen_step<false>, g, dim3(256), 0, s, n, in, hits, normals, lx, ly,
+                           lz, offset, shadow, RaySoAOut{}, count);
+    return hipGetLastError();
+}
+
+hipError_t launch_copy_hits(uint32_t n, const HitSoAIn& in, const HitSoA& out, hipStream_t s)
+{
+    if (n == 0)
+        return hipSuccess;
+    hipLaunchKernelGGL(k_copy_hits, dim3((n + 255) / 256), dim3(256), 0, s, n, in, out);
     return hipGetLastError();
 }
 

@@ -180,18 +180,14 @@ int issue_step(Job& j, const grt_serve_config& cfg, hipStream_t s, unsigned long
         const int c = (j.step - 1) & 1;
         const HitSoAIn hin = j.hit[c].in(j.sc->n_tris);
         const float* nrm = j.sc->normals.as<float>();
-        e = launch_gen_shadow(j.n, j.ray[c].in(), hin, nrm, cfg.light[0], cfg.light[1],
-                              cfg.light[2], cfg.offset, j.sh.out(), s);
-        if (e == hipSuccess && count)
-            e = launch_count_active(j.sh.f[6], j.sh.f[7], j.n, count, s);
+        const RaySoAOut mirror = j.ray[1 - c].out();
+        const bool bounce = j.step < j.depth;
+        e = launch_gen_step(j.n, j.ray[c].in(), hin, nrm, cfg.light[0], cfg.light[1],
+                            cfg.light[2], cfg.offset, j.sh.out(), bounce ? &mirror : nullptr,
+                            count, s);
         items.push_back(Item{j.sc, j.sh, HitSet{}, j.occ, j.n, j.width, true});
-        if (e == hipSuccess && j.step < j.depth) {
-            e = launch_gen_reflection(j.n, j.ray[c].in(), hin, nrm, cfg.offset,
-                                      j.ray[1 - c].out(), s);
-            if (e == hipSuccess && count)
-                e = launch_count_active(j.ray[1 - c].f[6], j.ray[1 - c].f[7], j.n, count, s);
+        if (bounce)
             items.push_back(Item{j.sc, j.ray[1 - c], j.hit[1 - c], nullptr, j.n, j.width, false});
-        }
     }
     return hip_check(e, "serve: ray generation");
 }
@@ -356,14 +352,9 @@ public:
             hipError_t e = hipSuccess;
             if (j.issued == 0 && r.out_hits.id && r.out_hits.t && r.out_hits.u && r.out_hits.v) {
                 // primary hits: copied before step 2 reuses the buffer (stream order)
-                const size_t b = (size_t)j.n * 4;
-                e = hipMemcpyAsync(r.out_hits.id, j.hit[0].id, b, hipMemcpyDeviceToDevice, s);
-                if (e == hipSuccess)
-                    e = hipMemcpyAsync(r.out_hits.t, j.hit[0].t, b, hipMemcpyDeviceToDevice, s);
-                if (e == hipSuccess)
-                    e = hipMemcpyAsync(r.out_hits.u, j.hit[0].u, b, hipMemcpyDeviceToDevice, s);
-                if (e == hipSuccess)
-                    e = hipMemcpyAsync(r.out_hits.v, j.hit[0].v, b, hipMemcpyDeviceToDevice, s);
+                e = launch_copy_hits(j.n, j.hit[0].in(j.sc->n_tris),
+                                     HitSoA{r.out_hits.id, r.out_hits.t, r.out_hits.u,
+                                            r.out_hits.v}, s);
             } else if (j.issued == 1 && r.out_occluded) {
                 e = hipMemcpyAsync(r.out_occluded, j.occ, j.n, hipMemcpyDeviceToDevice, s);
             }
