@@ -153,6 +153,7 @@ struct TraceArgs {
     uint32_t n;
     uint32_t image_width;   // 0: lane i traces ray i; else 8x8 pixel tiles per wave
     uint32_t* counters;     // NULL or 2 per ray {cells, tests}
+    bool flat = false;      // grid_flat() of the top grid
     const uint32_t* list = nullptr;        // or the rays to trace: slot s traces list[s] ...
     const uint32_t* list_count = nullptr;  // ... for s < *list_count (a device value) and s < n
     // Two-level grid (all set, or cellrec NULL for the top grid alone).  The
@@ -163,6 +164,14 @@ struct TraceArgs {
     const float4* sub_trir = nullptr;
     const float* sub_tab = nullptr;        // 96 floats: sub-cell sizes, reciprocals (G2Build)
 };
+// A grid whose longest axis is at least 2.5 times the cells per axis of a cube
+// of its size (the host's last known frame: it chooses a schedule only).
+inline bool grid_flat(const DevFrame& f)
+{
+    const int32_t a = f.n[0] > f.n[1] ? f.n[0] : f.n[1], n = a > f.n[2] ? a : f.n[2];
+    const double q = n / 2.5;
+    return f.m != 0 && q * q * q >= (double)f.m;
+}
 // Closest hit into hits, or any hit into occluded when `any`: waves walk their
 // rays in windows of cells, the tests of a window spread over the wave, with
 // `lanes` (1, 2, 4, 8 or 16) lanes per ray, or 0 for a number chosen by the

@@ -822,13 +822,22 @@ hipError_t launch_trace2(const TraceArgs& a, const RaySoA& rays, const HitSoA& h
 // 904x678 spheres primary 120 / 97 / 113 / 165, 1.2 M-slot batch 592 / 568 /
 // 612 / 813, 1.6 M ambient-occlusion rays with their frame 1229 / 1188 / 1276
 // / 1660, serving rounds of several million slots 9383 / 10080 / 11847 / -.
-static uint32_t window_lanes(uint64_t slots)
+//
+// Rays that run along a flat grid cross many times the cells of the others, so
+// its launches wait longer for their last waves, and up to a million slots
+// twice the lanes pay: 2^20-triangle stadium (us, 2 / 4 / 8 / 16 lanes),
+// 1280x720 frame at lambda 128 4026 / 3594 / 3517 / 4846; 960x540 primary at
+// lambda 8 6174 / 5354 / 4359 / 3312, at 64 1538 / 1341 / 1279 / 1601, at 256
+// 1044 / 907 / 1087 / 1880; 480x270 frame 2305 / 1736 / 1446 / 1419; 160x90
+// frame 2174 / 1458 / 1128 / 990.
+static uint32_t window_lanes(uint64_t slots, bool flat)
 {
     if (slots >= (4u << 20))
         return 1;
-    if (slots >= 400000)
+    if (slots >= 1000000 || (slots >= 400000 && !flat))
         return 2;
-    return slots >= 100000 ? 4 : 8;
+    const uint32_t l = slots >= 400000 ? 2 : slots >= 100000 ? 4 : 8;
+    return flat ? 2 * l : l;
 }
 
 template <bool ANY, bool COUNT>
@@ -855,7 +864,7 @@ hipError_t launch_trace_window(const TraceArgs& a, const RaySoA& rays, const Hit
         return hipErrorInvalidValue;
     const uint64_t slots = slot_count(a.n, a.image_width);
     if (lanes == 0)
-        lanes = window_lanes(slots);
+        lanes = window_lanes(slots, a.flat);
     const uint64_t threads = slots * lanes;
     if (lanes > 1 && threads > 0xffffffffull - block)
         return hipErrorInvalidValue;
@@ -885,7 +894,7 @@ hipError_t launch_trace_batch(const BatchTask* tasks, const uint32_t* map, uint3
     if (total_slots == 0)
         return hipSuccess;
     if (lanes == 0)
-        lanes = window_lanes(total_slots);
+        lanes = window_lanes(total_slots, false);
     if (lanes > 16 || (lanes & (lanes - 1)) != 0)
         return hipErrorInvalidValue;
     const uint64_t threads = (uint64_t)total_slots * lanes;
