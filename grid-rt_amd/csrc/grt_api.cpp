@@ -115,8 +115,6 @@ int grid_reserve_refs(grt_scene_t* sc, uint32_t refs)
     if ((rc = sc->refs.reserve(sc->ctx, cap * 4, false)) != GRT_OK)
         return rc;
     const uint64_t list_cap = cap / (kSortSmallCells + 1) + 1;
-    if ((rc = sc->sort_list.reserve(sc->ctx, list_cap * 4, false)) != GRT_OK)
-        return rc;
     if ((rc = sc->sort_list_small.reserve(sc->ctx, (cap / 2 + 1) * 4, false)) != GRT_OK)
         return rc;
     if ((rc = sc->sort_classes.reserve(sc->ctx, list_cap * 4 * kSortClasses, false)) != GRT_OK)
@@ -154,11 +152,11 @@ static void frame_to_info(const DevFrame& f, grt_grid_info* out)
 // The per-cell sort lists (empty before the reference buffers exist).
 static SortLists sort_lists(grt_scene_t* sc)
 {
-    if (!sc->sort_list_small.ptr || !sc->sort_list.ptr || !sc->sort_classes.ptr)
+    if (!sc->sort_list_small.ptr || !sc->sort_classes.ptr)
         return SortLists{};
-    return SortLists{sc->sort_list_small.as<uint32_t>(), sc->sort_list.as<uint32_t>(),
-                     sc->small_counters.as<uint32_t>() + 4, sc->refs_cap / 2 + 1, sc->list_cap,
-                     sc->sort_classes.as<uint32_t>()};
+    return SortLists{sc->sort_list_small.as<uint32_t>(),
+                     sc->small_counters.as<uint32_t>() + kSortCounters, sc->refs_cap / 2 + 1,
+                     sc->list_cap, sc->sort_classes.as<uint32_t>()};
 }
 
 // prefixes_ready: the tile sums were already scanned by an earlier scan of
@@ -403,7 +401,7 @@ int scene_common_buffers(grt_scene_t* sc)
         return rc;
     if ((rc = sc->partial.reserve(sc->ctx, 6 * kBBoxMaxBlocks * sizeof(float), false)) != GRT_OK)
         return rc;
-    if ((rc = sc->small_counters.reserve(sc->ctx, 64, true)) != GRT_OK)
+    if ((rc = sc->small_counters.reserve(sc->ctx, kBuildCounters * 4, true)) != GRT_OK)
         return rc;
     return GRT_OK;
 }

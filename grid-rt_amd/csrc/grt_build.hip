@@ -501,12 +501,16 @@ __global__ __launch_bounds__(256) void k_grid_pass_huge(const DevFrame* __restri
     }
 }
 
-__global__ void k_zero_build_counters(uint32_t* __restrict__ c)
+// Clears the build's counters and the scan tiles' sums.
+__global__ __launch_bounds__(256) void k_build_clear(uint32_t* __restrict__ counters,
+                                                     uint32_t* __restrict__ tile_sums,
+                                                     uint32_t tiles)
 {
-    if (threadIdx.x == 0) {
-        c[0] = 0u;
-        c[3] = 0u;
-    }
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < kBuildCounters)
+        counters[i] = 0u;
+    for (uint32_t t = i; t < tiles; t += gridDim.x * blockDim.x)
+        tile_sums[t] = 0u;
 }
 
 // Triangles on the medium list: one block per triangle, threads stride its cells.
@@ -646,8 +650,14 @@ __global__ __launch_bounds__(1024) void k_scan_blocks(uint32_t* __restrict__ bsu
     }
 }
 
+// Size class of a cell of n > kSortSmallCells references.
+__device__ __forceinline__ uint32_t sort_class(uint32_t n)
+{
+    return n <= 64u ? 0u : n <= 256u ? 1u : n <= 1024u ? 2u : n <= kSortWaveMax ? 3u : 4u;
+}
+
 // With lists.small set, also appends every cell with 2..kSortSmallCells
-// references to lists.small and every larger cell to lists.large (the cells
+// references to lists.small and every larger cell to its size class (the cells
 // the sort pass has to visit), one atomic per block and list.
 // When the total exceeds the reference capacity (kStatusRefsOver) the scatter
 // will not run, so nothing would return the counts to zero: with `clear` set
@@ -661,8 +671,8 @@ __global__ __launch_bounds__(256) void k_scan_apply(const uint32_t* __restrict__
                                                     uint32_t* clear)
 {
     __shared__ uint32_t lds[8];
-    __shared__ uint32_t lds2[8];
-    __shared__ uint32_t list_base[2];
+    __shared__ uint32_t cls[kSortClasses];   // the tile's cells per class, then their place
+    __shared__ uint32_t small_base;
     uint32_t n;
     if (!scan_len(fr, n_host, n))
         return;
@@ -731,29 +741,35 @@ __global__ __launch_bounds__(256) void k_scan_apply(const uint32_t* __restrict__
     for (int k = 0; k < 16; ++k)
         s += v[k];
     if (lists.small && !(fr->status & kStatusRefsOver)) {
-        uint32_t ns = 0, nl = 0;
+        if (threadIdx.x < (uint32_t)kSortClasses)
+            cls[threadIdx.x] = 0u;
+        __syncthreads();
+        uint32_t ns = 0;
 #pragma unroll
         for (int k = 0; k < 16; ++k) {
             ns += (v[k] >= 2u && v[k] <= kSortSmallCells) ? 1u : 0u;
-            nl += (v[k] > kSortSmallCells) ? 1u : 0u;
+            if (v[k] > kSortSmallCells)
+                atomicAdd(cls + sort_class(v[k]), 1u);
         }
-        uint32_t ts, tl;
-        uint32_t ps = block_excl_scan<256>(ns, lds, ts);
-        uint32_t pl = block_excl_scan<256>(nl, lds2, tl);
+        uint32_t ts;
+        uint32_t ps = block_excl_scan<256>(ns, lds, ts);   // barriers: the counts are complete
         if (threadIdx.x == 0) {
-            // both list lengths in one 64-bit atomic: every block adds to
-            // the same counters, and such atomics serialise (each length
+            // the two commonest lists in one 64-bit atomic: every block adds
+            // to the same counters, and such atomics serialise (each length
             // stays below 2^32, so the low half never carries)
+            const uint32_t t0 = cls[0];
             const unsigned long long old =
-                (ts | tl) ? atomicAdd(reinterpret_cast<unsigned long long*>(lists.counts),
-                                      (unsigned long long)ts | ((unsigned long long)tl << 32))
+                (ts | t0) ? atomicAdd(reinterpret_cast<unsigned long long*>(lists.counts),
+                                      (unsigned long long)ts | ((unsigned long long)t0 << 32))
                           : 0ull;
-            list_base[0] = (uint32_t)old;
-            list_base[1] = (uint32_t)(old >> 32);
+            small_base = (uint32_t)old;
+            cls[0] = (uint32_t)(old >> 32);
+        } else if (threadIdx.x < (uint32_t)kSortClasses) {
+            const uint32_t t = cls[threadIdx.x];
+            cls[threadIdx.x] = t ? atomicAdd(lists.counts + 1 + threadIdx.x, t) : 0u;
         }
         __syncthreads();
-        ps += list_base[0];
-        pl += list_base[1];
+        ps += small_base;
 #pragma unroll
         for (int k = 0; k < 16; ++k) {
             if (v[k] >= 2u && v[k] <= kSortSmallCells) {
@@ -761,9 +777,9 @@ __global__ __launch_bounds__(256) void k_scan_apply(const uint32_t* __restrict__
                     lists.small[ps] = i0 + (uint32_t)k;
                 ++ps;
             } else if (v[k] > kSortSmallCells) {
-                if (pl < lists.large_cap)
-                    lists.large[pl] = i0 + (uint32_t)k;
-                ++pl;
+                const uint32_t q = sort_class(v[k]), at = atomicAdd(cls + q, 1u);
+                if (at < lists.large_cap)
+                    lists.cls[(size_t)q * lists.large_cap + at] = i0 + (uint32_t)k;
             }
         }
     }
@@ -889,141 +905,66 @@ __global__ __launch_bounds__(256) void k_compact_write(uint32_t n, uint32_t img_
 // ---------------------------------------------------------------------------
 // 5. Per-cell sort
 // ---------------------------------------------------------------------------
-// Cells of 2..kSortSmallCells references (lists.small), one thread per cell.
-__global__ __launch_bounds__(256) void k_sort_small(const DevFrame* __restrict__ fr,
-                                                    const uint32_t* __restrict__ offsets,
-                                                    uint32_t* __restrict__ refs, SortLists lists)
-{
-    if (fr->status & (kStatusFrameInvalid | kStatusCellsOver | kStatusRefsOver))
-        return;
-    uint32_t nl = lists.counts[0];
-    nl = nl < lists.small_cap ? nl : lists.small_cap;
-    for (uint32_t li = blockIdx.x * blockDim.x + threadIdx.x; li < nl;
-         li += gridDim.x * blockDim.x)
-        sort_small_cell(offsets, refs, lists.small[li]);
-}
-
-
-
-// Split lists.large by size class (see SortLists).  The waves of a block
-// reserve their runs in an LDS count per class, and the block then takes one
-// global atomic per class it holds: many blocks adding to the same few
-// counters serialise, so the fewer such atomics the better.
-__global__ __launch_bounds__(256) void k_sort_classify(const DevFrame* __restrict__ fr,
-                                                       const uint32_t* __restrict__ offsets,
-                                                       SortLists lists)
-{
-    __shared__ uint32_t block_cnt[kSortClasses];
-    __shared__ uint32_t block_base[kSortClasses];
-    if (fr->status & (kStatusFrameInvalid | kStatusCellsOver | kStatusRefsOver))
-        return;
-    uint32_t cnt = lists.counts[1];
-    cnt = cnt < lists.large_cap ? cnt : lists.large_cap;
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t stride = gridDim.x * blockDim.x;
-    // the loop runs over whole blocks (li0 is the block's first entry), so
-    // every thread takes part in the ballots and barriers
-    for (uint32_t li0 = blockIdx.x * blockDim.x; li0 < cnt; li0 += stride) {
-        const uint32_t li = li0 + threadIdx.x;
-        int cls = -1;
-        uint32_t c = 0;
-        if (li < cnt) {
-            c = lists.large[li];
-            const uint32_t n = offsets[c + 1] - offsets[c];
-            cls = n <= 64u ? 0 : n <= 256u ? 1 : n <= 1024u ? 2 : n <= kSortWaveMax ? 3 : 4;
-        }
-        if (threadIdx.x < (uint32_t)kSortClasses)
-            block_cnt[threadIdx.x] = 0u;
-        __syncthreads();
-        uint32_t at = 0;
-        uint64_t mine = 0;
-#pragma unroll
-        for (int q = 0; q < kSortClasses; ++q) {
-            const uint64_t m = __ballot(cls == q);
-            if (m == 0)
-                continue;
-            const uint32_t leader = (uint32_t)__builtin_ctzll(m);
-            uint32_t w = 0;
-            if (lane == leader)
-                w = atomicAdd(block_cnt + q, (uint32_t)__popcll(m));
-            w = (uint32_t)__builtin_amdgcn_readlane((int)w, (int)leader);
-            if (cls == q) {
-                at = w;
-                mine = m;
-            }
-        }
-        __syncthreads();
-        if (threadIdx.x < (uint32_t)kSortClasses) {
-            const uint32_t k = block_cnt[threadIdx.x];
-            block_base[threadIdx.x] = k ? atomicAdd(lists.counts + 2 + threadIdx.x, k) : 0u;
-        }
-        __syncthreads();
-        if (cls >= 0)
-            lists.cls[(size_t)cls * lists.large_cap + block_base[cls] + at + lanes_below(mine)] = c;
-    }
-}
-
-// Cells of size class Q (E = 4^Q: 16E < n <= 64E references), one wave each.
+// Cells of one size class, a wave each, from wave `wave` of `waves`: class Q
+// (E = 4^Q) holds 16E < n <= 64E references.
 template <int E, int Q>
-__global__ __launch_bounds__(256) void k_sort_wave(const DevFrame* __restrict__ fr,
-                                                   const uint32_t* __restrict__ offsets,
-                                                   uint32_t* __restrict__ refs, SortLists lists)
+__device__ __forceinline__ void sort_wave_class(const uint32_t* __restrict__ offsets,
+                                                uint32_t* __restrict__ refs,
+                                                const SortLists& lists, uint32_t wave,
+                                                uint32_t waves)
 {
-    if (fr->status & (kStatusFrameInvalid | kStatusCellsOver | kStatusRefsOver))
-        return;
-    uint32_t cnt = lists.counts[2 + Q];
+    uint32_t cnt = lists.counts[1 + Q];
     cnt = cnt < lists.large_cap ? cnt : lists.large_cap;
     const uint32_t* __restrict__ list = lists.cls + (size_t)Q * lists.large_cap;
-    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const uint32_t n_waves = (gridDim.x * blockDim.x) >> 6;
-    for (uint32_t li = wave; li < cnt; li += n_waves) {
+    for (uint32_t li = wave; li < cnt; li += waves) {
         const uint32_t c = list[li];
         const uint32_t b = offsets[c];
         wave_sort<E>(refs + b, offsets[c + 1] - b);
     }
 }
 
-// Cells of 1025..kSortWaveMax references (size class 3), one 256-thread
-// block each: four register-sorted runs merged through LDS.
-__global__ __launch_bounds__(256) void k_sort_block(const DevFrame* __restrict__ fr,
-                                                    const uint32_t* __restrict__ offsets,
-                                                    uint32_t* __restrict__ refs, SortLists lists)
+// Every listed cell in one launch.  The classes are independent, and a launch
+// for each left the GPU to a few long blocks or waves at a time: the first
+// blocks (up to half of them) take the cells of more than 1024 references, the
+// longest class first, a block each; the others the wave classes and then the
+// small cells, a thread each.  64 KB of LDS: two blocks of 16 waves a CU.
+__global__ __launch_bounds__(1024, 8) void k_sort_cells(const DevFrame* __restrict__ fr,
+                                                        const uint32_t* __restrict__ offsets,
+                                                        uint32_t* __restrict__ refs,
+                                                        SortLists lists)
 {
-    __shared__ uint32_t lds[2 * kSortWaveMax];
+    __shared__ uint32_t lds[kSortTile];
     if (fr->status & (kStatusFrameInvalid | kStatusCellsOver | kStatusRefsOver))
         return;
-    uint32_t cnt = lists.counts[2 + 3];
-    cnt = cnt < lists.large_cap ? cnt : lists.large_cap;
-    const uint32_t* __restrict__ list = lists.cls + (size_t)3 * lists.large_cap;
-    for (uint32_t li = blockIdx.x; li < cnt; li += gridDim.x) {
-        const uint32_t c = list[li];
-        const uint32_t b = offsets[c];
-        block_merge_sort<256>(refs + b, offsets[c + 1] - b, lds, lds + kSortWaveMax);
-    }
-}
-
-// Cells of more than kSortWaveMax references (size class 4), one 1024-thread
-// block each: up to kSortTile by sixteen register-sorted runs merged through
-// LDS, longer ones by the tiled bitonic sort.
-__global__ __launch_bounds__(1024) void k_sort_large(const DevFrame* __restrict__ fr,
-                                                     const uint32_t* __restrict__ offsets,
-                                                     uint32_t* __restrict__ refs, SortLists lists)
-{
-    __shared__ uint32_t lds[2 * kSortTile];
-    if (fr->status & (kStatusFrameInvalid | kStatusCellsOver | kStatusRefsOver))
+    uint32_t c3 = lists.counts[1 + 3], c4 = lists.counts[1 + 4];
+    c3 = c3 < lists.large_cap ? c3 : lists.large_cap;
+    c4 = c4 < lists.large_cap ? c4 : lists.large_cap;
+    const uint32_t heavy = c3 + c4, half = gridDim.x / 2u;
+    const uint32_t hb = heavy < half ? heavy : half;   // blocks for the long cells
+    if (blockIdx.x < hb) {
+        for (uint32_t li = blockIdx.x; li < heavy; li += hb) {
+            const uint32_t c = li < c4 ? lists.cls[(size_t)4 * lists.large_cap + li]
+                                       : lists.cls[(size_t)3 * lists.large_cap + (li - c4)];
+            const uint32_t b = offsets[c];
+            const uint32_t n = offsets[c + 1] - b;
+            if (n <= kSortTile / 2)
+                block_merge_sort<1024>(refs + b, n, lds, lds + kSortTile / 2);
+            else if (n <= kSortTile)
+                block_merge_sort<1024>(refs + b, n, lds, refs + b);
+            else
+                block_sort_cell(refs + b, n, lds);
+        }
         return;
-    uint32_t cnt = lists.counts[2 + 4];
-    cnt = cnt < lists.large_cap ? cnt : lists.large_cap;
-    const uint32_t* __restrict__ list = lists.cls + (size_t)4 * lists.large_cap;
-    for (uint32_t li = blockIdx.x; li < cnt; li += gridDim.x) {
-        const uint32_t c = list[li];
-        const uint32_t b = offsets[c];
-        const uint32_t n = offsets[c + 1] - b;
-        if (n <= kSortTile)
-            block_merge_sort<1024>(refs + b, n, lds, lds + kSortTile);
-        else
-            block_sort_cell(refs + b, n, lds);
     }
+    const uint32_t first = blockIdx.x - hb, blocks = gridDim.x - hb;
+    const uint32_t wave = first * 16u + (threadIdx.x >> 6), waves = blocks * 16u;
+    sort_wave_class<16, 2>(offsets, refs, lists, wave, waves);
+    sort_wave_class<4, 1>(offsets, refs, lists, wave, waves);
+    sort_wave_class<1, 0>(offsets, refs, lists, wave, waves);
+    uint32_t cnt = lists.counts[0];
+    cnt = cnt < lists.small_cap ? cnt : lists.small_cap;
+    for (uint32_t li = first * 1024u + threadIdx.x; li < cnt; li += blocks * 1024u)
+        sort_small_cell(offsets, refs, lists.small[li]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1173,13 +1114,13 @@ hipError_t launch_frame_from_box(const float bmin[3], const float bmax[3], uint3
 }
 
 hipError_t launch_grid_count(const DevFrame* fr, const float* verts, uint32_t n_tris,
-                             uint32_t* counts, uint32_t* big_list, uint32_t* big_count,
+                             uint32_t* counts, uint32_t* big_list, uint32_t* counters,
                              uint32_t* tile_sums, uint32_t cells_cap, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_zero_build_counters, dim3(1), dim3(64), 0, s, big_count);
+    uint32_t* big_count = counters;
     const uint32_t nb = grid_for(cells_cap, kScanTile);
-    hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(nb, 256, 1024)), dim3(256), 0, s, tile_sums, 0u,
-                       (uint64_t)nb);
+    hipLaunchKernelGGL(k_build_clear, dim3(grid_for(nb, 256, 1024)), dim3(256), 0, s, counters,
+                       tile_sums, nb);
     hipLaunchKernelGGL(k_grid_pass<false>, dim3(grid_for(n_tris, 256)), dim3(256), 0, s, fr, verts,
                        n_tris, counts, (const uint32_t*)nullptr, (uint32_t*)nullptr, big_list,
                        big_count, tile_sums);
@@ -1197,9 +1138,6 @@ hipError_t launch_grid_scan(DevFrame* fr, uint32_t* counts, uint32_t* offsets,
                             const SortLists& lists, bool prefixes_ready, hipStream_t s)
 {
     const uint32_t nb = grid_for(cells_cap, kScanTile);
-    if (lists.small)
-        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, lists.counts, 0u,
-                           (uint64_t)(2 + kSortClasses));
     // block_sums holds the count pass's tile sums: scan them into tile
     // offsets (in place), unless an earlier scan of the same counts did.
     if (!prefixes_ready)
@@ -1260,13 +1198,10 @@ hipError_t launch_grid_scatter(const DevFrame* fr, const float* verts, uint32_t 
 hipError_t launch_grid_sort(const DevFrame* fr, const uint32_t* offsets, uint32_t* refs,
                             const SortLists& lists, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_sort_small, dim3(2048), dim3(256), 0, s, fr, offsets, refs, lists);
-    hipLaunchKernelGGL(k_sort_classify, dim3(512), dim3(256), 0, s, fr, offsets, lists);
-    hipLaunchKernelGGL((k_sort_wave<1, 0>), dim3(2048), dim3(256), 0, s, fr, offsets, refs, lists);
-    hipLaunchKernelGGL((k_sort_wave<4, 1>), dim3(2048), dim3(256), 0, s, fr, offsets, refs, lists);
-    hipLaunchKernelGGL((k_sort_wave<16, 2>), dim3(1024), dim3(256), 0, s, fr, offsets, refs, lists);
-    hipLaunchKernelGGL(k_sort_block, dim3(1024), dim3(256), 0, s, fr, offsets, refs, lists);
-    hipLaunchKernelGGL(k_sort_large, dim3(256), dim3(1024), 0, s, fr, offsets, refs, lists);
+    // a block per 2048 references, up to twice what the GPU holds
+    const uint32_t refs_cap = 2u * lists.small_cap, g = refs_cap / 2048u;
+    hipLaunchKernelGGL(k_sort_cells, dim3(g < 32u ? 32u : g < 1024u ? g : 1024u), dim3(1024), 0, s,
+                       fr, offsets, refs, lists);
     return hipGetLastError();
 }
 

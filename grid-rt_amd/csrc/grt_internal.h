@@ -88,7 +88,7 @@ struct grt_scene_t {
     hipEvent_t xf_copied = nullptr;   // recorded after each copy out of xf_host
     bool xf_pending = false;
     // Grid.
-    grt::DevMem frame, partial, counts, offsets, refs, block_sums, big_list, sort_list,
+    grt::DevMem frame, partial, counts, offsets, refs, block_sums, big_list,
         sort_list_small, sort_classes, small_counters, trir;
     uint32_t cells_cap = 0, refs_cap = 0, list_cap = 0;
     // Second grid level: sub-grids of the dense top cells (g2_lambda = 0: off).
@@ -108,7 +108,7 @@ struct grt_scene_t {
     {
         return {&verts,  &normals,    &rest_verts, &rest_normals, &tri,       &xf,
                 &frame,  &partial,    &counts,     &offsets,      &refs,      &block_sums,
-                &big_list, &sort_list, &sort_list_small, &sort_classes, &small_counters,
+                &big_list, &sort_list_small, &sort_classes, &small_counters,
                 &trir, &g2frame, &g2tab, &cellrec, &g2skip, &g2tiles, &g2dense, &g2box, &g2big, &g2long,
                 &sub_offsets, &sub_refs, &sub_trir};
     }

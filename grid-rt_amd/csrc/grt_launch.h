@@ -22,25 +22,29 @@ hipError_t launch_frame_from_verts(const float* verts, uint32_t n_tris, float la
 hipError_t launch_frame_from_box(const float bmin[3], const float bmax[3], uint32_t n_tris,
                                  float lambda, uint32_t cells_cap, DevFrame* fr, hipStream_t s);
 
+// Words of a build's counters: [0] medium and [3] huge triangles of the count
+// pass, [4 ..] the lengths of the sort lists.
+constexpr uint32_t kBuildCounters = 16;
+constexpr uint32_t kSortCounters = 4;
+
 // Count pass: per-cell counts (atomics), per-scan-tile sums into tile_sums
-// (zeroed first; ceil(cells_cap/kScanTile) entries) and the lists of triangles spanning
+// (ceil(cells_cap/kScanTile) entries) and the lists of triangles spanning
 // more than 16 cells (medium: from the front of big_list, count in
-// big_count[0]; huge, over 65536 cells: from the back, count in big_count[3]).
-// big_list holds n_tris entries; counts must be zero on entry.
+// counters[0]; huge, over 65536 cells: from the back, count in counters[3]).
+// Clears the counters and tile_sums first.  big_list holds n_tris entries;
+// counts must be zero on entry.
 hipError_t launch_grid_count(const DevFrame* fr, const float* verts, uint32_t n_tris,
-                             uint32_t* counts, uint32_t* big_list, uint32_t* big_count,
+                             uint32_t* counts, uint32_t* big_list, uint32_t* counters,
                              uint32_t* tile_sums, uint32_t cells_cap, hipStream_t s);
 // Cells the per-cell sort has to visit, collected by the scan: `small` holds
-// the cells of 2..kSortSmallCells references, `large` the larger ones;
-// counts[0], counts[1] their lengths (zeroed by launch_grid_scan; counts is
-// 8-byte aligned, the scan adds to both with one 64-bit atomic).
-// `cls` (large_cap entries per class) receives the large list split by size
-// for the sort kernels: (16,64], (64,256], (256,1024], (1024,4096], larger;
-// counts[2..6] their lengths.
+// the cells of 2..kSortSmallCells references, `cls` (large_cap entries per
+// class) the larger ones by size: (16,64], (64,256], (256,1024], (1024,4096],
+// larger.  counts[0] is the length of `small`, counts[1..5] those of the
+// classes (cleared by launch_grid_count; 8-byte aligned, the scan adds to the
+// first two with one 64-bit atomic).
 constexpr int kSortClasses = 5;
 struct SortLists {
     uint32_t* small;
-    uint32_t* large;
     uint32_t* counts;
     uint32_t small_cap;
     uint32_t large_cap;
