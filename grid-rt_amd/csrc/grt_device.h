@@ -68,8 +68,12 @@ __device__ __forceinline__ float spec_cbrtf(float xf)
     m = ldexp(m, r);
     double y = 1.0;
 #pragma unroll 1
-    for (int i = 0; i < 8; ++i)
-        y = (2.0 * y + m / (y * y)) / 3.0;
+    for (int i = 0; i < 8; ++i) {
+        const double z = (2.0 * y + m / (y * y)) / 3.0;
+        if (z == y)
+            break;   // a fixed point: the remaining steps change nothing
+        y = z;
+    }
     return (float)ldexp(y, q);
 }
 

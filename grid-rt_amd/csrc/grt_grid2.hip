@@ -14,7 +14,7 @@
 //
 // Work layout: the plan of every top cell comes from 4096-cell tiles (16
 // consecutive cells per thread); the dense cells -- few, and clustered where
-// the scene is -- then get one 1024-thread block each, one reference per
+// the scene is -- then get one 256-thread block each, one reference per
 // thread: the count pass adds to LDS counters over the reference's sub-cell
 // box (and keeps the box, 4 bits per bound, at the reference's position), the
 // fill pass scatters through LDS cursors, and every sub-cell's ids are then
@@ -203,10 +203,15 @@ __global__ __launch_bounds__(256) void k_g2_skip_line(G2Build b)
 // record stores are coalesced; in-tile positions come from a wave scan per slot
 // (sub-cells in bits 0..23, the dense flag in bits 24..31: a wave's sums stay
 // below 2^18 and 64) and a scan of the 64 (slot, wave) totals in slot-major
-// order.
+// order.  The cells dense enough for a plan are collected in LDS and planned by
+// all threads together: a plan is a cube root in binary64, which every wave
+// with such a cell paid for on each of its slots.
 template <bool LIST>
 __global__ __launch_bounds__(256) void k_g2_plan(G2Build b)
 {
+    __shared__ uint32_t s_plan[kScanTile];   // of the listed cells: references, then the plan
+    __shared__ uint16_t s_list[kScanTile];
+    __shared__ uint32_t s_listed;
     __shared__ uint32_t s_tot[2][64];
     __shared__ uint32_t s_scan[8];
     __shared__ uint64_t s_occ[kScanTile / 64u + 2u];   // occupancy, 64 cells either side
@@ -224,21 +229,34 @@ __global__ __launch_bounds__(256) void k_g2_plan(G2Build b)
     }
     const bool sub_ok = !LIST || b.g2->status == 0;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    uint32_t packed[16], ms[16], nd = 0, msum = 0, empty = 0;
+    uint32_t nd = 0, msum = 0, empty = 0, dense = 0;
+    if (threadIdx.x == 0)
+        s_listed = 0u;
+    __syncthreads();
 #pragma unroll
     for (uint32_t k = 0; k < 16; ++k) {
-        const uint32_t c = base + 256u * k + threadIdx.x;
+        const uint32_t i = 256u * k + threadIdx.x, c = base + i;
         const uint32_t n = c < m_top ? b.offsets[c + 1] - b.offsets[c] : 0u;
-        ms[k] = 0;
-        packed[k] = sub_ok ? g2_plan(fr, n, b.lambda2, b.min_refs, ms[k]) : 0u;
         empty |= (c < m_top && n == 0u ? 1u : 0u) << k;
-        nd += packed[k] ? 1u : 0u;
-        msum += ms[k];
+        if (sub_ok && n != 0u && n >= b.min_refs) {
+            dense |= 1u << k;
+            s_plan[i] = n;
+            s_list[atomicAdd(&s_listed, 1u)] = (uint16_t)i;
+        }
         if (!LIST) {
             const uint64_t w = __ballot(n != 0u);   // cells base + 64 (4 k + wave) ...
             if (lane == 0u)
                 s_occ[1u + 4u * k + wave] = w;
         }
+    }
+    __syncthreads();
+    for (uint32_t j = threadIdx.x; j < s_listed; j += 256u) {
+        const uint32_t i = s_list[j];
+        uint32_t m;
+        const uint32_t p = g2_plan(fr, s_plan[i], b.lambda2, b.min_refs, m);
+        s_plan[i] = p;
+        nd += p ? 1u : 0u;
+        msum += m;
     }
     if (!LIST) {
         // D_x of the tile's cells: the occupancy of 64 cells either side too
@@ -270,10 +288,13 @@ __global__ __launch_bounds__(256) void k_g2_plan(G2Build b)
         }
         return;
     }
-    // ms[k] becomes the exclusive prefix within (slot k, this wave)
-    uint32_t ed[16];
+    __syncthreads();
+    // ms[k]: the exclusive prefix of the sub-cells within (slot k, this wave)
+    uint32_t packed[16], ms[16], ed[16];
 #pragma unroll
     for (uint32_t k = 0; k < 16; ++k) {
+        packed[k] = (dense >> k) & 1u ? s_plan[256u * k + threadIdx.x] : 0u;
+        ms[k] = (packed[k] & 255u) * ((packed[k] >> 8) & 255u) * ((packed[k] >> 16) & 255u);
         const uint32_t v = ms[k] | ((packed[k] ? 1u : 0u) << 24);
         const uint32_t inc = wave_incl_scan(v);
         const uint32_t ex = inc - v;
@@ -365,20 +386,24 @@ __global__ __launch_bounds__(1024) void k_g2_scan_tiles(G2Build b, uint32_t n_ti
 
 // Frame of dense cell c's sub-grid.
 struct G2Cell {
-    uint32_t kb, ke, pk, m;
+    uint32_t kb, ke, sub, m;   // references, first sub-cell, sub-cells
     uint32_t r[3];
     float sb[3], si[3];
 };
 
+// (from its record, which the plan's second pass wrote: planning it again costs
+// a cube root in binary64 per block)
 __device__ __forceinline__ void g2_cell(const G2Build& b, uint32_t c, G2Cell& g)
 {
     const DevFrame* fr = b.fr;
+    const uint2 rec = b.cellrec[c];
     g.kb = b.offsets[c];
     g.ke = b.offsets[c + 1];
-    g.pk = g2_plan(fr, g.ke - g.kb, b.lambda2, b.min_refs, g.m);
-    g.r[0] = g.pk & 255u;
-    g.r[1] = (g.pk >> 8) & 255u;
-    g.r[2] = (g.pk >> 16) & 255u;
+    g.sub = rec.x & 0x7fffffffu;
+    g.r[0] = rec.y & 255u;
+    g.r[1] = (rec.y >> 8) & 255u;
+    g.r[2] = (rec.y >> 16) & 255u;
+    g.m = g.r[0] * g.r[1] * g.r[2];
     const uint32_t nx = (uint32_t)fr->n[0], ny = (uint32_t)fr->n[1];
     const uint32_t cc[3] = {c % nx, (c / nx) % ny, c / (nx * ny)};
     for (int a = 0; a < 3; ++a) {
@@ -414,10 +439,16 @@ __device__ __forceinline__ uint32_t g2_box(const float* __restrict__ verts, uint
 // into b.box (at its top-reference position), the sub-cell counts into the
 // cell's sub_offsets slots (when present) and the cell's sub-reference total
 // into dense_refs.  References go one per thread with LDS atomic counters.
-__global__ __launch_bounds__(1024) void k_g2_count(G2Build b)
+//
+// A cell's block is a chain of dependent loads (its record, references,
+// vertices), so four of them share a CU (stadium preview frame, us: 1268 / 1210
+// / 1194 / 1215 with 128 / 256 / 512 / 1024 threads).
+constexpr uint32_t kG2Block = 512;
+
+__global__ __launch_bounds__(kG2Block) void k_g2_count(G2Build b)
 {
     __shared__ uint32_t s_cnt[kSubMax * kSubMax * kSubMax];
-    __shared__ uint32_t s_scan[17];
+    __shared__ uint32_t s_scan[kG2Block / 64 + 1];
     if (!top_ok(b.fr) || (b.g2->status & ~kStatusRefsOver) != 0)
         return;
     const uint32_t nd = (uint32_t)b.g2->n[0];
@@ -430,7 +461,7 @@ __global__ __launch_bounds__(1024) void k_g2_count(G2Build b)
         __syncthreads();
         const uint32_t r0 = g.r[0], r01 = g.r[0] * g.r[1];
         uint32_t tot = 0;
-        for (uint32_t k = g.kb + threadIdx.x; k < g.ke; k += blockDim.x) {
+        for (uint32_t k = g.kb + threadIdx.x; k < g.ke; k += kG2Block) {
             const uint32_t p = g2_box(b.verts, b.refs[k], g);
             b.box[k] = p;
             const uint32_t xlo = p & 15u, xhi = (p >> 4) & 15u;
@@ -443,11 +474,11 @@ __global__ __launch_bounds__(1024) void k_g2_count(G2Build b)
                         atomicAdd(s_cnt + z * r01 + y * r0 + x, 1u);
         }
         uint32_t cell_total;
-        block_excl_scan<1024>(tot, s_scan, cell_total);   // barrier: counts complete
+        block_excl_scan<kG2Block>(tot, s_scan, cell_total);   // barrier: counts complete
         if (threadIdx.x == 0)
             b.dense_refs[d] = cell_total;
         if (b.sub_offsets) {
-            uint32_t* out = b.sub_offsets + (b.cellrec[c].x & 0x7fffffffu);
+            uint32_t* out = b.sub_offsets + g.sub;
             for (uint32_t s = threadIdx.x; s < g.m; s += blockDim.x)
                 out[s] = s_cnt[s];
         }
@@ -471,8 +502,7 @@ __global__ __launch_bounds__(1024) void k_g2_fill(G2Build b)
         const uint32_t c = b.dense[d];
         G2Cell g;
         g2_cell(b, c, g);
-        const uint32_t sub_base = b.cellrec[c].x & 0x7fffffffu;
-        uint32_t* out = b.sub_offsets + sub_base;
+        uint32_t* out = b.sub_offsets + g.sub;
         // offsets: 4 consecutive sub-cells per thread (m <= 4096)
         const uint32_t s0 = 4u * threadIdx.x;
         uint32_t v[4], sum = 0;
@@ -647,8 +677,8 @@ hipError_t launch_grid2_skip_records(const G2Build& b, uint32_t top_cells_cap, h
 hipError_t launch_grid2_plan_refs(const G2Build& b, uint32_t sub_refs_cap, uint32_t dense_cap,
                                   hipStream_t s)
 {
-    const uint32_t nb = dense_cap < 2048u ? (dense_cap ? dense_cap : 1u) : 2048u;
-    hipLaunchKernelGGL(k_g2_count, dim3(nb), dim3(1024), 0, s, b);
+    const uint32_t nb = dense_cap < 4096u ? (dense_cap ? dense_cap : 1u) : 4096u;
+    hipLaunchKernelGGL(k_g2_count, dim3(nb), dim3(kG2Block), 0, s, b);
     hipLaunchKernelGGL(k_g2_scan_dense, dim3(1), dim3(1024), 0, s, b, sub_refs_cap);
     return hipGetLastError();
 }
