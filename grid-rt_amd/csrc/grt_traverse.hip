@@ -189,20 +189,49 @@ __device__ __forceinline__ void trace_window(const DevFrame* __restrict__ fr,
                                              uint32_t i, bool valid, WaveWin& W)
 {
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t j = lane & (lanes - 1u), owner = lane - j;
-    const uint32_t c = lanes * S <= 16u ? (uint32_t)S : 16u / lanes, cell0 = j * c;
     float4 ro = make_float4(0.0f, 0.0f, 0.0f, 0.0f), rd = ro;
     DdaW w = {};
-    bool walk = false;   // the lane stands on a cell of its ray
-    if (valid) {
-        ro = make_float4(rays.ox[i], rays.oy[i], rays.oz[i], rays.tmin[i]);
-        rd = make_float4(rays.dx[i], rays.dy[i], rays.dz[i], rays.tmax[i]);
-        Dda s;
-        walk = grid_ok(fr) && dda_setup(fr, ro.x, ro.y, ro.z, rd.x, rd.y, rd.z, ro.w, rd.w, s);
-        if (walk)
-            w = dda_window(fr, s);
+    bool walk;   // the lane stands on a cell of its ray
+    bool open;   // the ray's result is not written yet
+    const auto write_miss = [&]() {
+        if (ANY) {
+            occluded[i] = 0;
+        } else {
+            hits.id[i] = -1;
+            hits.t[i] = INFINITY;
+            hits.u[i] = 0.0f;
+            hits.v[i] = 0.0f;
+        }
+    };
+    for (bool again = false;; again = true) {
+        walk = false;
+        open = valid;
+        if (valid) {
+            ro = make_float4(rays.ox[i], rays.oy[i], rays.oz[i], rays.tmin[i]);
+            rd = make_float4(rays.dx[i], rays.dy[i], rays.dz[i], rays.tmax[i]);
+            Dda s;
+            walk = grid_ok(fr) && dda_setup(fr, ro.x, ro.y, ro.z, rd.x, rd.y, rd.z, ro.w, rd.w, s);
+            if (walk)
+                w = dda_window(fr, s);
+        }
+        // Few rays to walk: the misses are written, the others share the wave.
+        const bool head = (lane & (lanes - 1u)) == 0;
+        const uint64_t heads = __ballot(walk && head);
+        const uint32_t more = win_lanes((uint32_t)__popcll(heads), lanes, 16u / (uint32_t)S);
+        if (again || heads == 0 || more == lanes)
+            break;
+        if (valid && !walk && head) {
+            write_miss();
+            if (COUNT) {
+                counters[2ull * i] = 0u;
+                counters[2ull * i + 1] = 0u;
+            }
+        }
+        lanes = (uint32_t)__builtin_amdgcn_readfirstlane((int)more);
+        valid = win_regroup(W, heads, lanes, i);
     }
-    bool open = valid;   // the ray's result is not written yet
+    const uint32_t j = lane & (lanes - 1u), owner = lane - j;
+    const uint32_t c = lanes * S <= 16u ? (uint32_t)S : 16u / lanes, cell0 = j * c;
     uint32_t cells = 0, tests = 0;
     if (__ballot(walk) != 0) {
         W.ro[lane] = make_float4(ro.x, ro.y, ro.z, win_lo(ro.w));
@@ -284,16 +313,8 @@ __device__ __forceinline__ void trace_window(const DevFrame* __restrict__ fr,
             counters[2ull * i + 1] = st;
         }
     }
-    if (open && j == 0) {
-        if (ANY) {
-            occluded[i] = 0;
-        } else {
-            hits.id[i] = -1;
-            hits.t[i] = INFINITY;
-            hits.u[i] = 0.0f;
-            hits.v[i] = 0.0f;
-        }
-    }
+    if (open && j == 0)
+        write_miss();
 }
 
 extern __shared__ WaveWin win_lds[];   // one per wave of the block
@@ -577,11 +598,9 @@ __global__ __launch_bounds__(128) void k_trace2_window(TraceArgs a, RaySoA rays,
     stage_sub_tab(a, tab);
     WaveWin& W = win_lds[threadIdx.x >> 6];
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t j = lane & (lanes - 1u), owner = lane - j, cell0 = j * (uint32_t)S;
-    const uint32_t units = lanes * (uint32_t)S;
     bool valid;
-    const uint32_t i = trace_ray(
-        a, (blockIdx.x * blockDim.x + threadIdx.x) >> __builtin_ctz(lanes), valid);
+    uint32_t i = trace_ray(a, (blockIdx.x * blockDim.x + threadIdx.x) >> __builtin_ctz(lanes),
+                           valid);
     const DevFrame* __restrict__ fr = a.fr;
     const uint32_t nx = (uint32_t)fr->n[0], ny = (uint32_t)fr->n[1];
     // Over its capacity the second level's records are not complete: the top
@@ -591,8 +610,39 @@ __global__ __launch_bounds__(128) void k_trace2_window(TraceArgs a, RaySoA rays,
     Dda s = {};
     float t_enter = 0.0f;
     uint2 rec = make_uint2(0u, 0u);
-    bool top = valid && ray2_setup(fr, rays, i, r, s, t_enter);   // an item of the top walk is next
-    bool open = valid;                                            // the result is not written yet
+    bool top;    // an item of the top walk is next
+    bool open;   // the result is not written yet
+    const auto write_miss = [&]() {
+        if (ANY) {
+            occluded[i] = 0;
+        } else {
+            hits.id[i] = -1;
+            hits.t[i] = INFINITY;
+            hits.u[i] = 0.0f;
+            hits.v[i] = 0.0f;
+        }
+    };
+    for (bool again = false;; again = true) {
+        top = valid && ray2_setup(fr, rays, i, r, s, t_enter);
+        open = valid;
+        // Few rays to walk: the misses are written, the others share the wave.
+        const bool head = (lane & (lanes - 1u)) == 0;
+        const uint64_t heads = __ballot(top && head);
+        const uint32_t more = win_lanes((uint32_t)__popcll(heads), lanes, 16u / (uint32_t)S);
+        if (again || heads == 0 || more == lanes)
+            break;
+        if (valid && !top && head) {
+            write_miss();
+            if (COUNT) {
+                a.counters[2ull * i] = 0u;
+                a.counters[2ull * i + 1] = 0u;
+            }
+        }
+        lanes = (uint32_t)__builtin_amdgcn_readfirstlane((int)more);
+        valid = win_regroup(W, heads, lanes, i);
+    }
+    const uint32_t j = lane & (lanes - 1u), owner = lane - j, cell0 = j * (uint32_t)S;
+    const uint32_t units = lanes * (uint32_t)S;
     uint32_t cells = 0, tests = 0;
     if (__ballot(top) != 0) {
         W.ro[lane] = make_float4(r.o0, r.o1, r.o2, win_lo(r.tmin));
@@ -740,16 +790,8 @@ __global__ __launch_bounds__(128) void k_trace2_window(TraceArgs a, RaySoA rays,
             a.counters[2ull * i + 1] = st;
         }
     }
-    if (open && j == 0) {
-        if (ANY) {
-            occluded[i] = 0;
-        } else {
-            hits.id[i] = -1;
-            hits.t[i] = INFINITY;
-            hits.u[i] = 0.0f;
-            hits.v[i] = 0.0f;
-        }
-    }
+    if (open && j == 0)
+        write_miss();
 }
 
 template <bool ANY, bool COUNT>

@@ -92,3 +92,29 @@ def test_lanes_by_launch_size(gpu_ctx, n):
             c = cnt.cpu().numpy().view(np.uint32).reshape(n, 2)
             assert_same(c[:, 0], oa["cells"], "cells visited")
             assert_same(c[:, 1], oa["tests"], "triangle tests")
+
+
+# Waves with few rays to walk give them more lanes: every number of walking
+# rays per wave around the powers of two, first, last and scattered in it, on
+# one level and two.
+@pytest.mark.parametrize("two", [False, True])
+@pytest.mark.parametrize("n", [64 * 40 + 7, 1_000_003])
+def test_sparse_waves(gpu_ctx, two, n):
+    v = np.concatenate([_soup(300, 3, 0.6), _soup(400, 4, 0.02) * np.float32(0.1) +
+                        np.float32(0.45)])
+    sc = _built(gpu_ctx, v, np.zeros_like(v), 2.0, 4.0 if two else 0.0, 16)
+    rays = _random_rays(n, 11)
+    w, l = np.arange(n) // 64, np.arange(n) % 64
+    k = np.array([1, 2, 3, 4, 5, 8, 9, 15, 16, 17, 31, 32, 33, 63, 64, 0])[w % 16]
+    place = np.where(w // 16 % 3 == 0, l, np.where(w // 16 % 3 == 1, 63 - l, l * 37 % 64))
+    off = place >= k
+    rays["tmin"][off], rays["tmax"][off] = 1.0, -1.0
+    if two:
+        fr, offs, refs, g2 = check_levels(sc, v, 2.0, 4.0, 16)
+        check_trace2(sc, fr, offs, refs, g2, v, rays, one_level=False,
+                     modes=[("simple", 16), ("split", 2), ("split", 8)])
+        return
+    _, offs, refs = sc.download_grid()
+    fr = orc.grid_frame(v, 2.0)
+    check_closest(sc, fr, offs, refs, v, rays)
+    check_any(sc, fr, offs, refs, v, rays)
