@@ -111,10 +111,13 @@ def grid_tag(lam, sub):
 
 
 def kernel_name(closest, sched_char, two_level=False):
-    """The traversal kernel a stage launches (under every schedule; a two-level
-    grid is walked by its own kernel)."""
-    return "%s<%s, false>" % ("k_trace2_window" if two_level else "k_trace_window",
-                              "false" if closest else "true")
+    """The traversal kernel a stage launches, and its lanes per ray where the
+    schedule character fixes them (a two-level grid is walked by its own
+    kernel)."""
+    lanes = {"2": 2, "4": 4, "8": 8, "x": 16}.get(sched_char)
+    return "%s<%s, false>%s" % ("k_trace2_window" if two_level else "k_trace_window",
+                                "false" if closest else "true",
+                                " %d lanes" % lanes if lanes else "")
 
 
 class Frame:

@@ -5,10 +5,10 @@ that depend on the grid):
   lam     grid resolution factor (cells ~ lam * triangles; the reference fixed
           k = 6 in UniformGridAccStructBuilder.cpp:91 and exposed it in its GUI,
           WdgTransformEdit.cpp:49-69)
-  sched   per traversal stage, 's' one ray per lane, 'w' one ray per lane with
-          the wave's triangle tests pooled, 'p' persistent refill, or '2', '4',
-          '8' lanes per ray
-  refill  idle lanes that trigger a refill in the persistent schedule
+  sched   per traversal stage, 's', 'w' or 'p': lanes per ray chosen by the size
+          of the launch; '2', '4', '8' or 'x': 2, 4, 8 or 16 lanes per ray
+  refill  the parameter of grt_set_trace_mode under the first three (checked,
+          otherwise unused)
   block   threads per block of the traversal kernels
 
 The tuner measures candidates with a caller-supplied timing function and keeps

@@ -71,8 +71,7 @@ def serve_vs_plain(ctx: Context, scenes, n_requests: int = 120,
     torch.cuda.synchronize()
     closed = _requests(scenes, W.serve_requests(n_requests, 0.0, len(scenes)))
     # Each path runs with the traversal schedule that saturates it best (the
-    # batched path runs the split schedule as one ray per lane, so it tries
-    # the first two only).
+    # batched path tries the first two, with lanes per ray by its launches).
     modes = {"simple": 16, "pooled": 16, "split": 4}
     sat = {True: {}, False: {}}
     for mode, param in modes.items():
@@ -253,9 +252,8 @@ def _time(fn, reps, torch):
 
 def batch_config(reps: int = 5):
     """Batched (one launch per level, hipGraph) vs plain; the autotuner picks
-    the schedule (one ray per lane, pooled, persistent, or 2/4/8 lanes per ray,
-    i.e. 64/32/16/8 rays per wave), lambda in {2,5,8}, block size and refill
-    threshold.  The plain path gets its best of the single-scene schedules, the
+    the schedule (lanes per ray by the size of the launch, or 2/4/8 of them),
+    lambda in {2,5,8} and the block size.  The plain path gets its best of the single-scene schedules, the
     split one (4 lanes per ray) included."""
     torch = _torch()
     ctx = Context(0)
@@ -445,7 +443,7 @@ def kdtree_config(lam: float = 256.0, reps: int = 5, width: int = 1920, height: 
     rigid cluster transforms): the same four traversal stages -- primary,
     shadow, mirror bounce, bounce shadow, rays generated from the grid's hits --
     timed per launch (HIP events, median of `reps`) through the one-level grid
-    (best of one ray per lane, pooled tests and 2 / 16 lanes per ray), through
+    (best of the lanes per ray the launch chooses and 2 / 16), through
     the kd-tree and through the two-level grid, with the per-ray work of each
     (cells or leaves, triangle tests) and the build times (the grids' device
     rebuilds, the kd-tree's host build)."""

@@ -47,9 +47,8 @@ def check_levels(sc, v, lam, lam2, min_refs, tag=""):
     return fr, ooffs, orefs, (ocs, oso, osr)
 
 
-# Trace modes: one ray per lane (simple; pooled and persistent launch the same
-# kernel on a two-level grid), and 2, 8 and 16 lanes per ray walking the ray's
-# top items in turn (the split schedule).
+# Trace modes: lanes per ray by the size of the launch (simple; pooled and
+# persistent launch the same), and 2, 8 and 16 lanes per ray (split).
 MODES = [("simple", 16), ("pooled", 16), ("persistent", 16), ("split", 2), ("split", 8),
          ("split", 16)]
 
