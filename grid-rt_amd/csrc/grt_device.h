@@ -286,8 +286,8 @@ __device__ __forceinline__ void wave_sort(uint32_t* __restrict__ seg, uint32_t n
 // network), then runs are merged pairwise through LDS -- src and dst
 // ping-pong, n words each -- every thread writing 16 consecutive outputs from
 // its merge-path split (a binary search on the diagonal; ties take the left
-// run first).  dst may be seg itself when an even number of merges brings the
-// ids back to src (n over half of 1024 x the runs' power of two).  Run boundaries are multiples of 2048 and the outputs of a
+// run first).  dst may be seg itself for an even number of merges (n over 8192,
+// up to 16384: four), which end in src.  Run boundaries are multiples of 2048 and the outputs of a
 // thread start at a multiple of 16, so no thread's outputs straddle two
 // merges.
 template <int BLOCK>
