@@ -108,6 +108,8 @@ int grid_reserve_refs(grt_scene_t* sc, uint32_t refs)
 {
     if (refs <= sc->refs_cap && sc->refs.ptr)
         return GRT_OK;
+    if (refs > kRefsMax)
+        return set_error(GRT_CAPACITY, "grid of %u references is too large", refs);
     uint64_t cap = (uint64_t)refs + refs / 8 + 1024;
     if (cap > 0xfffffff0ull)
         cap = 0xfffffff0ull;
@@ -1013,6 +1015,8 @@ int grt_grid_upload(grt_scene sc, const grt_grid_info* info, const uint32_t* off
         return set_error(GRT_INVALID_PARAM, "grt_grid_upload: refs is NULL");
     if (offsets_host[0] != 0)
         return set_error(GRT_INVALID_PARAM, "grt_grid_upload: offsets[0] must be 0");
+    if (r > kRefsMax)
+        return set_error(GRT_CAPACITY, "grt_grid_upload: %u references are too many", r);
     for (uint64_t c = 0; c < m; ++c)
         if (offsets_host[c + 1] < offsets_host[c])
             return set_error(GRT_INVALID_PARAM, "grt_grid_upload: offsets not monotone at %llu",

@@ -11,6 +11,9 @@ namespace grt {
 // ---- grid build (grt_build.hip) --------------------------------------------
 constexpr uint32_t kScanTile = 4096;    // elements per scan block (256 threads x 16)
 constexpr uint32_t kBBoxMaxBlocks = 1024;
+// References of a grid, at most: its buffers hold up to 0xfffffff0, and the
+// wave's walk of one long list steps 128 records past its end in 32 bits.
+constexpr uint32_t kRefsMax = 0xffffff80u;
 constexpr uint32_t kSortSmallCells = 16;  // cells up to this size sort in one thread
 
 // Frame from the vertices: block partial boxes, then one block computes the

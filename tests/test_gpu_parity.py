@@ -212,6 +212,26 @@ def test_trace_edge(gpu_ctx, name):
     check_any(sc, fr, offs, refs, v, rays)
 
 
+def test_more_references_than_a_grid_holds(gpu_ctx, c1_scene):
+    """Refused before anything is allocated; the scene's grid stays."""
+    v, n = c1_scene
+    sc = grt.Scene(gpu_ctx)
+    sc.upload(v, n)
+    sc.build_grid(5.0)
+    before = gpu_ctx.memory_used()
+    for refs in (0xffffff81, 0xfffffff1, 0xffffffff):
+        with pytest.raises(grt.GrtError) as e:
+            sc.reserve_grid(64, refs)
+        assert e.value.code == grt.GRT_CAPACITY
+        with pytest.raises(grt.GrtError) as e:   # the offsets are checked first
+            sc.upload_grid(dict(orc.grid_frame(v, 1e-6), n=(1, 1, 1)), [0, refs],
+                           np.zeros(1, np.uint32))
+        assert e.value.code == grt.GRT_CAPACITY
+    assert gpu_ctx.memory_used() == before
+    sc.check_grid()
+    sc.close()
+
+
 @pytest.mark.parametrize("over", ["cells", "refs"])
 def test_rebuild_over_capacity_is_safe(gpu_ctx, c1_scene, over):
     """An asynchronous rebuild that outgrows the reserved grid (more cells, or
