@@ -1210,6 +1210,7 @@ static TraceArgs trace_args(grt_scene sc, uint32_t n, uint32_t image_width, uint
     a.image_width = image_width;
     a.counters = counters;
     a.flat = grid_flat(sc->info_host);
+    a.spans = sc->spans();
     if (sc->g2_built) {
         a.g2 = sc->g2frame.as<DevFrame>();
         a.cellrec = sc->cellrec.as<uint2>();

@@ -19,6 +19,7 @@ struct grt_batch_t {
     uint32_t max_items = 0;
     uint32_t n_items = 0;
     uint32_t total_slots = 0;
+    bool spans = false;   // an item's scene may hold lists of more than kWinSpan records
     DevMem tasks, map;
     BatchTask* staging = nullptr;   // pinned
     hipEvent_t staged = nullptr;    // staging may be reused once this completes
@@ -96,6 +97,7 @@ int grt_batch_set(grt_batch b, const grt_batch_item* items, uint32_t n_items)
         b->staged_pending = false;
     }
     uint64_t slots = 0;
+    bool spans = false;
     for (uint32_t i = 0; i < n_items; ++i) {
         const grt_batch_item& it = items[i];
         grt_scene_t* sc = it.scene;
@@ -128,6 +130,7 @@ int grt_batch_set(grt_batch b, const grt_batch_item* items, uint32_t n_items)
         t.slot_begin = (uint32_t)slots;
         t.slots = (uint32_t)s;
         t.any = it.any ? 1u : 0u;
+        spans |= sc->spans();
         slots += s;
         if (slots > 0xffffffc0ull)
             return set_error(GRT_CAPACITY, "grt_batch_set: more than 2^32 ray slots");
@@ -151,6 +154,7 @@ int grt_batch_set(grt_batch b, const grt_batch_item* items, uint32_t n_items)
         return hip_check(e, "grt_batch_set");
     b->n_items = n_items;
     b->total_slots = (uint32_t)slots;
+    b->spans = spans;
     return GRT_OK;
 }
 
@@ -160,7 +164,7 @@ int grt_batch_trace(grt_batch b)
         return set_error(GRT_INVALID_PARAM, "grt_batch_trace: NULL batch");
     grt_context_t* ctx = b->ctx;
     return hip_check(launch_trace_batch(b->tasks.as<BatchTask>(), b->map.as<uint32_t>(),
-                                        b->total_slots, window_lanes_of(ctx),
+                                        b->total_slots, b->spans, window_lanes_of(ctx),
                                         ctx->block_closest, ctx->stream),
                      "grt_batch_trace");
 }

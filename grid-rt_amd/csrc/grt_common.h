@@ -82,6 +82,10 @@ struct DevCamera {
 
 constexpr float kRayEpsilon = 2e-4f;                          // Context.cpp:505
 constexpr float kExitScale = 1.0f + 1.0f / 1048576.0f;        // cell-exit bound factor
+// Records of a list that a closest-hit key of the windowed walk counts
+// (win_key); longer lists, which only an uploaded grid can hold, are tested
+// span by span.
+constexpr uint32_t kWinSpan = 1u << 28;
 
 __device__ __forceinline__ float tmin_f(float a, float b) { return a < b ? a : b; }
 __device__ __forceinline__ float tmax_f(float a, float b) { return a > b ? a : b; }

@@ -99,6 +99,8 @@ struct grt_scene_t {
         sub_offsets, sub_refs, sub_trir;
     uint32_t g2_top_cap = 0, g2_box_cap = 0, g2_cells_cap = 0, g2_refs_cap = 0, g2_dense_cap = 0,
              g2_big_cap = 0, g2_long_cap = 0;
+    // (by capacity, so a captured launch stays right for every grid its buffers take)
+    bool spans() const { return refs_cap > grt::kWinSpan; }
     bool grid_valid = false;
     bool info_stale = false;
     float lambda = 0.0f;

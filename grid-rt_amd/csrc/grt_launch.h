@@ -161,6 +161,7 @@ struct TraceArgs {
     uint32_t image_width;   // 0: lane i traces ray i; else 8x8 pixel tiles per wave
     uint32_t* counters;     // NULL or 2 per ray {cells, tests}
     bool flat = false;      // grid_flat() of the top grid
+    bool spans = false;     // the buffers could hold a list of more than kWinSpan records
     const uint32_t* list = nullptr;        // or the rays to trace: slot s traces list[s] ...
     const uint32_t* list_count = nullptr;  // ... for s < *list_count (a device value) and s < n
     // Two-level grid (all set, or cellrec NULL for the top grid alone).  The
@@ -211,9 +212,9 @@ struct alignas(16) BatchTask {
 hipError_t launch_task_map(const BatchTask* tasks, uint32_t n_tasks, uint32_t* map,
                            hipStream_t s);
 // Multi-scene traversal over all tasks (mixed closest / any hit), each wave in
-// one task; lanes as for launch_trace_window.
+// one task; lanes as for launch_trace_window, spans as TraceArgs::spans of any item.
 hipError_t launch_trace_batch(const BatchTask* tasks, const uint32_t* map, uint32_t total_slots,
-                              uint32_t lanes, uint32_t block, hipStream_t s);
+                              bool spans, uint32_t lanes, uint32_t block, hipStream_t s);
 hipError_t launch_gen_primary(const DevCamera& cam, const RaySoAOut& out, hipStream_t s);
 hipError_t launch_gen_shadow(uint32_t n, const RaySoA& in, const HitSoAIn& hits,
                              const float* normals, float lx, float ly, float lz, float offset,

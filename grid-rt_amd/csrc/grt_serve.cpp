@@ -454,6 +454,7 @@ private:
             a.n = it.n;
             a.image_width = it.width;
             a.counters = nullptr;
+            a.spans = it.sc->spans();
             const hipError_t e = launch_trace_window(
                 a, it.rays.in(), it.hits.out(), it.occ, it.any, window_lanes_of(ctx_),
                 it.any ? ctx_->block_any : ctx_->block_closest, s);

@@ -63,8 +63,11 @@ __device__ __forceinline__ uint32_t win_t_bits(float t)
     return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
 
-// Keys: cell (4 bits), t (32), position in the list (28; a cell lists a
-// triangle at most once and a scene has at most 2^28).
+// Keys: cell (4 bits), t (32), position in the list (28).  A built grid lists
+// each of a scene's at most 2^28 triangles once per cell; an uploaded one may
+// repeat them, so a closest-hit position is modulo kWinSpan: a longer list is
+// tested span by span (SPANS), and the one-level walk finds the record again.
+// An any-hit key has no t: its position takes those bits too, for any length.
 __device__ __forceinline__ unsigned long long win_key(uint32_t cell, uint32_t tbits, uint32_t j)
 {
     return ((unsigned long long)cell << 60) | ((unsigned long long)tbits << 28) | j;
@@ -75,9 +78,15 @@ __device__ __forceinline__ uint32_t win_cell(unsigned long long key)
     return (uint32_t)(key >> 60);
 }
 
+__device__ __forceinline__ uint32_t win_t_bits(unsigned long long key)
+{
+    return (uint32_t)(key >> 28);
+}
+
+template <bool ANY>
 __device__ __forceinline__ uint32_t win_pos(unsigned long long key)
 {
-    return (uint32_t)key & 0x0fffffffu;
+    return ANY ? (uint32_t)key : (uint32_t)key & (kWinSpan - 1u);
 }
 
 // A ray as the pooled tests read it: {origin, lo} and {direction, tmin}, lo a
@@ -253,9 +262,9 @@ __device__ __forceinline__ unsigned long long win_wave_min(unsigned long long v)
     return v;
 }
 
-// One long list of lane l's ray (cell s of its window): the whole wave, 64
-// records a round.
-template <bool ANY>
+// One long list of lane l's ray (cell s of its window): the whole wave, 128
+// records a round (n is at most kRefsMax: j0 does not wrap).
+template <bool ANY, bool SPANS>
 __device__ __forceinline__ void win_long(WaveWin& W, const float4* __restrict__ trir, uint32_t l,
                                          uint32_t s, uint32_t b, uint32_t n, float end)
 {
@@ -280,7 +289,8 @@ __device__ __forceinline__ void win_long(WaveWin& W, const float4* __restrict__ 
             break;
     }
     key = win_wave_min(key);
-    if (lane == 0 && key < W.win[l])
+    // at the same t a hit of an earlier span of the list stays
+    if (lane == 0 && (SPANS ? (key >> 28) < (W.win[l] >> 28) : key < W.win[l]))
         W.win[l] = key;
 }
 
@@ -289,7 +299,7 @@ __device__ __forceinline__ void win_long(WaveWin& W, const float4* __restrict__ 
 // wave calls it; W.ro and W.rd hold the rays.  The lanes that share a ray name
 // the same owner lane.  Bit s of `subs`: list s is in the second record array
 // (TWO).  Returns the ray's key, ~0 without a hit.
-template <bool ANY, bool TWO, int S>
+template <bool ANY, bool TWO, int S, bool SPANS>
 __device__ __forceinline__ unsigned long long win_tests(WaveWin& W, const WinRecs recs,
                                                         const WinU<S> b, const WinU<S> n,
                                                         const WinU<S> end, uint32_t subs,
@@ -336,6 +346,7 @@ __device__ __forceinline__ unsigned long long win_tests(WaveWin& W, const WinRec
         win_round<ANY, TWO, 1>(W, recs, base, all_tests, all_lists, k0, carry);
     wave_lds_sync();
     if (any_long != 0) {
+        uint32_t done = 0;   // records of the list in spans tested already
         for (;;) {
             const uint64_t m = __ballot(longm != 0);
             if (m == 0)
@@ -349,15 +360,18 @@ __device__ __forceinline__ unsigned long long win_tests(WaveWin& W, const WinRec
             const float4* __restrict__ rec =
                 TWO && __builtin_amdgcn_readlane((int)((subs >> s) & 1u), (int)l) != 0 ? recs.sub
                                                                                        : recs.top;
-            if (lane == l)
+            const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)lb, (int)l) + done;
+            const uint32_t left = (uint32_t)__builtin_amdgcn_readlane((int)ln, (int)l) - done;
+            const bool rest = !SPANS || left <= kWinSpan;
+            if (lane == l && rest)
                 longm &= longm - 1u;
+            done = rest ? 0u : done + kWinSpan;
             if (__builtin_amdgcn_readlane((int)skip, (int)l))
                 continue;
-            win_long<ANY>(W, rec, (uint32_t)__builtin_amdgcn_readlane((int)owner, (int)l),
-                          (uint32_t)__builtin_amdgcn_readlane((int)(cell0 + s), (int)l),
-                          (uint32_t)__builtin_amdgcn_readlane((int)lb, (int)l),
-                          (uint32_t)__builtin_amdgcn_readlane((int)ln, (int)l),
-                          __int_as_float(__builtin_amdgcn_readlane((int)le, (int)l)));
+            win_long<ANY, SPANS>(W, rec, (uint32_t)__builtin_amdgcn_readlane((int)owner, (int)l),
+                                 (uint32_t)__builtin_amdgcn_readlane((int)(cell0 + s), (int)l),
+                                 first, rest ? left : kWinSpan,
+                                 __int_as_float(__builtin_amdgcn_readlane((int)le, (int)l)));
             wave_lds_sync();
         }
     }

@@ -1,6 +1,8 @@
 """GPU tests of the windowed one-level traversal at the sizes where its pooled
 tests, its long lists and its choice of lanes per ray change path.  Bar:
 bit-exact to the oracle, counters included, under every schedule."""
+import contextlib
+
 import numpy as np
 import pytest
 
@@ -118,3 +120,69 @@ def test_sparse_waves(gpu_ctx, two, n):
     fr = orc.grid_frame(v, 2.0)
     check_closest(sc, fr, offs, refs, v, rays)
     check_any(sc, fr, offs, refs, v, rays)
+
+
+# An uploaded cell may list triangles again and again, past the 28 bits of a
+# window key's position: the nearest record decides also there, of two at the
+# same t the first, and an any-hit ray stops at the first occluder.
+def test_list_longer_than_a_key_position(gpu_ctx):
+    import torch
+    sec, n = 1 << 28, (1 << 28) + 300
+    tri = lambda x, z: [x, 0.1, z, x + 0.15, 0.1, z, x, 0.9, z]
+    v = np.array([[0.97, 0.97, 0.97, 0.98, 0.97, 0.97, 0.97, 0.98, 0.97],   # 0: in no ray's way
+                  tri(0.0, 0.5), tri(0.0, 0.3), tri(0.25, 0.4), tri(0.25, 0.4),
+                  tri(0.5, 0.5), tri(0.75, 0.6), tri(0.75, 0.2)], np.float32)
+    fr = orc.grid_frame(v, 1e-6)
+    assert list(fr["n"]) == [1, 1, 1]
+    refs = np.zeros(n, np.uint32)
+    refs[100], refs[sec + 5] = 1, 2       # the nearer one in the second 2^28
+    refs[200], refs[sec + 7] = 3, 4       # the same t in both: the first
+    refs[sec + 131] = 5                   # only there
+    refs[9], refs[sec + 9] = 6, 7         # at the same position modulo 2^28
+    offs = np.array([0, n], np.uint32)
+    at = [0, 8, 16, 24]                   # each in a wave of its own
+    rays = {k: np.zeros(32, np.float32) for k in ("ox", "oy", "oz", "dx", "dy", "dz")}
+    rays.update(tmin=np.ones(32, np.float32), tmax=-np.ones(32, np.float32))
+    rays["ox"][at] = [0.02, 0.27, 0.52, 0.77]
+    rays["oy"][:], rays["oz"][:], rays["dz"][:] = 0.2, -1.0, 1.0
+    rays["tmin"][at], rays["tmax"][at] = 0.0, np.inf
+    sc = grt.Scene(gpu_ctx)
+    sc.upload(v, np.zeros_like(v))
+    sc.upload_grid(fr, offs, refs)
+    gpu_ctx.set_trace_mode("simple", 16)
+    rb, hb = grt.RayBatch.from_numpy(rays), grt.HitBatch.empty(32)
+    sc.trace_closest(rb, hb)
+    # triangle 0 is never hit: the oracle walks the others alone, in their order
+    few = refs[refs != 0]
+    foffs = np.array([0, len(few)], np.uint32)
+    g, o = hb.numpy(), orc.trace_closest(fr, foffs, few, v, rays)
+    assert list(o["id"][at]) == [2, 3, 5, 7]
+    for k in ("id", "t", "u", "v"):
+        assert_same(g[k], o[k], f"hit.{k}")
+    # in a batch; all four in one wave, with counters
+    hb = grt.HitBatch.empty(32)
+    with contextlib.closing(grt.Batch(gpu_ctx, 1)) as batch:
+        batch.set([(sc, rb, hb, None, 0)])
+        batch.trace()
+    for k in ("id", "t", "u", "v"):
+        assert_same(hb.numpy()[k], o[k], f"hit.{k}")
+    cnt = torch.full((64,), -7, dtype=torch.int32, device="cuda:0")
+    hb = grt.HitBatch.empty(32)
+    gpu_ctx.set_trace_mode("split", 2)
+    sc.trace_closest(rb, hb, counters=cnt)
+    gpu_ctx.set_trace_mode("simple", 16)
+    for k in ("id", "t", "u", "v"):
+        assert_same(hb.numpy()[k], o[k], f"hit.{k}")
+    c = cnt.cpu().numpy().view(np.uint32).reshape(32, 2)
+    assert list(c[at, 0]) == [1] * 4 and list(c[at, 1]) == [n] * 4
+    occ = torch.full((32,), 9, dtype=torch.uint8, device="cuda:0")
+    cnt = torch.full((64,), -7, dtype=torch.int32, device="cuda:0")
+    sc.trace_any(rb, occ, counters=cnt)
+    oa = orc.trace_any(fr, foffs, few, v, rays, counters=True)
+    assert list(few[oa["tests"][at] - 1]) == [1, 3, 5, 6]
+    oa["tests"][at] = [101, 201, sec + 132, 10]
+    assert_same(occ.cpu().numpy(), oa["occluded"], "occluded")
+    c = cnt.cpu().numpy().view(np.uint32).reshape(32, 2)
+    assert_same(c[:, 0], oa["cells"], "cells visited")
+    assert_same(c[:, 1], oa["tests"], "triangle tests")
+    sc.close()
