@@ -925,9 +925,14 @@ __device__ __forceinline__ void sort_wave_class(const uint32_t* __restrict__ off
 
 // Every listed cell in one launch.  The classes are independent, and a launch
 // for each left the GPU to a few long blocks or waves at a time: the first
-// blocks (up to half of them) take the cells of more than 1024 references, the
-// longest class first, a block each; the others the wave classes and then the
-// small cells, a thread each.  64 KB of LDS: two blocks of 16 waves a CU.
+// blocks take the cells of more than 1024 references, the longest class first,
+// a block each; the others, as many as their cells need up to half the launch,
+// the wave classes, one cell of a class to every block before a second (packed
+// into the first blocks, a few dozen cells waited for one another on a few
+// CUs), and then the small cells, a thread each.  64 KB of LDS: two blocks of
+// 16 waves a CU.  Rebuild of 20 k triangles in cells of 784 references 104 ->
+// 84 us, 100 k in cells of 1635 310 -> 292, stadium of
+// 2^20 triangles at lambda 128 412 -> 404.
 __global__ __launch_bounds__(1024, 8) void k_sort_cells(const DevFrame* __restrict__ fr,
                                                         const uint32_t* __restrict__ offsets,
                                                         uint32_t* __restrict__ refs,
@@ -940,7 +945,10 @@ __global__ __launch_bounds__(1024, 8) void k_sort_cells(const DevFrame* __restri
     c3 = c3 < lists.large_cap ? c3 : lists.large_cap;
     c4 = c4 < lists.large_cap ? c4 : lists.large_cap;
     const uint32_t heavy = c3 + c4, half = gridDim.x / 2u;
-    const uint32_t hb = heavy < half ? heavy : half;   // blocks for the long cells
+    const uint32_t light = (lists.counts[1] + lists.counts[2] + lists.counts[3] +
+                            lists.counts[0] / 64u) / 16u + 1u;
+    const uint32_t most = gridDim.x - (light < half ? light : half);
+    const uint32_t hb = heavy < most ? heavy : most;   // blocks for the long cells
     if (blockIdx.x < hb) {
         for (uint32_t li = blockIdx.x; li < heavy; li += hb) {
             const uint32_t c = li < c4 ? lists.cls[(size_t)4 * lists.large_cap + li]
@@ -957,7 +965,7 @@ __global__ __launch_bounds__(1024, 8) void k_sort_cells(const DevFrame* __restri
         return;
     }
     const uint32_t first = blockIdx.x - hb, blocks = gridDim.x - hb;
-    const uint32_t wave = first * 16u + (threadIdx.x >> 6), waves = blocks * 16u;
+    const uint32_t wave = (threadIdx.x >> 6) * blocks + first, waves = blocks * 16u;
     sort_wave_class<16, 2>(offsets, refs, lists, wave, waves);
     sort_wave_class<4, 1>(offsets, refs, lists, wave, waves);
     sort_wave_class<1, 0>(offsets, refs, lists, wave, waves);
@@ -1198,9 +1206,10 @@ hipError_t launch_grid_scatter(const DevFrame* fr, const float* verts, uint32_t 
 hipError_t launch_grid_sort(const DevFrame* fr, const uint32_t* offsets, uint32_t* refs,
                             const SortLists& lists, hipStream_t s)
 {
-    // a block per 2048 references, up to twice what the GPU holds
+    // a block per 2048 references, up to what the GPU holds (with twice that,
+    // half of a class's waves waited for the blocks of the other half)
     const uint32_t refs_cap = 2u * lists.small_cap, g = refs_cap / 2048u;
-    hipLaunchKernelGGL(k_sort_cells, dim3(g < 32u ? 32u : g < 1024u ? g : 1024u), dim3(1024), 0, s,
+    hipLaunchKernelGGL(k_sort_cells, dim3(g < 32u ? 32u : g < 512u ? g : 512u), dim3(1024), 0, s,
                        fr, offsets, refs, lists);
     return hipGetLastError();
 }

@@ -39,3 +39,35 @@ def test_all_classes_in_one_grid(gpu_ctx):
         _, offs2, refs2 = sc.download_grid()
         assert np.array_equal(offs2, offs) and np.array_equal(refs2, refs)
     sc.close()
+
+
+# More long cells than blocks for them, so blocks sort cells of different
+# classes (tile by tile, between LDS and the references, within LDS) one after
+# another in the same LDS; wave classes and small cells with fewer and with
+# more cells than waves.
+@pytest.mark.parametrize("short", [100, 3000])
+def test_more_cells_than_blocks(gpu_ctx, short):
+    r = np.random.default_rng(short)
+    sizes = np.concatenate([[4200, 5000, 8192, 8193, 9000, 16_384, 17_000, 40_000],
+                            r.integers(1025, 1500, 300), r.integers(257, 1024, 60),
+                            r.integers(65, 256, 100), r.integers(17, 64, short),
+                            r.integers(2, 16, 300)])
+    cells = r.permutation(4096)[:len(sizes)]
+    at = np.stack([cells % 16, cells // 16 % 16, cells // 256], 1).repeat(sizes, 0)
+    c = (at[:, None] + 0.5 + 0.1 * (r.random((len(at), 3, 3)) - 0.5)) / 16.0
+    # the corners of the box that the sixteenths divide
+    c = np.concatenate([c, np.zeros((1, 3, 3)), np.ones((1, 3, 3))])
+    v = c.astype(np.float32).reshape(-1, 9)
+    sc, fr, offs, refs = check_grid(gpu_ctx, v, np.zeros_like(v), 4090.0 / len(v))
+    assert list(fr["n"]) == [16, 16, 16]
+    n = np.diff(offs)
+    blocks = min(max((len(refs) * 9 // 8 + 1024) // 2048, 32), 512)   # of the launch
+    waves = ((n > 16) & (n <= 1024)).sum()
+    light = min((waves + ((n > 1) & (n <= 16)).sum() // 64) // 16 + 1, blocks // 2)
+    assert (n > 1024).sum() > blocks - light
+    assert (((n > 16) & (n <= 64)).sum() > 16 * light) == (short == 3000)
+    for _ in range(2):
+        sc.rebuild_grid_async(4090.0 / len(v))
+        _, offs2, refs2 = sc.download_grid()
+        assert np.array_equal(offs2, offs) and np.array_equal(refs2, refs)
+    sc.close()
