@@ -830,9 +830,11 @@ static void trace2_launch(const TraceArgs& a, const RaySoA& rays, const HitSoA& 
 // ones are bound by their longest wave.  Measured on the stadium (us, 1 / 2 /
 // 4 / 8 / 16 lanes): 1360x765 primary 496 / 529 / 720 / - / -; 960x540 primary
 // 434 / 393 / 447 / 628 / -, shadow 419 / 295 / 389 / 528 / -, bounce 623 / 570
-// / 605 / 735 / -; 720x405 primary - / 340 / 365 / 422 / 631; 480x270 primary
-// 432 / 315 / 295 / 293 / 372, shadow 417 / 298 / 239 / 211 / 282, bounce 580 /
-// 377 / 399 / 365 / 411; 160x90 shadow 424 / 277 / 218 / 185 / 174.
+// / 605 / 735 / -; 720x405 primary - / 348 / 368 / 421 / 615, shadow - / 293 /
+// 268 / 363 / 505, bounce - / 476 / 496 / 516 / 673, bounce shadow - / 220 / 214
+// / 197 / 218 (2 and 4 are level over the stages); 480x270 primary 432 / 315 /
+// 295 / 293 / 372, shadow 417 / 298 / 239 / 211 / 282, bounce 580 / 377 / 399 /
+// 365 / 411; 160x90 shadow 424 / 277 / 218 / 185 / 174.
 static uint32_t trace2_lanes(uint64_t slots)
 {
     if (slots >= 1000000)
@@ -844,6 +846,18 @@ static uint32_t trace2_lanes(uint64_t slots)
     return slots >= 32000 ? 8 : 16;
 }
 
+// A fixed number of lanes per ray (the split schedule) holds below kFixedSlots
+// ray slots, and for ray lists, which may name few of them; otherwise at most
+// kFixedLanes from there on.  Every lane of a group steps the whole walk,
+// sub-grids included, so more lanes do not pay there: stadium (us, 4 lanes / 2)
+// 1920x1080 primary 1346 / 879, bounce 1681 / 1204; 960x540 primary 445 / 401,
+// shadow 393 / 304, bounce 606 / 513, bounce shadow 238 / 230; below, at
+// 720x405, shadow 268 / 293 and bounce shadow 214 / 220.  The walk in which the
+// lanes of a group took sub-grids in turn had 1225 and 1700 with 4 lanes at
+// 1920x1080.
+constexpr uint32_t kFixedLanes = 2;
+constexpr uint64_t kFixedSlots = 500000;
+
 hipError_t launch_trace2(const TraceArgs& a, const RaySoA& rays, const HitSoA& hits,
                          uint8_t* occluded, uint32_t lanes, hipStream_t s)
 {
@@ -852,11 +866,14 @@ hipError_t launch_trace2(const TraceArgs& a, const RaySoA& rays, const HitSoA& h
     if (lanes > 16 || (lanes & (lanes - 1)) != 0)
         return hipErrorInvalidValue;
     const uint64_t slots = slot_count(a.n, a.image_width);
-    if (lanes == 0)
-        lanes = trace2_lanes(slots);
-    const uint64_t threads = slots * lanes;
+    uint64_t threads = slots * lanes;
     if (lanes > 1 && threads > 0xffffffffull - 256)
         return hipErrorInvalidValue;
+    if (lanes == 0)
+        lanes = trace2_lanes(slots);
+    else if (lanes > kFixedLanes && slots >= kFixedSlots && !a.list)
+        lanes = kFixedLanes;
+    threads = slots * lanes;
     const uint32_t g = (uint32_t)((threads + 127) / 128);
     if (occluded && a.counters)
         trace2_launch<true, true>(a, rays, hits, occluded, lanes, g, s);

@@ -89,8 +89,9 @@ int grt_set_block_size(grt_context ctx, uint32_t closest, uint32_t any);
  * the lanes per ray (1 to 8, on a two-level grid 1 to 16) by the size of the
  * launch; their `param` (1..64) is checked and otherwise unused.
  * GRT_TRACE_SPLIT: `param` (2, 4, 8 or 16) lanes per ray, each visiting some
- * of the ray's cells.  Results and counters are identical; only the schedule
- * differs.
+ * of the ray's cells; a two-level launch of 500,000 ray slots or more takes at
+ * most 2, a ray list always `param`.  Results and counters are identical; only
+ * the schedule differs.
  * The serving loop and batches (grt_batch_trace) follow the setting; a batch
  * under GRT_TRACE_SPLIT gives every ray of every item `param` lanes (64 /
  * param rays per wave). */

@@ -66,6 +66,17 @@ def test_two_level_lanes_by_launch_size(gpu_ctx, n):
                  modes=[("simple", 16)])
 
 
+# Both sides of the size up to which a fixed number of lanes per ray holds.
+@pytest.mark.parametrize("n", [499_999, 500_000])
+def test_two_level_fixed_lanes(gpu_ctx, n):
+    v = np.concatenate([_soup(230, 3, 1.2), _soup(400, 4, 0.02) * np.float32(0.1) +
+                        np.float32(0.45)])
+    sc = _built(gpu_ctx, v, np.zeros_like(v), 0.2, 0.1, 250)
+    fr, offs, refs, g2 = check_levels(sc, v, 0.2, 0.1, 250)
+    check_trace2(sc, fr, offs, refs, g2, v, _random_rays(n, 5), one_level=False,
+                 modes=[("split", k) for k in (2, 4, 8, 16)])
+
+
 # Both sides of every size at which the lanes per ray change.
 @pytest.mark.parametrize("n", [99_999, 100_000, 399_999, 400_000, (4 << 20) - 1, 4 << 20])
 def test_lanes_by_launch_size(gpu_ctx, n):
