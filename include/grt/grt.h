@@ -86,8 +86,10 @@ int grt_set_block_size(grt_context ctx, uint32_t closest, uint32_t any);
 /* Traversal scheduling.  Every schedule walks its rays in windows of cells and
  * spreads the triangle tests of a window over the lanes of the wave.
  * GRT_TRACE_SIMPLE (default), GRT_TRACE_POOLED and GRT_TRACE_PERSISTENT choose
- * the lanes per ray (1 to 8, on a two-level grid 1 to 16) by the size of the
- * launch; their `param` (1..64) is checked and otherwise unused.
+ * the lanes per ray (1 to 16) by the size of the launch and, one-level, by
+ * whether the grid is flat (as of the last build, check or upload: an
+ * asynchronous rebuild's frame is known once grt_grid_check has read it); their
+ * `param` (1..64) is checked and otherwise unused.
  * GRT_TRACE_SPLIT: `param` (2, 4, 8 or 16) lanes per ray, each visiting some
  * of the ray's cells; a two-level launch of 500,000 ray slots or more takes at
  * most 2, a ray list always `param`.  Results and counters are identical; only
@@ -224,7 +226,9 @@ int grt_grid_check(grt_scene scene);
 /* Upload a grid built elsewhere (cudaTransferCellPointers /
  * cudaTransferCellTriangleIds / cudaSetBoxMin / cudaSetBoxMax /
  * cudaSetGridParameters, RayTracing.h:31-36): frame from info (bmin, bmax,
- * cell, inv_cell, n), offsets[m+1], refs[offsets[m]] plain triangle ids. */
+ * cell, inv_cell, n), offsets[m+1], refs[offsets[m]] plain triangle ids.  A
+ * cell may list a triangle more than once; more than 2^32 - 128 references are
+ * GRT_CAPACITY. */
 int grt_grid_upload(grt_scene scene, const grt_grid_info* info, const uint32_t* offsets_host,
                     const uint32_t* refs_host);
 int grt_grid_info_get(grt_scene scene, grt_grid_info* out);
@@ -235,7 +239,7 @@ int grt_grid_info_get(grt_scene scene, grt_grid_info* out);
  * cells from the top frame's rule applied to the cell (x = lambda2 n / cell
  * volume, r_a = ceil(cell_a cbrt(x)), at most 16 per axis), rebuilt on the
  * device with the top grid.  grt_trace_closest / grt_trace_any and the _list
- * traces then walk both levels, one ray per lane whatever the trace mode: a
+ * traces then walk both levels, with the lanes per ray of the trace mode: a
  * subdivided cell is crossed by a DDA of its own, hits bounded by the
  * sub-cell's exit.  The closest hit is the one-level grid's triangle, t, u
  * and v except where two hits lie within the exit bound's 2^-20 of each other;
@@ -439,8 +443,8 @@ int grt_shade_phong(grt_scene scene, const grt_rays* rays, const grt_hits* hits,
 /* The reference traced one scene per launch (cudaRayTrace,
  * RayTracing.cu:227-253).  A batch holds items -- each a ray batch of one
  * scene, closest hit (any = 0, outputs in hits) or any hit (any = 1, output in
- * occluded) -- and traces all of them in one launch, each wave in one item.  Item pointers are captured at
- * grt_batch_set: call it again after a grt_grid_build or grt_grid_upload of any
+ * occluded) -- and traces all of them in one launch, each wave in one item.
+ * Item pointers are captured at grt_batch_set: call it again after a grt_grid_build or grt_grid_upload of any
  * item's scene (grt_grid_rebuild_async keeps the pointers valid). */
 typedef struct grt_batch_t* grt_batch;
 typedef struct {

@@ -69,8 +69,8 @@ def test_batch_items_match_oracle(gpu_ctx, three_scenes):
             items.append((sc, rb, hb, None, width))
             outs.append(hb)
             want.append(orc.trace_closest(fr, offs, refs, v, rays))
-    # every batched kernel (one ray per lane, persistent, several lanes per
-    # ray), cooperative pass on and off, two item orders
+    # every trace mode (lanes per ray chosen by the launch, or 2 to 16 of them),
+    # two item orders
     for mode, param, coop, rev in (("simple", 16, 16, False), ("simple", 16, 0, True),
                                    ("pooled", 16, 16, True), ("persistent", 16, 16, True),
                                    ("persistent", 1, 1, False), ("split", 2, 16, False),
@@ -182,8 +182,7 @@ def test_serve_result_same_alone_and_in_mix(gpu_ctx, three_scenes):
 
     mix, res_mix = make(reqs, True, [0.0] * len(reqs))
     assert np.all(res_mix[2] >= res_mix[1]) and np.all(res_mix[3] > 0)
-    # the persistent, pooled and split batched kernels serve the same mix
-    # identically
+    # every trace mode serves the same mix identically
     for mode, param in (("persistent", 16), ("pooled", 16), ("split", 4)):
         gpu_ctx.set_trace_mode(mode, param)
         try:

@@ -10,9 +10,9 @@ two resolutions the frame autotuner chooses between: lambda 256 (about
 
 The four traversal stages of the 1920 x 1080 frame -- primary closest hit,
 shadow any hit, one mirror bounce, bounce shadow -- run under every schedule
-the autotuner may pick (one ray per lane with per-lane or pooled tests,
-persistent refill, 2, 4, 8 and 16 lanes per ray), over the whole image and
-over compacted ray lists, and the Phong frame is shaded from them.
+the autotuner may pick (lanes per ray chosen by the launch, 2, 4, 8 and 16
+lanes per ray) and the other trace modes, over the whole image and over
+compacted ray lists, and the Phong frame is shaded from them.
 
 Bar: bit-exact against the oracle (its OpenMP path) -- transformed vertices,
 grid frame, offsets, references, generated rays, hit id / t / u / v,
@@ -38,9 +38,8 @@ WIDTH, HEIGHT = 1920, 1080
 EYE, CENTER, UP, FOVY = (0.5, 0.6, -1.5), (0.5, 0.3, 0.5), (0.0, 1.0, 0.0), 60.0
 LIGHT, OFFSET = (1000.0, 1000.0, 1000.0), 1e-4
 
-# (schedule, refill threshold or lanes per ray): every candidate of the frame
-# autotuner ('s', 'w', 'p', '2', '4', '8', 'x'), all with cooperative dense
-# cells at the bench's threshold of 16.
+# (trace mode, parameter): every schedule letter of the benchmark ('s', and 'w'
+# and 'p', which launch the same, '2', '4', '8', 'x').
 SCHEDULES = [("simple", 16), ("pooled", 16), ("persistent", 16), ("split", 2), ("split", 4),
              ("split", 8), ("split", 16)]
 
@@ -254,10 +253,10 @@ TWO_LEVEL = [(8.0, 4.0, 8), (16.0, 4.0, 8), (16.0, 4.0, 4), (8.0, 8.0, 8), (4.0,
 
 
 def _two_level_stage(ctx, sc, rays, fr, offs, refs, g2, ov, closest, tag, lst, count):
-    """One stage through the two-level grid: whole image one ray per lane
-    (simple, pooled, persistent: the same kernel), 4 and 16 lanes per ray
-    (split), and as compacted lists, all equal to the oracle's two-level
-    traversal; returns the oracle's result."""
+    """One stage through the two-level grid: whole image with the lanes per ray
+    of the launch (simple, pooled, persistent: the same) and 4 and 16 asked for
+    (2 at this size), and as compacted lists, 8 lanes per ray among them, all
+    equal to the oracle's two-level traversal; returns the oracle's result."""
     n = rays.n
     o = rays.numpy()
     active = o["tmin"] <= o["tmax"]
@@ -377,9 +376,7 @@ def test_bench_frame_branches_concurrent_same_as_sequential(gpu_ctx, grid, sched
     """The benchmarked frame with its shadow and bounce branches on two streams
     (the bounce rays, their shadow rays, list compaction and both traces on a
     second stream) writes exactly what the one-stream frame writes: hits,
-    occlusion flags of both levels and the RGBA8 image, for two frames; on the
-    one-level grid both branches run the persistent schedule at once (each
-    stream has its own slot counter)."""
+    occlusion flags of both levels and the RGBA8 image, for two frames."""
     import os
     import sys
     sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))

@@ -56,9 +56,9 @@ def _oracle_grid_equal(sc, v, lam, tag):
 @pytest.mark.parametrize("mode,param", [("pooled", 16), ("split", 4)])
 def test_batch64_levels_match_alone_and_oracle(gpu_ctx, mode, param):
     """The 64 jobs of the batching workload, one batched launch per depth
-    level (the autotuner's lambda 2; pooled one ray per lane, and 4 lanes per
-    ray).  Every item of every level equals the same item traced alone (one
-    ray per lane), and 512 seeded rays per item equal the oracle."""
+    level (the autotuner's lambda 2; lanes per ray chosen by the launch, and 4).
+    Every item of every level equals the same item traced alone, and 512 seeded
+    rays per item equal the oracle."""
     ctx = gpu_ctx
     lam = 2.0
     jobs = W.batch_jobs()

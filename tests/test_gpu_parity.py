@@ -57,12 +57,10 @@ def check_grid(ctx, v, n, lam):
     return sc, fr, ooffs, orefs
 
 
-# Every traversal schedule must give identical per-ray results and counters:
-# (schedule, refill threshold or lanes per ray, cooperative threshold).  The
-# per-lane, split and persistent schedules finish dense cells cooperatively;
-# thresholds 1 and 2 make nearly every such cell cooperative, 0 turns the pass
-# off.  The pooled schedule spreads every wave's tests over its lanes; the
-# split schedule gives each ray 2..16 lanes that take its cells in turn.
+# Every trace mode must give identical per-ray results and counters: (mode,
+# parameter, cooperative threshold).  Simple, pooled and persistent are one
+# schedule, the lanes per ray chosen by the launch, whatever the parameter and
+# the threshold; split fixes 2..16 lanes per ray.
 MODES = [("simple", 16, 16), ("simple", 16, 0), ("pooled", 16, 16), ("persistent", 16, 0),
          ("persistent", 16, 16), ("persistent", 1, 1), ("persistent", 64, 2),
          ("split", 2, 16), ("split", 4, 0), ("split", 8, 1), ("split", 16, 16)]
@@ -196,8 +194,8 @@ def test_grid_build_edge(gpu_ctx, name):
 @pytest.mark.parametrize("name", ["degenerate", "duplicates", "big_triangle", "hot_cell"])
 def test_trace_edge(gpu_ctx, name):
     """Traversal on the edge scenes.  Duplicates put exact t ties in one cell
-    (the earliest reference must win, also in cooperative passes); the hot
-    cell holds 40,000 references, so drained waves test it cooperatively."""
+    (the earliest reference must win, whichever lane tests it); the hot cell
+    holds 40,000 references, a list that a whole wave tests on its own."""
     v = _edge_scenes()[name]
     n = np.zeros_like(v)
     sc, fr, offs, refs = check_grid(gpu_ctx, v, n, 5.0)

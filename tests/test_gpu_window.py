@@ -1,4 +1,4 @@
-"""GPU tests of the windowed one-level traversal at the sizes where its pooled
+"""GPU tests of the windowed traversals at the sizes where its pooled
 tests, its long lists and its choice of lanes per ray change path.  Bar:
 bit-exact to the oracle, counters included, under every schedule."""
 import contextlib
@@ -21,6 +21,19 @@ def _soup(n, seed, size=0.2):
     c = r.random((n, 1, 3)).astype(np.float32)
     return (c + (r.random((n, 3, 3)).astype(np.float32) - np.float32(0.5)) * np.float32(size)
             ).reshape(n, 9)
+
+
+def _check_plain(sc, rb, o, oa):
+    """Traces without counters against the oracle's results."""
+    import torch
+    hb = grt.HitBatch.empty(rb.n)
+    occ = torch.full((rb.n,), 9, dtype=torch.uint8, device="cuda:0")
+    sc.trace_closest(rb, hb)
+    sc.trace_any(rb, occ)
+    g = hb.numpy()
+    for k in ("id", "t", "u", "v"):
+        assert_same(g[k], o[k], f"hit.{k}")
+    assert_same(occ.cpu().numpy(), oa["occluded"], "occluded")
 
 
 # One cell that lists every triangle: rounds of 64 and 128 pooled tests with
@@ -62,8 +75,11 @@ def test_two_level_lanes_by_launch_size(gpu_ctx, n):
     lens, sub = np.diff(offs), np.diff(g2[1])
     plain = lens[(lens > 0) & (lens < 250)]
     assert plain.max() >= 192 and plain.min() < 192 and sub.max() >= 192 and sub.min() < 192
-    check_trace2(sc, fr, offs, refs, g2, v, _random_rays(n, 5), one_level=False,
-                 modes=[("simple", 16)])
+    rays = _random_rays(n, 5)
+    check_trace2(sc, fr, offs, refs, g2, v, rays, one_level=False, modes=[("simple", 16)])
+    _check_plain(sc, grt.RayBatch.from_numpy(rays),
+                 orc.grid2_trace_closest(fr, offs, refs, g2, v, rays),
+                 orc.grid2_trace_any(fr, offs, refs, g2, v, rays))
 
 
 # Both sides of the size up to which a fixed number of lanes per ray holds.
@@ -75,6 +91,13 @@ def test_two_level_fixed_lanes(gpu_ctx, n):
     fr, offs, refs, g2 = check_levels(sc, v, 0.2, 0.1, 250)
     check_trace2(sc, fr, offs, refs, g2, v, _random_rays(n, 5), one_level=False,
                  modes=[("split", k) for k in (2, 4, 8, 16)])
+    rb = grt.RayBatch.from_numpy(_random_rays(n, 5))
+    o, oa = (f(fr, offs, refs, g2, v, _random_rays(n, 5))
+             for f in (orc.grid2_trace_closest, orc.grid2_trace_any))
+    for k in (2, 4, 8, 16):
+        gpu_ctx.set_trace_mode("split", k)
+        _check_plain(sc, rb, o, oa)
+    gpu_ctx.set_trace_mode("simple", 16)
 
 
 # Both sides of every size at which the lanes per ray change.
@@ -107,6 +130,42 @@ def test_lanes_by_launch_size(gpu_ctx, n):
             assert_same(c[:, 1], oa["tests"], "triangle tests")
 
 
+# Flat grids take other lanes per ray: both sides of every size at which these
+# change, with the flat grid known to the host, and not known (no build, no
+# check since the reservation), where the launch goes by its size alone.
+@pytest.mark.parametrize("n", [99_999, 100_000, 399_999, 400_000, 999_999, 1_000_000,
+                               (4 << 20) - 1, 4 << 20])
+def test_flat_lanes_by_launch_size(gpu_ctx, n):
+    import torch
+    v = (_soup(64, 3, 0.4).reshape(-1, 3) * np.float32([1.0, 0.04, 1.0])).reshape(-1, 9)
+    sc, fr, offs, refs = check_grid(gpu_ctx, v, np.zeros_like(v), 4.0)
+    cells = fr["n"][0] * fr["n"][1] * fr["n"][2]
+    assert (max(fr["n"]) / 2.5) ** 3 >= cells
+    rays = _random_rays(n, 5)
+    o = orc.trace_closest(fr, offs, refs, v, rays, counters=True)
+    oa = orc.trace_any(fr, offs, refs, v, rays, counters=True)
+    rb, hb = grt.RayBatch.from_numpy(rays), grt.HitBatch.empty(n)
+    occ = torch.full((n,), 9, dtype=torch.uint8, device="cuda:0")
+    cnt = torch.full((2 * n,), -7, dtype=torch.int32, device="cuda:0")
+    gpu_ctx.set_trace_mode("simple", 16)
+    _check_plain(sc, rb, o, oa)
+    for r in (o, oa):
+        if r is o:
+            sc.trace_closest(rb, hb, counters=cnt)
+        else:
+            sc.trace_any(rb, occ, counters=cnt)
+        c = cnt.cpu().numpy().view(np.uint32).reshape(n, 2)
+        assert_same(c[:, 0], r["cells"], "cells visited")
+        assert_same(c[:, 1], r["tests"], "triangle tests")
+    unchecked = grt.Scene(gpu_ctx)
+    unchecked.upload(v, np.zeros_like(v))
+    unchecked.reserve_grid(int(cells), len(refs))
+    unchecked.rebuild_grid_async(4.0)
+    _check_plain(unchecked, rb, o, oa)
+    unchecked.close()
+    sc.close()
+
+
 # Waves with few rays to walk give them more lanes: every number of walking
 # rays per wave around the powers of two, first, last and scattered in it, on
 # one level and two.
@@ -126,11 +185,16 @@ def test_sparse_waves(gpu_ctx, two, n):
         fr, offs, refs, g2 = check_levels(sc, v, 2.0, 4.0, 16)
         check_trace2(sc, fr, offs, refs, g2, v, rays, one_level=False,
                      modes=[("simple", 16), ("split", 2), ("split", 8)])
+        _check_plain(sc, grt.RayBatch.from_numpy(rays),
+                     orc.grid2_trace_closest(fr, offs, refs, g2, v, rays),
+                     orc.grid2_trace_any(fr, offs, refs, g2, v, rays))
         return
     _, offs, refs = sc.download_grid()
     fr = orc.grid_frame(v, 2.0)
     check_closest(sc, fr, offs, refs, v, rays)
     check_any(sc, fr, offs, refs, v, rays)
+    _check_plain(sc, grt.RayBatch.from_numpy(rays), orc.trace_closest(fr, offs, refs, v, rays),
+                 orc.trace_any(fr, offs, refs, v, rays))
 
 
 # An uploaded cell may list triangles again and again, past the 28 bits of a
