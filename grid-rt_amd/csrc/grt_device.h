@@ -287,9 +287,9 @@ __device__ __forceinline__ void wave_sort(uint32_t* __restrict__ seg, uint32_t n
 // ping-pong, n words each -- every thread writing 16 consecutive outputs from
 // its merge-path split (a binary search on the diagonal; ties take the left
 // run first).  dst may be seg itself for an even number of merges (n over 8192,
-// up to 16384: four), which end in src.  Run boundaries are multiples of 2048 and the outputs of a
-// thread start at a multiple of 16, so no thread's outputs straddle two
-// merges.
+// up to 16384: four), which end in src.  Run boundaries are multiples of 2048
+// and the outputs of a thread start at a multiple of 16, so no thread's outputs
+// straddle two merges.
 template <int BLOCK>
 __device__ inline void block_merge_sort(uint32_t* seg, uint32_t n, uint32_t* src, uint32_t* dst)
 {

@@ -14,12 +14,12 @@
 //
 // Work layout: the plan of every top cell comes from 4096-cell tiles (16
 // consecutive cells per thread); the dense cells -- few, and clustered where
-// the scene is -- then get one 256-thread block each, one reference per
-// thread: the count pass adds to LDS counters over the reference's sub-cell
-// box (and keeps the box, 4 bits per bound, at the reference's position), the
-// fill pass scatters through LDS cursors, and every sub-cell's ids are then
-// sorted ascending over the whole level -- by a thread, a wave or, past 1024
-// ids, a block.
+// the scene is -- then get a block each, of 512 threads in the count pass and
+// 1024 in the fill, one reference per thread: the count pass adds to LDS
+// counters over the reference's sub-cell box (and keeps the box, 4 bits per
+// bound, at the reference's position), the fill pass scatters through LDS
+// cursors, and every sub-cell's ids are then sorted ascending over the whole
+// level -- by a thread, a wave or, past 1024 ids, a block.
 //   k_g2_plan<false>  per tile: sub-cells and dense cells (tile sums); the
 //                     x pass of the empty cells' skip radii
 //   k_g2_scan_tiles   exclusive scan of both; totals, capacity

@@ -160,10 +160,11 @@ __global__ __launch_bounds__(256) void k_gen_reflection(uint32_t n, RaySoA in, H
 
 // The secondary rays of one step of a render request -- shadow rays and, with
 // MIRROR, mirror rays -- from one read of its hits, their active rays (tmin <=
-// tmax) added to *count.  Bound by its 48 (80 with MIRROR) bytes in and out per
-// ray plus the normals' gather.  A block takes kStepRays rays and adds to the
-// count once: with one atomic per wave on the request's one address, counting
-// 1024 x 1024 rays took 61 us, three times the generation itself.
+// tmax) added to *count.  Bound by its 72 (104 with MIRROR) bytes per ray -- 24
+// of the ray and 16 of its hit in, 32 (64) out -- plus the normals' gather.  A
+// block takes kStepRays rays and adds to the count once: with one atomic per
+// wave on the request's one address, counting 1024 x 1024 rays took 61 us,
+// three times the generation itself.
 constexpr uint32_t kStepRays = 1024;
 
 template <bool MIRROR>

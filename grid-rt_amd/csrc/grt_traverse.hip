@@ -137,7 +137,7 @@ __device__ __forceinline__ DdaW dda_window(const DevFrame* __restrict__ fr, cons
     return w;
 }
 
-// One step (on ties x before y before z) when `go`; false when the ray does not go
+// One step (on ties y before x, z before both) when `go`; false when the ray does not go
 // on (the state then stays in the grid).
 __device__ __forceinline__ bool dda_window_step(DdaW& w, bool go)
 {

@@ -822,8 +822,8 @@ static void grid2_trace_one(const orc_frame* f, const uint32_t* offsets, const u
         /* The top walk goes item by item: a cell, or for an empty cell of skip
          * radius rr > 0 the cells within rr ahead of it on every axis, left in
          * one step.  An item's exit is its first boundary plane crossed, t =
-         * ((float)k cell_a + bmin_a - o_a) / d_a, in the DDA's tie order (x
-         * before y before z on ties).  After a skip the other two axes take
+         * ((float)k cell_a + bmin_a - o_a) / d_a, in the DDA's tie order (y
+         * before x, z before both).  After a skip the other two axes take
          * the cells of the exit point (vox), kept within the skipped cells. */
         for (;;) {
             ++cells;
