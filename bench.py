@@ -62,18 +62,17 @@ def parse():
     p.add_argument("--block", type=int, default=0, help="traversal block size (0 = default)")
     p.add_argument("--sched", default=None,
                    help="traversal schedule per stage (primary, shadow, bounce, bounce "
-                        "shadow): s = one ray per lane, w = one ray per lane with pooled "
-                        "tests, p = persistent refill, 2/4/8 = lanes per ray, x = 16 lanes "
-                        "per ray; default: tuned")
-    p.add_argument("--refill", type=int, default=16)
+                        "shadow): s (w and p launch the same) = lanes per ray chosen by the "
+                        "launch, 2/4/8 = lanes per ray, x = 16 lanes per ray; default: tuned")
+    p.add_argument("--refill", type=int, default=16,
+                   help="parameter of the trace mode under s, w and p (no effect)")
     p.add_argument("--ray-lists", nargs="?", const="ccc", default=None,
                    help="ray lists of the three secondary stages (shadow, bounce, bounce "
                         "shadow), one letter each: - = none, c = compacted in slot order; "
                         "the flag alone means ccc; default: tuned with the schedule "
                         "(--- when --sched is given)")
     p.add_argument("--coop", type=int, default=16,
-                   help="cooperative cell tests in drained persistent waves: minimum "
-                        "references left (0 = off)")
+                   help="accepted and without effect: every schedule pools its tests")
     p.add_argument("--lam", type=float, default=None,
                    help="grid resolution factor; default: tuned over %s" % (LAMBDAS,))
     p.add_argument("--sub", default=None,
@@ -110,11 +109,13 @@ def grid_tag(lam, sub):
     return "%g" % lam if sub is None else "%g/%g/%d" % (lam, sub[0], sub[1])
 
 
-def kernel_name(closest, sched_char, two_level=False):
+def kernel_name(closest, sched_char, two_level=False, listed=True):
     """The traversal kernel a stage launches, and its lanes per ray where the
     schedule character fixes them (a two-level grid is walked by its own
-    kernel)."""
+    kernel, whose launches over the whole image take at most 2)."""
     lanes = {"2": 2, "4": 4, "8": 8, "x": 16}.get(sched_char)
+    if lanes and two_level and not listed:
+        lanes = 2
     return "%s<%s, false>%s" % ("k_trace2_window" if two_level else "k_trace_window",
                                 "false" if closest else "true",
                                 " %d lanes" % lanes if lanes else "")
@@ -123,7 +124,7 @@ def kernel_name(closest, sched_char, two_level=False):
 class Frame:
     """Device buffers and the per-frame pipeline of the stadium workload."""
 
-    def __init__(self, grt, torch, lam=LAMBDA, sched="spsp", refill=16, sub=None):
+    def __init__(self, grt, torch, lam=LAMBDA, sched="ssss", refill=16, sub=None):
         self.grt, self.torch = grt, torch
         self.lam = lam
         self.sub = sub
@@ -201,10 +202,9 @@ class Frame:
         return self.xf[frame]
 
     def concurrent_ok(self):
-        """Whether the shadow and bounce stages may run on two streams (the
-        persistent schedules keep their slot counter per stream, the ray-list
-        compaction its block sums per context: the frame compacts before the
-        branches split)."""
+        """Whether the shadow and bounce stages may run on two streams: always
+        (traces keep no state, and the ray-list compaction, whose block sums are
+        per context, comes before the branches split)."""
         return True
 
     def run(self, frame, events=None, concurrent=False):
@@ -341,9 +341,8 @@ class Frame:
     SPLIT_LANES = {"2": 2, "4": 4, "8": 8, "x": 16}
 
     def mode(self, stage):
-        """Traversal schedule of a stage: 's' one ray per lane, 'w' one ray per
-        lane with the wave's tests pooled, 'p' persistent, '2'/'4'/'8' that
-        many lanes per ray, 'x' 16 lanes per ray."""
+        """Traversal schedule of a stage: 's' ('w', 'p') lanes per ray chosen by
+        the launch, '2'/'4'/'8' that many lanes per ray, 'x' 16 lanes per ray."""
         ch = self.sched[stage]
         self.ctx.set_trace_mode(self.SCHEDULES[ch], self.SPLIT_LANES.get(ch, self.refill))
 
@@ -355,12 +354,12 @@ class Frame:
 def autotune(frame, grids, sched, lists):
     """Pick the grid, the per-stage traversal schedule and the secondary stages'
     ray lists on the frame itself (outside the timed region).  grids lists
-    (lambda, sub) pairs, sub = None for one level or (lambda2, min_refs).  For
-    a one-level grid, every stage is timed under each schedule, with and
-    without ray lists (each stage's time includes its ray generation and list
-    compaction), and the fastest per stage is kept; a two-level grid likewise,
-    with the lanes per ray chosen by the launch ('s') or given ('2', '4', '8',
-    'x')."""
+    (lambda, sub) pairs, sub = None for one level or (lambda2, min_refs).
+    Every stage is timed with the lanes per ray chosen by the launch ('s') and
+    given ('2', '4', '8', 'x'), with and without ray lists (each stage's time
+    includes its ray generation and list compaction), and the fastest per stage
+    is kept.  Launches over the whole image take at most 2 lanes on a two-level
+    grid, so more are timed over ray lists alone."""
     from grt.autotune import Autotuner
     tuner = Autotuner()
     table = {}
@@ -377,19 +376,22 @@ def autotune(frame, grids, sched, lists):
                           "frame_ms": round(sum(ms), 3), "lam": c["lam"], "sub": c["sub"]}
             return sum(ms)
         by = {}
-        # 's', 'w' and 'p' are the same launch on a two-level grid
-        for ch in (Frame.SCHEDULES if sub is None else "s248x"):
+        for ch in "s248x":
             for kind in (("-",) if lists else ("-", "c")):
+                if sub is not None and ch in "48x" and (lists or kind) in ("-", "---"):
+                    continue
                 frame.sched = ch * 4
                 frame.lists_kind = lists or kind * 3
                 by[(ch, kind)] = frame.time_stages(frames=3)
         # primary rays are never listed; each secondary stage takes its best
-        # pair, a ray list only when it beats the same schedule without one by 2%
+        # pair, a ray list only when it beats the same launch without one (of 2
+        # lanes, where more are timed over lists alone) by 2%
         picks = []
         for i in range(4):
             k = min((k for k in by if i > 0 or k[1] == "-"), key=lambda k: by[k][2 + i])
-            if k[1] == "c" and by[(k[0], "-")][2 + i] <= 1.02 * by[k][2 + i]:
-                k = (k[0], "-")
+            k2 = (k[0], "-") if (k[0], "-") in by else ("2", "-")
+            if k[1] == "c" and by[k2][2 + i] <= 1.02 * by[k][2 + i]:
+                k = k2
             picks.append(k)
         best = "".join(ch for ch, _ in picks)
         best_lists = lists or "".join(kind for _, kind in picks[1:])
@@ -576,14 +578,13 @@ def main():
     if args.sub is not None and args.sub != "off":
         l2, mr = args.sub.split(",")
         sub_arg = (float(l2), int(mr))
-    frame = Frame(grt, torch, args.lam or LAMBDA, args.sched or "spsp", args.refill, sub_arg)
+    frame = Frame(grt, torch, args.lam or LAMBDA, args.sched or "ssss", args.refill, sub_arg)
     if args.ray_lists is not None and (len(args.ray_lists) != 3 or
                                        set(args.ray_lists) - set("-c")):
         raise SystemExit("--ray-lists takes three letters of - and c (shadow, bounce, "
                          "bounce shadow)")
     if args.block:
         frame.ctx.set_block_size(args.block, args.block)
-    frame.ctx.set_coop(args.coop)
     if args.copy_calibration:
         copy_calibration(torch)
     if args.lam:
@@ -629,7 +630,7 @@ def main():
                 "raygen": d["gen0"] + d["gen1"] + d["gen2"] + d["gen3"],
                 **trace_ms, "shade": d["shade"]}
     if args.profile:
-        print(json.dumps({"mode": "profile", "grid": tag, "schedule": sched, "coop": args.coop,
+        print(json.dumps({"mode": "profile", "grid": tag, "schedule": sched,
                           "lists": frame.lists_kind, "concurrent_branches": concurrent,
                           "ms_per_step": round(ms_per_step, 3),
                           "stage_ms": {k: round(v, 3) for k, v in stage_ms.items()}}))
@@ -647,15 +648,16 @@ def main():
     # achieved = that stage's algorithmic bytes over its launch duration.
     dom_stage = max(trace_ms, key=trace_ms.get)
     si = [name for name, _ in STAGES].index(dom_stage)
-    dom = kernel_name(STAGES[si][1], sched[si], sub is not None)
+    list_of = ["-"] + list(frame.lists_kind)   # of every stage: primary rays have none
+    kernel_of = [kernel_name(closest, sched[i], sub is not None, list_of[i] != "-")
+                 for i, (_, closest) in enumerate(STAGES)]
+    dom = kernel_of[si]
     dom_bytes = counters[dom_stage]["algorithmic_bytes"]
     achieved = dom_bytes / (trace_ms[dom_stage] * 1e-3) / 1e9
     # DRAM bytes of that launch at this lambda, from the committed
     # FETCH_SIZE / WRITE_SIZE profile (null if it has no such line).
-    traffic_of = {name: profile_traffic(tag, name,
-                                        kernel_name(closest, sched[i], sub is not None),
-                                        "-" if i == 0 else frame.lists_kind[i - 1])
-                  for i, (name, closest) in enumerate(STAGES)}
+    traffic_of = {name: profile_traffic(tag, name, kernel_of[i], list_of[i])
+                  for i, (name, _) in enumerate(STAGES)}
     traffic = traffic_of[dom_stage]
     per_stage_roof = {}
     for name, _ in STAGES:
@@ -713,8 +715,8 @@ def main():
             "roofline_primary_shadow": roof_ps,
             "roofline_by_stage": per_stage_roof,
             "stage_counters": counters,
-            "traversal": {"schedule_per_stage": sched, "refill": args.refill,
-                          "block": args.block or 128, "grid": tag, "coop": args.coop,
+            "traversal": {"schedule_per_stage": sched,
+                          "block": args.block or 128, "grid": tag,
                           "secondary_ray_lists": frame.lists_kind,
                           "concurrent_branches": concurrent},
             "stage_ms_note": ("shadow and bounce branches run on two streams: a traversal "

@@ -13,7 +13,7 @@
 // ignores the second level still traces correctly.
 //
 // Work layout: the plan of every top cell comes from 4096-cell tiles (16
-// consecutive cells per thread); the dense cells -- few, and clustered where
+// cells per thread); the dense cells -- few, and clustered where
 // the scene is -- then get a block each, of 512 threads in the count pass and
 // 1024 in the fill, one reference per thread: the count pass adds to LDS
 // counters over the reference's sub-cell box (and keeps the box, 4 bits per

@@ -5,10 +5,8 @@ that depend on the grid):
   lam     grid resolution factor (cells ~ lam * triangles; the reference fixed
           k = 6 in UniformGridAccStructBuilder.cpp:91 and exposed it in its GUI,
           WdgTransformEdit.cpp:49-69)
-  sched   per traversal stage, 's', 'w' or 'p': lanes per ray chosen by the size
-          of the launch; '2', '4', '8' or 'x': 2, 4, 8 or 16 lanes per ray
-  refill  the parameter of grt_set_trace_mode under the first three (checked,
-          otherwise unused)
+  sched   per traversal stage, 's': lanes per ray chosen by the launch; '2', '4',
+          '8' or 'x': 2, 4, 8 or 16 lanes per ray
   block   threads per block of the traversal kernels
 
 The tuner measures candidates with a caller-supplied timing function and keeps

@@ -64,15 +64,14 @@ def serve_vs_plain(ctx: Context, scenes, n_requests: int = 120,
     p99 headroom is the ratio at load 1.0 (arrivals at the plain path's own
     capacity), or at the highest load of the sweep when 1.0 is not in it."""
     torch = _torch()
-    ctx.set_coop(16)
     warm = _requests(scenes, W.serve_requests(6, 0.0, len(scenes), seed=W.SEED_SERVE + 7))
     serve_run(ctx, warm, True, budget, max_active)
     serve_run(ctx, warm, False, budget, max_active)
     torch.cuda.synchronize()
     closed = _requests(scenes, W.serve_requests(n_requests, 0.0, len(scenes)))
-    # Each path runs with the traversal schedule that saturates it best (the
-    # batched path tries the first two, with lanes per ray by its launches).
-    modes = {"simple": 16, "pooled": 16, "split": 4}
+    # The batched path takes the lanes per ray of its launches; the plain path
+    # those or 4, whichever saturates it best.
+    modes = {"simple": 16, "split": 4}
     sat = {True: {}, False: {}}
     for mode, param in modes.items():
         ctx.set_trace_mode(mode, param)
@@ -142,7 +141,7 @@ def serve_vs_plain(ctx: Context, scenes, n_requests: int = 120,
 
 
 # ---------------------------------------------------------------------------
-# Batching: 64 scenes in one persistent launch per depth level, hipGraph
+# Batching: 64 scenes in one launch per depth level, hipGraph
 # ---------------------------------------------------------------------------
 class BatchedJobs:
     """Buffers and per-level batches of the batched configuration."""
@@ -253,8 +252,8 @@ def _time(fn, reps, torch):
 def batch_config(reps: int = 5):
     """Batched (one launch per level, hipGraph) vs plain; the autotuner picks
     the schedule (lanes per ray by the size of the launch, or 2/4/8 of them),
-    lambda in {2,5,8} and the block size.  The plain path gets its best of the single-scene schedules, the
-    split one (4 lanes per ray) included."""
+    lambda in {2,5,8} and the block size.  The plain path gets the better of
+    lanes per ray by the size of each launch and 4."""
     torch = _torch()
     ctx = Context(0)
     stream = stream_create()
@@ -263,13 +262,10 @@ def batch_config(reps: int = 5):
     jobs = W.batch_jobs()
     bj = BatchedJobs(ctx, jobs, 5.0)
     tuner = Autotuner()
-    cands = [{"lam": lam, "block": blk, "mode": m, "refill": 16}
-             for lam in (2.0, 5.0, 8.0) for blk in (64, 128, 256) for m in ("simple", "pooled")]
-    cands += [{"lam": lam, "block": blk, "mode": "persistent", "refill": rf}
-              for lam in (2.0, 5.0, 8.0) for blk in (64, 128, 256) for rf in (8, 16, 32)]
-    # several lanes per ray: 32, 16 or 8 rays per wave ("refill" carries the lanes)
-    cands += [{"lam": lam, "block": blk, "mode": "split", "refill": lanes}
-              for lam in (2.0, 5.0, 8.0) for blk in (128, 256) for lanes in (2, 4, 8)]
+    # param: of grt_set_trace_mode (the lanes per ray of the split schedule)
+    cands = [{"lam": lam, "block": blk, "mode": m, "param": k}
+             for lam in (2.0, 5.0, 8.0) for blk in (64, 128, 256)
+             for m, k in (("simple", 16), ("split", 2), ("split", 4), ("split", 8))]
     cur = {"lam": 5.0}
 
     def measure(c):
@@ -277,7 +273,7 @@ def batch_config(reps: int = 5):
             bj.set_lambda(c["lam"])
             cur["lam"] = c["lam"]
         ctx.set_block_size(c["block"], c["block"])
-        ctx.set_trace_mode(c["mode"], c["refill"])
+        ctx.set_trace_mode(c["mode"], c["param"])
         bj.run_batched()
         ctx.synchronize()
         t0 = time.perf_counter()
@@ -289,7 +285,7 @@ def batch_config(reps: int = 5):
     if best["lam"] != cur["lam"]:
         bj.set_lambda(best["lam"])
     ctx.set_block_size(best["block"], best["block"])
-    ctx.set_trace_mode(best["mode"], best["refill"])
+    ctx.set_trace_mode(best["mode"], best["param"])
     rays = bj.active_rays()
     g = Graph(ctx)
     g.begin()
@@ -306,17 +302,16 @@ def batch_config(reps: int = 5):
     t_eager = _time(lambda: (bj.run_batched(), ctx.synchronize()), reps, torch)
     # the plain path at the same lambda, with its best schedule
     t_plain_by = {}
-    for mode, param in (("simple", best["refill"]), ("pooled", best["refill"]),
-                        ("persistent", best["refill"]), ("split", 4)):
+    for mode, param in (("simple", 16), ("split", 4)):
         ctx.set_trace_mode(mode, param)
         t_plain_by[mode] = _time(lambda: (bj.run_plain(), ctx.synchronize()), reps, torch)
     t_plain = min(t_plain_by.values())
-    ctx.set_trace_mode(best["mode"], best["refill"])
+    ctx.set_trace_mode(best["mode"], best["param"])
     g.close()
     out = {"jobs": len(jobs), "triangles": int(sum(j["tris"] for j in bj.jobs)),
            "primary_rays": int(sum(j["n"] for j in bj.jobs)), "rays_per_run": rays,
            "tuned": best,
-           "rays_per_wave": 64 // best["refill"] if best["mode"] == "split" else 64,
+           "lanes_per_ray": best["param"] if best["mode"] == "split" else "by launch",
            "batched_graph_ms": round(t_graph * 1e3, 3), "batched_eager_ms": round(t_eager * 1e3, 3),
            "plain_ms": round(t_plain * 1e3, 3),
            "plain_ms_by_schedule": {k: round(v * 1e3, 3) for k, v in t_plain_by.items()},
@@ -382,20 +377,20 @@ def ao_config(lams=(4.0, 8.0, 16.0), reps: int = 3, width: int = 1024, height: i
     def measure(c):
         setup(c["lam"])
         best = {}
-        for mode in ("simple", "pooled", "persistent"):
-            ctx.set_trace_mode(mode, 16)
+        for mode, param in (("simple", 16), ("split", 2), ("split", 4)):
+            ctx.set_trace_mode(mode, param)
             frame(c["lam"], state["extent"])
             frame(c["lam"], state["extent"], record=True)
             torch.cuda.synchronize()
-            best[mode] = sum(ev[i].elapsed_time(ev[i + 1]) for i in range(4))
-        c["mode"] = min(best, key=best.get)
-        return best[c["mode"]] * 1e-3
+            best[mode, param] = sum(ev[i].elapsed_time(ev[i + 1]) for i in range(4))
+        c["mode"], c["param"] = min(best, key=best.get)
+        return best[c["mode"], c["param"]] * 1e-3
 
     tuner = Autotuner()
     cands = [{"lam": lam} for lam in lams]
     pick = tuner.tune("ao-16M", cands, measure)
     setup(pick["lam"])
-    ctx.set_trace_mode(pick["mode"], 16)
+    ctx.set_trace_mode(pick["mode"], pick["param"])
     frame(pick["lam"], state["extent"])
     torch.cuda.synchronize()
     stage = np.zeros(4)
@@ -419,7 +414,7 @@ def ao_config(lams=(4.0, 8.0, 16.0), reps: int = 3, width: int = 1024, height: i
     build_ms, prim_ms, gen_ms, ao_ms = (float(x) for x in stage)
     gbs = active * bytes_ray / (ao_ms * 1e-3) / 1e9
     return {"triangles": n_tris, "ao_rays": active, "spp": spp, "lambda": pick["lam"],
-            "schedule": pick["mode"],
+            "lanes_per_ray": pick["param"] if pick["mode"] == "split" else "by launch",
             "primary_hit_rate": round(float((hits.f["id"] >= 0).float().mean().item()), 4),
             "grid": {"n": [int(x) for x in info["n"]], "cells": info["m"], "refs": info["r"]},
             "frame_ms": round(float(stage.sum()), 3),
@@ -510,7 +505,7 @@ def kdtree_config(lam: float = 256.0, reps: int = 5, width: int = 1920, height: 
         n_act = int(active.sum().item())
         n_rays += n_act
         grid_ms = {}
-        for mode, param in (("simple", 16), ("pooled", 16), ("split", 2), ("split", 16)):
+        for mode, param in (("simple", 16), ("split", 2), ("split", 16)):
             ctx.set_trace_mode(mode, param)
             if closest:
                 grid_ms[f"{mode}{param if mode == 'split' else ''}"] = timed(
@@ -543,8 +538,8 @@ def kdtree_config(lam: float = 256.0, reps: int = 5, width: int = 1920, height: 
             "grid_cells_tests_per_ray": [round(float(gc[0]), 2), round(float(gc[1]), 2)],
             "kd_leaves_tests_per_ray": [round(float(kc[0]), 2), round(float(kc[1]), 2)]}
     # The same rays through the two-level grid (top lambda 8, sub-grids at
-    # lambda2 4 in cells of >= 8 references), one ray per lane or 8 / 16 lanes
-    # per ray, per stage the faster.
+    # lambda2 4 in cells of >= 8 references), with the lanes per ray of the launch
+    # or 2, per stage the faster.
     lam1, lam2, min_refs = two_level
     sc.set_subgrid(lam2, min_refs)
     sc.build_grid(lam1)
@@ -561,7 +556,7 @@ def kdtree_config(lam: float = 256.0, reps: int = 5, width: int = 1920, height: 
     for name, (rays, closest) in stages.items():
         active = rays.f["tmin"] <= rays.f["tmax"]
         g2_ms = {}
-        for mode, param in (("simple", 16), ("split", 8), ("split", 16)):
+        for mode, param in (("simple", 16), ("split", 2)):
             ctx.set_trace_mode(mode, param)
             if closest:
                 g2_ms[f"{mode}{param if mode == 'split' else ''}"] = timed(
