@@ -931,8 +931,8 @@ __device__ __forceinline__ void sort_wave_class(const uint32_t* __restrict__ off
 // into the first blocks, a few dozen cells waited for one another on a few
 // CUs), and then the small cells, a thread each.  64 KB of LDS: two blocks of
 // 16 waves a CU.  Rebuild of 20 k triangles in cells of 784 references 104 ->
-// 84 us, 100 k in cells of 1635 310 -> 292, stadium of
-// 2^20 triangles at lambda 128 412 -> 404.
+// 84 us, 100 k in cells of 1635 310 -> 292, stadium of 2^20 triangles at lambda
+// 128 412 -> 404.
 __global__ __launch_bounds__(1024, 8) void k_sort_cells(const DevFrame* __restrict__ fr,
                                                         const uint32_t* __restrict__ offsets,
                                                         uint32_t* __restrict__ refs,
@@ -1206,10 +1206,17 @@ hipError_t launch_grid_scatter(const DevFrame* fr, const float* verts, uint32_t 
 hipError_t launch_grid_sort(const DevFrame* fr, const uint32_t* offsets, uint32_t* refs,
                             const SortLists& lists, hipStream_t s)
 {
-    // a block per 2048 references, up to what the GPU holds (with twice that,
-    // half of a class's waves waited for the blocks of the other half)
-    const uint32_t refs_cap = 2u * lists.small_cap, g = refs_cap / 2048u;
-    hipLaunchKernelGGL(k_sort_cells, dim3(g < 32u ? 32u : g < 512u ? g : 512u), dim3(1024), 0, s,
+    if (!lists.small)
+        return hipErrorInvalidValue;   // no reference buffers
+    // A block per 2048 references, up to what the GPU holds: with twice that,
+    // half of a class's waves waited for the blocks of the other half (stadium
+    // rebuild at lambda 128 421 us against 405, at 16 with a second level 537
+    // against 518).  Grids of 34 M to 67 M references and more take up to twice
+    // that all the same: their blocks of small cells even out (2^24 triangles at
+    // lambda 4, 84 M references, 3548 us with 512 blocks, 3523 with 1024).
+    const uint32_t refs_cap = 2u * (lists.small_cap - 1u), g = refs_cap / 2048u;
+    const uint32_t q = refs_cap / 65536u, most = q < 512u ? 512u : q < 1024u ? q : 1024u;
+    hipLaunchKernelGGL(k_sort_cells, dim3(g < 32u ? 32u : g < most ? g : most), dim3(1024), 0, s,
                        fr, offsets, refs, lists);
     return hipGetLastError();
 }
