@@ -905,34 +905,28 @@ __global__ __launch_bounds__(256) void k_compact_write(uint32_t n, uint32_t img_
 // ---------------------------------------------------------------------------
 // 5. Per-cell sort
 // ---------------------------------------------------------------------------
-// Cells of one size class, a wave each, from wave `wave` of `waves`: class Q
-// (E = 4^Q) holds 16E < n <= 64E references.
+// Cell li of size class Q (E = 4^Q: 16E < n <= 64E references), by a wave.
 template <int E, int Q>
-__device__ __forceinline__ void sort_wave_class(const uint32_t* __restrict__ offsets,
-                                                uint32_t* __restrict__ refs,
-                                                const SortLists& lists, uint32_t wave,
-                                                uint32_t waves)
+__device__ __forceinline__ void sort_wave_cell(const uint32_t* __restrict__ offsets,
+                                               uint32_t* __restrict__ refs, const SortLists& lists,
+                                               uint32_t li)
 {
-    uint32_t cnt = lists.counts[1 + Q];
-    cnt = cnt < lists.large_cap ? cnt : lists.large_cap;
-    const uint32_t* __restrict__ list = lists.cls + (size_t)Q * lists.large_cap;
-    for (uint32_t li = wave; li < cnt; li += waves) {
-        const uint32_t c = list[li];
-        const uint32_t b = offsets[c];
-        wave_sort<E>(refs + b, offsets[c + 1] - b);
-    }
+    const uint32_t c = lists.cls[(size_t)Q * lists.large_cap + li];
+    const uint32_t b = offsets[c];
+    wave_sort<E>(refs + b, offsets[c + 1] - b);
 }
 
 // Every listed cell in one launch.  The classes are independent, and a launch
 // for each left the GPU to a few long blocks or waves at a time: the first
 // blocks take the cells of more than 1024 references, the longest class first,
 // a block each; the others, as many as their cells need up to half the launch,
-// the wave classes, one cell of a class to every block before a second (packed
-// into the first blocks, a few dozen cells waited for one another on a few
-// CUs), and then the small cells, a thread each.  64 KB of LDS: two blocks of
-// 16 waves a CU.  Rebuild of 20 k triangles in cells of 784 references 104 ->
-// 84 us, 100 k in cells of 1635 310 -> 292, stadium of 2^20 triangles at lambda
-// 128 412 -> 404.
+// the wave classes as one list, a cell to every block before a second (packed
+// into the first blocks, a few dozen cells waited for one another on a few CUs;
+// listed class by class, the same waves took a cell of each), and then the
+// small cells, a thread each.  64 KB of LDS: two blocks of 16 waves a CU.
+// Rebuild of 20 k triangles in cells of 784 references 104 -> 84 us, 100 k in
+// cells of 1635 310 -> 292, stadium of 2^20 triangles at lambda 128 415 -> 402,
+// at 16 with a second level 525 -> 513.
 __global__ __launch_bounds__(1024, 8) void k_sort_cells(const DevFrame* __restrict__ fr,
                                                         const uint32_t* __restrict__ offsets,
                                                         uint32_t* __restrict__ refs,
@@ -941,12 +935,13 @@ __global__ __launch_bounds__(1024, 8) void k_sort_cells(const DevFrame* __restri
     __shared__ uint32_t lds[kSortTile];
     if (fr->status & (kStatusFrameInvalid | kStatusCellsOver | kStatusRefsOver))
         return;
-    uint32_t c3 = lists.counts[1 + 3], c4 = lists.counts[1 + 4];
-    c3 = c3 < lists.large_cap ? c3 : lists.large_cap;
-    c4 = c4 < lists.large_cap ? c4 : lists.large_cap;
+    const auto listed = [&](int q) {
+        const uint32_t c = lists.counts[1 + q];
+        return c < lists.large_cap ? c : lists.large_cap;
+    };
+    const uint32_t c0 = listed(0), c1 = listed(1), c2 = listed(2), c3 = listed(3), c4 = listed(4);
     const uint32_t heavy = c3 + c4, half = gridDim.x / 2u;
-    const uint32_t light = (lists.counts[1] + lists.counts[2] + lists.counts[3] +
-                            lists.counts[0] / 64u) / 16u + 1u;
+    const uint32_t light = (c0 + c1 + c2 + lists.counts[0] / 64u) / 16u + 1u;
     const uint32_t most = gridDim.x - (light < half ? light : half);
     const uint32_t hb = heavy < most ? heavy : most;   // blocks for the long cells
     if (blockIdx.x < hb) {
@@ -966,9 +961,14 @@ __global__ __launch_bounds__(1024, 8) void k_sort_cells(const DevFrame* __restri
     }
     const uint32_t first = blockIdx.x - hb, blocks = gridDim.x - hb;
     const uint32_t wave = (threadIdx.x >> 6) * blocks + first, waves = blocks * 16u;
-    sort_wave_class<16, 2>(offsets, refs, lists, wave, waves);
-    sort_wave_class<4, 1>(offsets, refs, lists, wave, waves);
-    sort_wave_class<1, 0>(offsets, refs, lists, wave, waves);
+    for (uint32_t i = wave; i < c0 + c1 + c2; i += waves) {
+        if (i < c2)
+            sort_wave_cell<16, 2>(offsets, refs, lists, i);
+        else if (i - c2 < c1)
+            sort_wave_cell<4, 1>(offsets, refs, lists, i - c2);
+        else
+            sort_wave_cell<1, 0>(offsets, refs, lists, i - c2 - c1);
+    }
     uint32_t cnt = lists.counts[0];
     cnt = cnt < lists.small_cap ? cnt : lists.small_cap;
     for (uint32_t li = first * 1024u + threadIdx.x; li < cnt; li += blocks * 1024u)
@@ -1210,8 +1210,8 @@ hipError_t launch_grid_sort(const DevFrame* fr, const uint32_t* offsets, uint32_
         return hipErrorInvalidValue;   // no reference buffers
     // A block per 2048 references, up to what the GPU holds: with twice that,
     // half of a class's waves waited for the blocks of the other half (stadium
-    // rebuild at lambda 128 421 us against 405, at 16 with a second level 537
-    // against 518).  Grids of 34 M to 67 M references and more take up to twice
+    // rebuild at lambda 128 416 us against 402, at 16 with a second level 552
+    // against 513).  Grids of 34 M to 67 M references and more take up to twice
     // that all the same: their blocks of small cells even out (2^24 triangles at
     // lambda 4, 84 M references, 3548 us with 512 blocks, 3523 with 1024).
     const uint32_t refs_cap = 2u * (lists.small_cap - 1u), g = refs_cap / 2048u;
