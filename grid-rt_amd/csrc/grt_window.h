@@ -360,17 +360,22 @@ __device__ __forceinline__ unsigned long long win_tests(WaveWin& W, const WinRec
             const float4* __restrict__ rec =
                 TWO && __builtin_amdgcn_readlane((int)((subs >> s) & 1u), (int)l) != 0 ? recs.sub
                                                                                        : recs.top;
-            const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)lb, (int)l) + done;
-            const uint32_t left = (uint32_t)__builtin_amdgcn_readlane((int)ln, (int)l) - done;
-            const bool rest = !SPANS || left <= kWinSpan;
+            // the span of the list to test now: from record `at` on
+            const uint32_t at = done;
+            bool rest = true;
+            if (SPANS) {
+                rest = (uint32_t)__builtin_amdgcn_readlane((int)ln, (int)l) - at <= kWinSpan;
+                done = rest ? 0u : at + kWinSpan;
+            }
             if (lane == l && rest)
                 longm &= longm - 1u;
-            done = rest ? 0u : done + kWinSpan;
             if (__builtin_amdgcn_readlane((int)skip, (int)l))
                 continue;
-            win_long<ANY, SPANS>(W, rec, (uint32_t)__builtin_amdgcn_readlane((int)owner, (int)l),
-                                 (uint32_t)__builtin_amdgcn_readlane((int)(cell0 + s), (int)l),
-                                 first, rest ? left : kWinSpan,
+            const uint32_t ray = (uint32_t)__builtin_amdgcn_readlane((int)owner, (int)l);
+            const uint32_t cell = (uint32_t)__builtin_amdgcn_readlane((int)(cell0 + s), (int)l);
+            const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)lb, (int)l) + at;
+            const uint32_t left = (uint32_t)__builtin_amdgcn_readlane((int)ln, (int)l) - at;
+            win_long<ANY, SPANS>(W, rec, ray, cell, first, rest ? left : kWinSpan,
                                  __int_as_float(__builtin_amdgcn_readlane((int)le, (int)l)));
             wave_lds_sync();
         }
