@@ -919,14 +919,16 @@ __device__ __forceinline__ void sort_wave_cell(const uint32_t* __restrict__ offs
 // Every listed cell in one launch.  The classes are independent, and a launch
 // for each left the GPU to a few long blocks or waves at a time: the first
 // blocks take the cells of more than 1024 references, the longest class first,
-// a block each; the others, as many as their cells need up to half the launch,
-// the wave classes as one list, a cell to every block before a second (packed
-// into the first blocks, a few dozen cells waited for one another on a few CUs;
-// listed class by class, the same waves took a cell of each), and then the
-// small cells, a thread each.  64 KB of LDS: two blocks of 16 waves a CU.
+// a block each; the others, as many as their cells need (eight small cells to a
+// thread) up to half the launch, the wave classes as one list, a cell to every
+// block before a second (packed into the first blocks, a few dozen cells waited
+// for one another on a few CUs; listed class by class, the same waves took a
+// cell of each), and then the small cells, a thread each.  64 KB of LDS: two
+// blocks of 16 waves a CU.
 // Rebuild of 20 k triangles in cells of 784 references 104 -> 84 us, 100 k in
 // cells of 1635 310 -> 292, stadium of 2^20 triangles at lambda 128 415 -> 402,
-// at 16 with a second level 525 -> 513.
+// at 16 with a second level 525 -> 512, at 8 452 -> 438 (457 with one small cell
+// to a thread).
 __global__ __launch_bounds__(1024, 8) void k_sort_cells(const DevFrame* __restrict__ fr,
                                                         const uint32_t* __restrict__ offsets,
                                                         uint32_t* __restrict__ refs,
@@ -941,7 +943,7 @@ __global__ __launch_bounds__(1024, 8) void k_sort_cells(const DevFrame* __restri
     };
     const uint32_t c0 = listed(0), c1 = listed(1), c2 = listed(2), c3 = listed(3), c4 = listed(4);
     const uint32_t heavy = c3 + c4, half = gridDim.x / 2u;
-    const uint32_t light = (c0 + c1 + c2 + lists.counts[0] / 64u) / 16u + 1u;
+    const uint32_t light = (c0 + c1 + c2 + lists.counts[0] / 512u) / 16u + 1u;
     const uint32_t most = gridDim.x - (light < half ? light : half);
     const uint32_t hb = heavy < most ? heavy : most;   // blocks for the long cells
     if (blockIdx.x < hb) {

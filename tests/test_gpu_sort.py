@@ -63,7 +63,7 @@ def test_more_cells_than_blocks(gpu_ctx, short):
     n = np.diff(offs)
     blocks = min(max((len(refs) * 9 // 8 + 1024) // 2048, 32), 512)   # of the launch
     waves = ((n > 16) & (n <= 1024)).sum()
-    light = min((waves + ((n > 1) & (n <= 16)).sum() // 64) // 16 + 1, blocks // 2)
+    light = min((waves + ((n > 1) & (n <= 16)).sum() // 512) // 16 + 1, blocks // 2)
     assert (n > 1024).sum() > blocks - light
     assert (((n > 16) & (n <= 64)).sum() > 16 * light) == (short == 3000)
     for _ in range(2):
