@@ -924,7 +924,7 @@ __device__ __forceinline__ void sort_wave_cell(const uint32_t* __restrict__ offs
 // block before a second (packed into the first blocks, a few dozen cells waited
 // for one another on a few CUs; listed class by class, the same waves took a
 // cell of each), and then the small cells, a thread each.  64 KB of LDS: two
-// blocks of 16 waves a CU.
+// blocks of 16 waves a CU, which leaves 64 VGPRs (8 bytes of scratch a lane).
 // Rebuild of 20 k triangles in cells of 784 references 104 -> 84 us, 100 k in
 // cells of 1635 310 -> 292, stadium of 2^20 triangles at lambda 128 415 -> 402,
 // at 16 with a second level 525 -> 512, at 8 452 -> 438 (457 with one small cell

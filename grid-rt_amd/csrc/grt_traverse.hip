@@ -902,7 +902,10 @@ hipError_t launch_trace2(const TraceArgs& a, const RaySoA& rays, const HitSoA& h
 // 1280x720 frame at lambda 128 4026 / 3594 / 3517 / 4846; 960x540 primary at
 // lambda 8 6174 / 5354 / 4359 / 3312, at 64 1538 / 1341 / 1279 / 1601, at 256
 // 1044 / 907 / 1087 / 1880; 480x270 frame 2305 / 1736 / 1446 / 1419; 160x90
-// frame 2174 / 1458 / 1128 / 990.
+// frame 2174 / 1458 / 1128 / 990.  The rule knows only size and flatness, so it
+// stays where a fine grid, which such a scene needs, does best (lambda 256: 4
+// lanes at 960x540); a coarse one, with its long lists, would gain from more
+// (lambda 64 5% with 8, lambda 8 38% with 16).
 static uint32_t window_lanes(uint64_t slots, bool flat)
 {
     if (slots >= (4u << 20))
